@@ -190,6 +190,82 @@ def test_decode_splits_agree(vm):
         assert mx <= 4e-3
 
 
+def _decode_bound(ref, v):
+    """The bf16 rounding of the result (half an ulp: 2^-8 of the result's power of
+    two) plus what the fp32 products leave: p is held to 2^-17 of itself (its two
+    bf16 parts), sums and exp2 to a few 2^-23 of the convex combination's largest
+    |v|."""
+    binade = np.exp2(np.floor(np.log2(np.maximum(np.abs(ref), 1e-30))))
+    return 2.0 ** -8 * binade * 1.001 + 2.0 ** -15 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("Dh,H,Hk,n_splits", [(128, 16, 4, 0), (128, 8, 8, 1), (128, 24, 4, 8),
+                                              (128, 16, 2, 3), (64, 16, 4, 0), (64, 8, 1, 2),
+                                              (64, 3, 3, 5)])
+def test_decode_attention_stream_head_dims(vm, orc, Dh, H, Hk, n_splits):
+    """decode_attention! at D = 128 and 64 with groups up to 8 (the stream kernel):
+    lengths at the edges of its 16-token blocks and ring slots, 0 and the whole
+    cache, on a strided cache view; to the bf16 rounding of the result."""
+    banner(f"decode_attention_ stream D={Dh} H={H} Hk={Hk} n_splits={n_splits}")
+    ctx = 2100
+    lens = np.array([ctx, 0, 1, 15, 16, 17, 31, 33, 63, 64, 65, 127, 129, 1000], np.int32)
+    B = len(lens)
+    q_bits = normal_bf16((B, H, Dh), 445)
+    k_bits = normal_bf16((B, Hk, ctx, Dh), 446)
+    v_bits = normal_bf16((B, Hk, ctx, Dh), 447)
+    K, V = (torch.zeros((B, Hk, ctx, Dh + 8), dtype=torch.bfloat16, device="cuda")[..., :Dh]
+            for _ in range(2))
+    K.copy_(to_dev(k_bits))
+    V.copy_(to_dev(v_bits))
+    O = torch.empty((B, H, Dh), dtype=torch.bfloat16, device="cuda")
+    vm.decode_attention_({"O": O}, to_dev(q_bits), K, V, lengths=i32(lens), n_splits=n_splits)
+    torch.cuda.synchronize()
+    vf = bf16_to_f32(v_bits)
+    ref = orc.attention(bf16_to_f32(q_bits)[:, :, None], bf16_to_f32(k_bits), vf, causal=False,
+                        k_lengths=lens)[:, :, 0]
+    got = dev_f32(O)
+    over = (np.abs(got - ref) / _decode_bound(ref, vf)).max()
+    print(f"max {np.abs(got - ref).max():.3e}, {over:.3f} of the bound")
+    assert over <= 1.0
+    assert not got[1].any()  # no key: O = 0
+
+
+def test_decode_attention_stream_limits(vm, orc):
+    """At D = 128: an infinity in V reaches its own column of its own sequence
+    only; keys that all score -inf give O = 0; a workspace sized for the generic
+    kernel alone is still accepted and gives the same result."""
+    banner("decode_attention_ stream limits")
+    B, H, Hk, Dh, ctx = 2, 8, 2, 128, 300
+    q = to_dev(normal_bf16((B, H, Dh), 450))
+    k = to_dev(normal_bf16((B, Hk, ctx, Dh), 451))
+    v = to_dev(normal_bf16((B, Hk, ctx, Dh), 452))
+    lens = i32(np.array([300, 77], np.int32))
+
+    def run(k, v, scratch=None, n_splits=0):
+        O = torch.empty((B, H, Dh), dtype=torch.bfloat16, device="cuda")
+        vm.decode_attention_({"O": O}, q, k, v, lengths=lens, scratch=scratch, n_splits=n_splits)
+        torch.cuda.synchronize()
+        return dev_f32(O)
+
+    base = run(k, v)
+    vi = v.clone()
+    vi[0, 1, 5, 9] = float("inf")
+    vi[0, 1, 40, 9] = float("inf")
+    vi[1, 0, 200, 3] = float("inf")          # past the sequence's length
+    got = run(k, vi)
+    assert np.isposinf(got[0, 4:, 9]).all()
+    got[0, 4:, 9] = base[0, 4:, 9]
+    assert np.array_equal(got, base)
+    big = torch.full_like(q, 1.0)
+    q.copy_(big)
+    ki = torch.full_like(k, float("-inf"))
+    assert not run(ki, v).any()
+    small = torch.empty((2 * B * H * (Dh + 2) * 4 + 255) // 256 * 256, dtype=torch.uint8,
+                        device="cuda")
+    mx, _ = maxmean(run(k, v, scratch=small, n_splits=2), run(k, v, n_splits=2))
+    assert mx <= 4e-3
+
+
 # ---------------------------------------------------------------- DeltaNet
 def _f32dev(a):
     return torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda()

@@ -75,10 +75,12 @@ __device__ __forceinline__ f32x4 mfma16k16(const uint2& a, const uint2& b, f32x4
 }
 
 // chunk of the stream partition (token-heads per wave), identical in both kernels
+// (a multiple of the tokens of one ring slot)
+template <int TOK>
 __device__ __forceinline__ int stream_chunk(int W, int NW, int min_chunk) {
   int c = (W + NW - 1) / NW;
   c = max(c, min_chunk);
-  return (c + DSTEP - 1) / DSTEP * DSTEP;
+  return (c + TOK - 1) / TOK * TOK;
 }
 
 __device__ __forceinline__ int clamp_len(const int32_t* lengths, int b, int64_t ctx) {
@@ -106,17 +108,20 @@ struct StepBuf {
 // 512 B with chunk c of row r at c ^ swz(r).
 constexpr int STEP_ELEMS = DSTEP * HEAD_DIM;  // bf16 per K (or V) step: 8 KB
 
-// Issue the direct global->LDS loads of tokens [t, t + 16) of one (b, hk):
-// instruction u moves rows t+2u and t+2u+1 (1 KB contiguous per instruction,
-// non-temporal), 8 for K and 8 for V. Rows past `last` re-read row `last`.
+// Issue the direct global->LDS loads of one slot's tokens [t, t + 4096 / D) of
+// one (b, hk): instruction u moves the 512 / D rows from t + u * 512 / D (1 KB
+// contiguous per instruction, non-temporal), 8 for K and 8 for V. Rows past
+// `last` re-read row `last`.
+template <int D>
 __device__ __forceinline__ void issue_step(uint16_t* lk, uint16_t* lv, const uint16_t* kb,
                                            const uint16_t* vb, int t, int64_t last,
                                            int64_t c_st, int lane) {
+  constexpr int LPR = D / 8;  // lanes (16-byte chunks) per row
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
-    const int r = 2 * u + (lane >> 5);
+    const int r = (512 / D) * u + lane / LPR;
     const int64_t row = min((int64_t)(t + r), last);
-    const int64_t off = row * c_st + 8 * ((lane & 31) ^ swz(r));
+    const int64_t off = row * c_st + 8 * ((lane % LPR) ^ swz(r));
     __builtin_amdgcn_global_load_lds(kb + off, (__attribute__((address_space(3))) void*)(lk + 512 * u),
                                      16, 0, 2);
     __builtin_amdgcn_global_load_lds(vb + off, (__attribute__((address_space(3))) void*)(lv + 512 * u),
@@ -299,7 +304,8 @@ __device__ __forceinline__ bool seg_next(Seg& s, int gw1, const DecodeArgs& a, b
   return true;
 }
 
-// Issue side of the step pipeline: the next 16-token step of the chunk.
+// Issue side of the step pipeline: the next slot (4096 / D tokens) of the chunk.
+template <int D>
 struct Issuer {
   Seg s;
   int t;
@@ -310,11 +316,82 @@ struct Issuer {
       t = s.lo;
     }
     const int64_t base = (int64_t)s.b * a.c_sb + (int64_t)s.hk * a.c_sh;
-    issue_step(slot, slot + STEP_ELEMS, a.kc + base, a.vc + base, t, last, a.c_st, lane);
-    t += DSTEP;
+    issue_step<D>(slot, slot + STEP_ELEMS, a.kc + base, a.vc + base, t, last, a.c_st, lane);
+    t += STEP_ELEMS / D;
     return true;
   }
 };
+
+// The stream partition, from the lengths on the device: this wave's chunk
+// [gw0, gw1) of the token-heads and the segment (b, hk) holding gw0; false when
+// the wave has none. raw_l: lengths[lane] (0 past B). Wave 0 writes the
+// snapshot that the merge reads.
+template <int TOK>
+__device__ __forceinline__ bool stream_partition(const DecodeArgs& a, int w, int lane, int raw_l,
+                                                 int& b, int& hk, int& len, int& raw,
+                                                 int& seg_b_start, int& gw0, int& gw1) {
+  const int Hk = a.Hk;
+  const int len_l = raw_l < 0 ? 0 : (raw_l > a.ctx ? (int)a.ctx : raw_l);
+  // clamped lengths of sequences b0 + lane, b0 a multiple of 64
+  auto lens_at = [&](int b0) __attribute__((always_inline)) {
+    return b0 == 0 ? len_l : ((b0 + lane < a.B) ? clamp_len(a.lengths, b0 + lane, a.ctx) : 0);
+  };
+  // ---- stream partition: total work and this wave's chunk [gw0, gw1).
+  // incl_at(b0): inclusive prefix of len * Hk (token-heads) over sequences
+  // b0 .. b0 + lane, relative to b0
+  const int incl0 = wave_scan_add(len_l * Hk);
+  auto incl_at = [&](int b0) __attribute__((always_inline)) {
+    return b0 == 0 ? incl0 : wave_scan_add(lens_at(b0) * Hk);
+  };
+  int W = __builtin_amdgcn_readlane(incl0, 63);
+  for (int b0 = 64; b0 < a.B; b0 += 64) W += __builtin_amdgcn_readlane(incl_at(b0), 63);
+  W = uniform(W);
+  const int chunk = stream_chunk<TOK>(W, a.NW, a.min_chunk);
+  if (w == 0) {
+    // snapshot of the partition for the merge, which then never reads lengths
+    // (so it may advance them): chunk, then per sequence its clamped length and
+    // first token-head
+    int pre = 0;
+    for (int b0 = 0; b0 < a.B; b0 += 64) {
+      const int l = lens_at(b0);
+      const int incl = incl_at(b0) + pre;
+      if (b0 + lane < a.B) {
+        a.geom[1 + b0 + lane] = l;
+        a.geom[1 + a.B + b0 + lane] = incl - l * Hk;
+      }
+      pre = __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (lane == 0) a.geom[0] = chunk;
+  }
+  gw0 = w * chunk;
+  if (gw0 >= W) return false;
+  gw1 = min(gw0 + chunk, W);
+
+  // ---- locate the segment holding gw0: first b whose prefix (token-heads) passes it
+  b = 0;
+  seg_b_start = 0;
+  {
+    int pre = 0;
+    for (int b0 = 0; b0 < a.B; b0 += 64) {
+      const int len = lens_at(b0);
+      const int incl = incl_at(b0) + pre;
+      const uint64_t m = __ballot(b0 + lane < a.B && incl > gw0);
+      if (m != 0ull) {
+        const int fl = uniform(__ffsll((unsigned long long)m) - 1);
+        b = b0 + fl;
+        seg_b_start = __builtin_amdgcn_readlane(incl - len * Hk, fl);
+        break;
+      }
+      pre = __builtin_amdgcn_readlane(incl, 63);
+    }
+  }
+  b = uniform(b);
+  seg_b_start = uniform(seg_b_start);
+  raw = seq_len_raw(a.lengths, raw_l, b);
+  len = raw < 0 ? 0 : (raw > a.ctx ? (int)a.ctx : raw);
+  hk = (gw0 - seg_b_start) / len;
+  return true;
+}
 
 template <bool FUSED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
@@ -335,64 +412,8 @@ void decode_stream_kernel(DecodeArgs a) {
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) qwv[kk] = load16(a.qw + 32 * kk + 8 * g);
   }
-  const int len_l = raw_l < 0 ? 0 : (raw_l > a.ctx ? (int)a.ctx : raw_l);
-  // clamped lengths of sequences b0 + lane, b0 a multiple of 64
-  auto lens_at = [&](int b0) __attribute__((always_inline)) {
-    return b0 == 0 ? len_l : ((b0 + lane < a.B) ? clamp_len(a.lengths, b0 + lane, a.ctx) : 0);
-  };
-  // ---- stream partition: total work and this wave's chunk [gw0, gw1).
-  // incl_at(b0): inclusive prefix of len * Hk (token-heads) over sequences
-  // b0 .. b0 + lane, relative to b0
-  const int incl0 = wave_scan_add(len_l * Hk);
-  auto incl_at = [&](int b0) __attribute__((always_inline)) {
-    return b0 == 0 ? incl0 : wave_scan_add(lens_at(b0) * Hk);
-  };
-  int W = __builtin_amdgcn_readlane(incl0, 63);
-  for (int b0 = 64; b0 < a.B; b0 += 64) W += __builtin_amdgcn_readlane(incl_at(b0), 63);
-  W = uniform(W);
-  const int chunk = stream_chunk(W, a.NW, a.min_chunk);
-  if (w == 0) {
-    // snapshot of the partition for the merge, which then never reads lengths
-    // (so it may advance them): chunk, then per sequence its clamped length and
-    // first token-head
-    int pre = 0;
-    for (int b0 = 0; b0 < a.B; b0 += 64) {
-      const int l = lens_at(b0);
-      const int incl = incl_at(b0) + pre;
-      if (b0 + lane < a.B) {
-        a.geom[1 + b0 + lane] = l;
-        a.geom[1 + a.B + b0 + lane] = incl - l * Hk;
-      }
-      pre = __builtin_amdgcn_readlane(incl, 63);
-    }
-    if (lane == 0) a.geom[0] = chunk;
-  }
-  const int gw0 = w * chunk;
-  if (gw0 >= W) return;
-  const int gw1 = min(gw0 + chunk, W);
-
-  // ---- locate the segment holding gw0: first b whose prefix (token-heads) passes it
-  int b = 0, seg_b_start = 0;
-  {
-    int pre = 0;
-    for (int b0 = 0; b0 < a.B; b0 += 64) {
-      const int len = lens_at(b0);
-      const int incl = incl_at(b0) + pre;
-      const uint64_t m = __ballot(b0 + lane < a.B && incl > gw0);
-      if (m != 0ull) {
-        const int fl = uniform(__ffsll((unsigned long long)m) - 1);
-        b = b0 + fl;
-        seg_b_start = __builtin_amdgcn_readlane(incl - len * Hk, fl);
-        break;
-      }
-      pre = __builtin_amdgcn_readlane(incl, 63);
-    }
-  }
-  b = uniform(b);
-  seg_b_start = uniform(seg_b_start);
-  const int raw = seq_len_raw(a.lengths, raw_l, b);
-  const int len = raw < 0 ? 0 : (raw > a.ctx ? (int)a.ctx : raw);
-  const int hk = (gw0 - seg_b_start) / len;
+  int b, hk, len, raw, seg_b_start, gw0, gw1;
+  if (!stream_partition<DSTEP>(a, w, lane, raw_l, b, hk, len, raw, seg_b_start, gw0, gw1)) return;
 
   // 0/1 selection operands for the V transpose: Sel_h[8g+j][n] = (8g+j == n+16h)
   uint4 sel[2];
@@ -432,7 +453,7 @@ void decode_stream_kernel(DecodeArgs a) {
   Seg cs;  // compute side
   cs.b = b; cs.hk = hk; cs.len = len; cs.seg_b_start = seg_b_start; cs.raw = raw;
   seg_bounds(cs, gw0, gw1, a, FUSED);
-  Issuer is;  // issue side, two steps ahead
+  Issuer<HEAD_DIM> is;  // issue side, two steps ahead
   is.s = cs;
   is.t = cs.lo;
   int ct = cs.lo, inflight = 0, cslot = 0;
@@ -573,6 +594,214 @@ void decode_stream_kernel(DecodeArgs a) {
   wait_vmcnt<0>();  // no LDS load may land after the wave is gone
 }
 
+// decode_attention! at D = 128 and 64 (q already normalised): the same stream
+// partition, ring and partials, with 4096 / D tokens per ring slot, so that a
+// slot is 8 KB of K and 8 KB of V at every D and a wave keeps 32 KB in flight.
+// HBM-bound: per 32 tokens 2 D/32 + D/16 MFMAs against 128 D bytes.
+//   - P stays at fp32 precision through the bf16 MFMA: a group has at most 8
+//     heads and the MFMA 16 columns, so columns n and n + 8 both score head n;
+//     column n multiplies hi = p truncated to bf16, column n + 8 the rest
+//     p - hi (p - hi - lo <= 2^-17 p), and the two accumulators are added once
+//     per segment. That costs no MFMA. hi is truncated and lo kept positive, so
+//     an infinite v times p stays infinite.
+//   - V^T operands are LDS transpose reads: no value of one key or column
+//     touches another's (a 0/1 selection MFMA would multiply an infinity by 0).
+//   - q is not scaled in bf16 (1/sqrt(128) is no power of two): the scale is in
+//     the fp32 exponent.
+// Measured at D = 128, B = 32, 16/4 heads, lengths U{1024..32768} (900 MB): 143.5
+// us with the merge, 6.3 TB/s; the generic split kernel, bound by its fp32 VALU
+// products, took 575 us (1.6 TB/s).
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void decode_stream_hd_kernel(DecodeArgs a) {
+  constexpr int TOK = STEP_ELEMS / D;  // tokens per ring slot
+  constexpr int NB = TOK / 16;         // 16-token blocks per slot
+  constexpr int NK = D / 32, ND = D / 16;
+  constexpr float SL2 = LOG2E * (D == 64 ? 0.125f : 0.08838834764831845f);
+  static_assert(D == 64 || D == 128, "head dims of this kernel");
+  const int lane = threadIdx.x & 63;
+  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int G = a.G;
+  const int raw_l = lane < a.B ? a.lengths[lane] : 0;
+  int b, hk, len, raw, seg_b_start, gw0, gw1;
+  if (!stream_partition<TOK>(a, w, lane, raw_l, b, hk, len, raw, seg_b_start, gw0, gw1)) return;
+
+  // one __shared__ object per ring slot: reads of one slot do not alias the
+  // loads still landing in the other
+  __shared__ __attribute__((aligned(16))) uint16_t ring0[4][2 * STEP_ELEMS];
+  __shared__ __attribute__((aligned(16))) uint16_t ring1[4][2 * STEP_ELEMS];
+  uint16_t* const r0 = ring0[threadIdx.x >> 6];
+  uint16_t* const r1 = ring1[threadIdx.x >> 6];
+  const int64_t last = a.ctx - 1;
+
+  Seg cs;  // compute side
+  cs.b = b; cs.hk = hk; cs.len = len; cs.seg_b_start = seg_b_start; cs.raw = raw;
+  seg_bounds(cs, gw0, gw1, a, false);
+  Issuer<D> is;  // issue side, two slots ahead
+  is.s = cs;
+  is.t = cs.lo;
+  int ct = cs.lo, inflight = 0, cslot = 0;
+  bool primed = false;
+
+  while (true) {
+    // Q operand for (b, hk): lane (n, g) holds q[head n % 8][32kk + 8g + j]
+    uint4 qop[NK];
+    {
+      const int hn = n & 7;
+      const uint16_t* qp = a.q + (int64_t)cs.b * a.q_sb +
+                           (int64_t)(cs.hk * G + (hn < G ? hn : 0)) * a.q_sh + 8 * g;
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) qop[kk] = load16(qp + 32 * kk);
+      if (!primed) {
+        if (is.next(r0, a, gw1, last, lane, false, raw_l)) ++inflight;
+        if (is.next(r1, a, gw1, last, lane, false, raw_l)) ++inflight;
+        primed = true;
+      }
+    }
+    f32x4 acc[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_part = 0.f;
+    auto step = [&](uint16_t* slot) __attribute__((always_inline)) {
+      // the oldest slot in flight is this one; the 16 loads of a later one may stay out
+      if (inflight >= 2) wait_vmcnt<16>(); else wait_vmcnt<0>();
+      const uint16_t* lk = slot;
+      const uint16_t* lv = slot + STEP_ELEMS;
+      uint4 k[NB][NK];
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk)
+          k[i][kk] = *reinterpret_cast<const uint4*>(lk + (16 * i + n) * D +
+                                                     8 * ((4 * kk + g) ^ swz(n)));
+      // V^T fragments: lane (n, g) of block i, column tile dt holds
+      // V[16i + 4g + r][16dt + n], r = 0..3; this lane reads row 4g + n/4
+      uint2 v[NB][ND];
+      const int vr = 4 * g + (n >> 2);
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+          v[i][dt] = lds_read_tr16(lv + (16 * i + vr) * D +
+                                   8 * ((2 * dt + ((n >> 1) & 1)) ^ swz(vr)) + 4 * (n & 1));
+      --inflight;
+      // the slot is free once its reads have returned; refill it
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (is.next(slot, a, gw1, last, lane, false, raw_l)) ++inflight;
+      const bool tail = ct + TOK > cs.hi;
+      if (tail) {
+        // rows past the range may hold anything: p = 0 must meet finite v
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          uint32_t m01 = 0, m23 = 0;
+          const int t0 = ct + 16 * i + 4 * g;
+          if (t0 < cs.hi) m01 |= 0xffffu;
+          if (t0 + 1 < cs.hi) m01 |= 0xffff0000u;
+          if (t0 + 2 < cs.hi) m23 |= 0xffffu;
+          if (t0 + 3 < cs.hi) m23 |= 0xffff0000u;
+#pragma unroll
+          for (int dt = 0; dt < ND; ++dt) {
+            v[i][dt].x &= m01;
+            v[i][dt].y &= m23;
+          }
+        }
+      }
+      f32x4 sc[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) sc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk)
+#pragma unroll
+        for (int i = 0; i < NB; ++i) sc[i] = mfma16(k[i][kk], qop[kk], sc[i]);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          sc[i][j] *= SL2;
+          if (tail && ct + 16 * i + 4 * g + j >= cs.hi) sc[i][j] = -INFINITY;
+          mx = fmaxf(mx, sc[i][j]);
+        }
+      // running max in log2 units, rescaled lazily: only when it grows by more
+      // than D_RESCALE_SLACK (wave-uniform branch)
+      mx = wave_max_xor(mx, 16);
+      mx = wave_max_xor(mx, 32);
+      const float m_new = fmaxf(m_run, mx);
+      const bool need = m_new > m_run + D_RESCALE_SLACK;
+      if (__ballot(need) != 0ull) {
+        const float m_use = need ? m_new : m_run;
+        const float alpha = (m_use == m_run) ? 1.0f : fast_exp2(m_run - m_use);
+        l_part *= alpha;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) acc[i] *= alpha;
+        m_run = m_use;
+      }
+      const float m_eff = m_run == -INFINITY ? 0.f : m_run;  // every key so far scored -inf
+      uint2 pop[NB];
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        uint32_t h[4];
+        float lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float p = fast_exp2(sc[i][j] - m_eff);
+          l_part += p;
+          h[j] = __float_as_uint(p) & 0xffff0000u;
+          lo[j] = p > 0.f ? fmaxf(p - __uint_as_float(h[j]), 0x1p-100f) : p;
+        }
+        const uint2 hi2 = make_uint2((h[0] >> 16) | h[1], (h[2] >> 16) | h[3]);
+        const uint2 lo2 = make_uint2(pack2(lo[0], lo[1]), pack2(lo[2], lo[3]));
+        pop[i] = n < 8 ? hi2 : lo2;
+      }
+      // O^T += V^T P^T over 32 tokens: k index 8g + j is token 4g + j of the first
+      // block (j < 4) or of the second
+#pragma unroll
+      for (int i = 0; i < NB; i += 2) {
+        const uint4 pb = make_uint4(pop[i].x, pop[i].y, pop[i + 1].x, pop[i + 1].y);
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt)
+          acc[dt] = mfma16(make_uint4(v[i][dt].x, v[i][dt].y, v[i + 1][dt].x, v[i + 1][dt].y), pb,
+                           acc[dt]);
+      }
+      ct += TOK;
+    };
+    if (cslot == 1 && ct < cs.hm) {
+      step(r1);
+      cslot = 0;
+    }
+    while (ct < cs.hm) {
+      step(r0);
+      cslot = 1;
+      if (ct >= cs.hm) break;
+      step(r1);
+      cslot = 0;
+    }
+
+    // partial for (w, segment): slot w + b*Hk + hk; columns n and n + 8 added
+    const float l_tot = col_sum4(l_part);
+    const int64_t slot = (int64_t)w + (int64_t)cs.b * a.Hk + cs.hk;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[dt][j] += __shfl_xor(acc[dt][j], 8, 64);
+    if (n < G) {
+      float* dst = a.part_o + (slot * G + n) * D + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+        *reinterpret_cast<float4*>(dst + 16 * dt) =
+            make_float4(acc[dt][0], acc[dt][1], acc[dt][2], acc[dt][3]);
+      if (g == 0) {
+        a.part_ml[2 * (slot * G + n)] = m_run;
+        a.part_ml[2 * (slot * G + n) + 1] = l_tot;
+      }
+    }
+    if (!seg_next(cs, gw1, a, false, raw_l)) break;
+    ct = cs.lo;
+  }
+  wait_vmcnt<0>();  // no LDS load may land after the wave is gone
+}
+
 // Log-sum-exp merge of a segment's partials (src/kernels/attention_decode.jl:91-132)
 // and the sigmoid gate (src/llm/qwen35.jl:205). One workgroup per (DW-wide d
 // range, head n of the group, hk, b); thread (sg, dq) merges slots w_first+sg,
@@ -583,9 +812,9 @@ void decode_stream_kernel(DecodeArgs a) {
 // (src/llm/generate.jl:82-88).
 constexpr int CM = 8;
 
-template <int DW>
+template <int DW, int D>
 __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgs a) {
-  constexpr int NDR = HEAD_DIM / DW;  // d ranges
+  constexpr int NDR = D / DW;  // d ranges
   constexpr int NDQ = DW / 4;         // float4 columns per range
   constexpr int NSG = 256 / NDQ;      // slot groups
   const int dr = blockIdx.x % NDR, n = blockIdx.x / NDR, hk = blockIdx.y, b = blockIdx.z;
@@ -618,7 +847,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgs a) {
         if (w <= w_last) {
           const int64_t r = (w + base) * a.G + n;
           ml[u] = *reinterpret_cast<const float2*>(a.part_ml + 2 * r);
-          o[u] = *reinterpret_cast<const float4*>(a.part_o + r * HEAD_DIM + d);
+          o[u] = *reinterpret_cast<const float4*>(a.part_o + r * D + d);
         } else {
           ml[u] = make_float2(-INFINITY, 0.f);
           o[u] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -682,25 +911,36 @@ int decode_stream_waves(int B, int Hk, int n_splits) {
   return (nw + 3) / 4 * 4;
 }
 
-hipError_t launch_decode(const DecodeArgs& a, bool fused_q, hipStream_t st) {
+hipError_t launch_decode(const DecodeArgs& a, bool fused_q, int D, hipStream_t st) {
   if (a.B == 0 || a.Hk == 0) return hipSuccess;
   dim3 grid(a.NW / 4);
   if (fused_q)
     hipLaunchKernelGGL(decode_stream_kernel<true>, grid, dim3(256), 0, st, a);
+  else if (D == 128)
+    hipLaunchKernelGGL(decode_stream_hd_kernel<128>, grid, dim3(256), 0, st, a);
+  else if (D == 64)
+    hipLaunchKernelGGL(decode_stream_hd_kernel<64>, grid, dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL(decode_stream_kernel<false>, grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
-hipError_t launch_combine(const CombineArgs& a, hipStream_t st) {
-  if (a.B == 0 || a.Hk == 0) return hipSuccess;
+template <int D>
+static void launch_combine_d(const CombineArgs& a, hipStream_t st) {
   // partials per segment on average: many -> narrow d ranges, more slot groups
-  const bool wide = a.NW >= 32 * a.B * a.Hk;
-  if (wide) {
-    hipLaunchKernelGGL(decode_combine_kernel<16>, dim3(16 * a.G, a.Hk, a.B), dim3(256), 0, st, a);
-  } else {
-    hipLaunchKernelGGL(decode_combine_kernel<64>, dim3(4 * a.G, a.Hk, a.B), dim3(256), 0, st, a);
-  }
+  if (a.NW >= 32 * a.B * a.Hk)
+    hipLaunchKernelGGL((decode_combine_kernel<16, D>), dim3(D / 16 * a.G, a.Hk, a.B), dim3(256), 0,
+                       st, a);
+  else
+    hipLaunchKernelGGL((decode_combine_kernel<64, D>), dim3(D / 64 * a.G, a.Hk, a.B), dim3(256), 0,
+                       st, a);
+}
+
+hipError_t launch_combine(const CombineArgs& a, int D, hipStream_t st) {
+  if (a.B == 0 || a.Hk == 0) return hipSuccess;
+  if (D == 128) launch_combine_d<128>(a, st);
+  else if (D == 64) launch_combine_d<64>(a, st);
+  else launch_combine_d<HEAD_DIM>(a, st);
   return hipGetLastError();
 }
 

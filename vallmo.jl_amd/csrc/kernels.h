@@ -88,7 +88,7 @@ struct DecodeArgs {
   const uint16_t* k_new;
   const uint16_t* v_new;
   int64_t new_sh, new_sb;
-  float* part_o;        // [slots][G][256], slots = NW + B*Hk
+  float* part_o;        // [slots][G][D], slots = NW + B*Hk
   float* part_ml;       // [slots][G][2]  (shift m in log2 units, sum l)
   int B, Hk, G;
   int NW;               // waves of the stream partition (multiple of 4)
@@ -173,8 +173,9 @@ hipError_t launch_sigmoid_gate(uint16_t* o, int64_t o_sh, int64_t o_sb, const ui
 hipError_t launch_advance(int32_t* positions, int B, hipStream_t st);
 hipError_t launch_fill_normal(uint16_t* dst, int64_t n, uint64_t seed, float scale, float shift,
                               hipStream_t st);
-hipError_t launch_decode(const DecodeArgs& a, bool fused_q, hipStream_t st);
-hipError_t launch_combine(const CombineArgs& a, hipStream_t st);
+// D: head dim (fused_q: 256; else 256, 128 or 64)
+hipError_t launch_decode(const DecodeArgs& a, bool fused_q, int D, hipStream_t st);
+hipError_t launch_combine(const CombineArgs& a, int D, hipStream_t st);
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st);
 // fused gated prefill (q norm+RoPE prologue, sigmoid-gate epilogue), persistent
 // t0 / t1 (nullable): events stamped by the dispatch itself at the kernel's

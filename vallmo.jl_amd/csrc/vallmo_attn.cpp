@@ -136,8 +136,8 @@ int check_stride(int64_t s, const char* name) {
   } while (0)
 
 size_t decode_slots(int B, int Hk, int NW) { return (size_t)NW + (size_t)B * Hk; }
-size_t decode_part_o_bytes(int B, int Hk, int NW, int G) {
-  return decode_slots(B, Hk, NW) * G * vm::HEAD_DIM_ABI * sizeof(float);
+size_t decode_part_o_bytes(int B, int Hk, int NW, int G, int D) {
+  return decode_slots(B, Hk, NW) * G * D * sizeof(float);
 }
 size_t decode_part_ml_bytes(int B, int Hk, int NW, int G) {
   return decode_slots(B, Hk, NW) * G * 2 * sizeof(float);
@@ -329,12 +329,12 @@ int vm_knorm_rope_append(vm_bf16* kc, int64_t kc_st, int64_t kc_sh, int64_t kc_s
 }
 
 // ---- a5 -------------------------------------------------------------------
-// the tuned split-KV decode's workspace (D = 256, groups up to 8)
-static size_t tuned_decode_scratch_bytes(int B, int H, int Hk, int64_t ctx, int n_splits) {
+// the stream decode's workspace (D = 256, 128 or 64, groups up to 8)
+static size_t tuned_decode_scratch_bytes(int B, int H, int Hk, int D, int64_t ctx, int n_splits) {
   if (B <= 0 || H <= 0 || Hk <= 0 || H % Hk || ctx <= 0 || n_splits < 0) return 0;
   const int NW = vm::decode_stream_waves(B, Hk, n_splits);
   const int G = H / Hk;
-  const size_t pm_end = decode_part_o_bytes(B, Hk, NW, G) + decode_part_ml_bytes(B, Hk, NW, G);
+  const size_t pm_end = decode_part_o_bytes(B, Hk, NW, G, D) + decode_part_ml_bytes(B, Hk, NW, G);
   return (pm_end + 255) / 256 * 256 + decode_geom_bytes(B);
 }
 // the generic decode's workspace: one (Dv + 2)-float partial row per split,
@@ -349,12 +349,12 @@ size_t vm_decode_scratch_bytes(int B, int H, int Hk, int D, int64_t ctx, int n_s
   if (B <= 0 || H <= 0 || Hk <= 0 || H % Hk || ctx <= 0 || n_splits < 0) return 0;
   if (D < 16 || D > 512 || (D & (D - 1))) return 0;
   const size_t generic = generic_decode_scratch_bytes(B, H, Hk, D, ctx, n_splits);
-  if (D != vm::HEAD_DIM_ABI || H / Hk > 8) return generic;
-  return std::max(generic, tuned_decode_scratch_bytes(B, H, Hk, ctx, n_splits));
+  if ((D != vm::HEAD_DIM_ABI && D != 128 && D != 64) || H / Hk > 8) return generic;
+  return std::max(generic, tuned_decode_scratch_bytes(B, H, Hk, D, ctx, n_splits));
 }
 
 static int decode_common(vm::DecodeArgs& a, vm::CombineArgs& c, void* scratch, size_t scratch_bytes,
-                         int B, int H, int Hk, int64_t ctx, int n_splits) {
+                         int B, int H, int Hk, int D, int64_t ctx, int n_splits) {
   TRY(check_gqa(H, Hk));
   const int G = H / Hk;
   REQUIRE(G <= 8, VM_E_UNSUPPORTED, "decode: GQA group %d > 8 is not supported", G);
@@ -363,7 +363,7 @@ static int decode_common(vm::DecodeArgs& a, vm::CombineArgs& c, void* scratch, s
   REQUIRE((int64_t)B * ctx * Hk < ((int64_t)1 << 31), VM_E_UNSUPPORTED,
           "decode: B*Ctx*Hk = %lld token-heads exceeds 2^31", (long long)B * ctx * Hk);
   const int NW = vm::decode_stream_waves(B, Hk, n_splits);
-  const size_t po = decode_part_o_bytes(B, Hk, NW, G), pm = decode_part_ml_bytes(B, Hk, NW, G);
+  const size_t po = decode_part_o_bytes(B, Hk, NW, G, D), pm = decode_part_ml_bytes(B, Hk, NW, G);
   const size_t geo = (po + pm + 255) / 256 * 256;  // partition snapshot offset
   const size_t need = geo + decode_geom_bytes(B);
   REQUIRE(scratch != nullptr && scratch_bytes >= need, VM_E_SCRATCH,
@@ -401,9 +401,15 @@ int vm_decode_attention(vm_bf16* o, int64_t o_sh, int64_t o_sb, const vm_bf16* q
   TRY(check_gqa(H, Hk));
   REQUIRE(n_splits >= 0, VM_E_ARG, "decode: n_splits = %d", n_splits);
   REQUIRE(ctx > 0, VM_E_ARG, "decode: Ctx = %lld", (long long)ctx);
-  const bool tuned = Dk == vm::HEAD_DIM_ABI && Dv == Dk && H / Hk <= 8 && k_st == v_st &&
-                     k_sh == v_sh && k_sb == v_sb &&
-                     (int64_t)B * ctx * Hk < ((int64_t)1 << 31);
+  // The stream kernels take D = 256, 128 and 64, groups up to 8, one set of
+  // K/V strides and 2^31 token-heads. At D = 128 and 64 the generic kernel keeps
+  // what only it serves: a workspace sized for it alone, and its own limits.
+  bool tuned = (Dk == vm::HEAD_DIM_ABI || Dk == 128 || Dk == 64) && Dv == Dk && H / Hk <= 8 &&
+               k_st == v_st && k_sh == v_sh && k_sb == v_sb &&
+               (int64_t)B * ctx * Hk < ((int64_t)1 << 31);
+  if (Dk != vm::HEAD_DIM_ABI)
+    tuned = tuned && (int64_t)B * Hk <= 65535 && n_splits <= 65535 &&
+            scratch_bytes >= tuned_decode_scratch_bytes(B, H, Hk, Dk, ctx, n_splits);
   if (!tuned) {  // the generic split-KV kernel and its merge
     REQUIRE((int64_t)B * Hk <= 65535 && n_splits <= 65535, VM_E_UNSUPPORTED,
             "decode: B*Hk = %lld, n_splits = %d (at most 65535 each)", (long long)B * Hk,
@@ -432,17 +438,17 @@ int vm_decode_attention(vm_bf16* o, int64_t o_sh, int64_t o_sb, const vm_bf16* q
   const int64_t c_st = k_st, c_sh = k_sh, c_sb = k_sb;
   vm::DecodeArgs a{};
   vm::CombineArgs c{};
-  TRY(decode_common(a, c, scratch, scratch_bytes, B, H, Hk, ctx, n_splits));
+  TRY(decode_common(a, c, scratch, scratch_bytes, B, H, Hk, Dk, ctx, n_splits));
   if (B == 0) return VM_OK;
   a.q = q; a.q_sh = q_sh; a.q_sb = q_sb;
   // read-only here: the unfused operator appends nothing (k_new stays NULL)
   a.kc = const_cast<uint16_t*>(kc); a.vc = const_cast<uint16_t*>(vc);
   a.c_st = c_st; a.c_sh = c_sh; a.c_sb = c_sb;
   a.lengths = lengths;
-  int rc = hip_status(timed(VM_K_DECODE_SPLIT, S(st), [&] { return vm::launch_decode(a, false, S(st)); }), "decode_attention split");
+  int rc = hip_status(timed(VM_K_DECODE_SPLIT, S(st), [&] { return vm::launch_decode(a, false, Dk, S(st)); }), "decode_attention split");
   if (rc) return rc;
   c.out = o; c.o_sh = o_sh; c.o_sb = o_sb; c.gate = nullptr;
-  return hip_status(timed(VM_K_DECODE_COMBINE, S(st), [&] { return vm::launch_combine(c, S(st)); }), "decode_attention combine");
+  return hip_status(timed(VM_K_DECODE_COMBINE, S(st), [&] { return vm::launch_combine(c, Dk, S(st)); }), "decode_attention combine");
 }
 
 // ---- a6 -------------------------------------------------------------------
@@ -479,7 +485,7 @@ static int gated_attn_decode(vm_bf16* out, int64_t out_sb, const vm_bf16* qkv, i
           (long long)(2 * Hq + 2 * Hk) * D);
   vm::DecodeArgs a{};
   vm::CombineArgs c{};
-  TRY(decode_common(a, c, scratch, scratch_bytes, B, Hq, Hk, ctx, n_splits));
+  TRY(decode_common(a, c, scratch, scratch_bytes, B, Hq, Hk, D, ctx, n_splits));
   if (B == 0) return VM_OK;
   const int64_t Dl = D;
   // a3 + a4 + a5: split-KV attention with the q norm+RoPE prologue fused; the
@@ -491,13 +497,13 @@ static int gated_attn_decode(vm_bf16* out, int64_t out_sb, const vm_bf16* qkv, i
   a.lengths = positions;
   a.k_new = qkv + 2 * Hq * Dl; a.v_new = qkv + (2 * Hq + Hk) * Dl;
   a.new_sh = Dl; a.new_sb = qkv_sb;
-  int rc = hip_status(timed(VM_K_DECODE_SPLIT, S(st), [&] { return vm::launch_decode(a, true, S(st)); }), "gated_attn_decode split");
+  int rc = hip_status(timed(VM_K_DECODE_SPLIT, S(st), [&] { return vm::launch_decode(a, true, D, S(st)); }), "gated_attn_decode split");
   if (rc) return rc;
   // a5 merge + a6 gate, written as the Wo input (D, Hq, B); a12 advance fused
   c.out = out; c.o_sh = Dl; c.o_sb = out_sb;
   c.gate = qkv + Dl; c.g_sh = 2 * Dl; c.g_sb = qkv_sb;
   c.advance = advance ? positions : nullptr;
-  return hip_status(timed(VM_K_DECODE_COMBINE, S(st), [&] { return vm::launch_combine(c, S(st)); }), "gated_attn_decode combine");
+  return hip_status(timed(VM_K_DECODE_COMBINE, S(st), [&] { return vm::launch_combine(c, D, S(st)); }), "gated_attn_decode combine");
 }
 
 int vm_gated_attn_decode(vm_bf16* out, int64_t out_sb, const vm_bf16* qkv, int64_t qkv_sb,
@@ -524,7 +530,7 @@ int vm_gated_attn_decode_noalloc(vm_bf16* out, int64_t out_sb, const vm_bf16* qk
           "gated_attn_decode_noalloc: B = %d, Hq = %d, Hk = %d, Ctx = %lld, n_splits = %d", B,
           Hq, Hk, (long long)ctx, n_splits);
   TRY(check_head(D, half_rot));
-  const size_t need = tuned_decode_scratch_bytes(B > 0 ? B : 1, Hq, Hk, ctx, n_splits);
+  const size_t need = tuned_decode_scratch_bytes(B > 0 ? B : 1, Hq, Hk, vm::HEAD_DIM_ABI, ctx, n_splits);
   REQUIRE(need <= vm::DECODE_STATIC_SCRATCH_BYTES, VM_E_SCRATCH,
           "gated_attn_decode_noalloc: this step needs %zu bytes of workspace, more than the "
           "%zu-byte static workspace (use vm_gated_attn_decode with a caller buffer)",
