@@ -541,17 +541,17 @@ int vm_deltanet_sequence(float* o, const float* q, const float* k, const float* 
 
 /* deltanet_sequence! in its chunked form: the same arguments and results
  * (within 5e-4 of the sequential fp32 result, the tests' bar), computed per
- * 64-token chunk as a lower-triangular solve and matrix products (delta = U -
- * W S_0, O = gamma Q S_0 + M delta, S_C = gamma_C S_0 + K~^T delta: the
- * sequential recurrence's exact algebra) on the bf16 MFMA in split precision
+ * 64-token chunk as a lower-triangular solve and matrix products (delta = T
+ * (beta V - beta gamma K S_0), O = gamma Q S_0 + M delta, S_C = gamma_C S_0 +
+ * K~^T delta: the sequential recurrence's exact algebra) on the bf16 MFMA in split precision
  * (each fp32 operand as bf16 hi + lo, products hi hi + hi lo + lo hi, fp32
  * accumulation and state), the chunks' state carried by one sequential scan. No separate reference
  * function: the reference runs the sequential loop (deltanet_recurrent.jl:
  * 109-172); this is the same operator, parallel over each chunk: a chunk
- * kernel, one sequential scan over the chunks' states, and a chunk-parallel
- * output kernel. workspace: vm_deltanet_sequence_workspace_bytes(T, Hv, B)
- * bytes, 256-byte aligned (about 197 KB per 64-token chunk per value head
- * and sequence). */
+ * kernel, then one sequential scan over the chunks' states that also forms O;
+ * T <= 36 runs the sequential kernel. workspace:
+ * vm_deltanet_sequence_workspace_bytes(T, Hv, B) bytes, 256-byte aligned
+ * (about 132 KB per 64-token chunk per value head and sequence). */
 size_t vm_deltanet_sequence_workspace_bytes(int T, int Hv, int B);
 int vm_deltanet_sequence_chunked(float* o, const float* q, const float* k, const float* v,
                                  const float* beta, const float* gate, const float* s_in,
@@ -561,8 +561,8 @@ int vm_deltanet_sequence_chunked(float* o, const float* q, const float* k, const
 /* forward(::DeltaNetLayer)'s recurrence and gated norm in one call
  * (src/llm/qwen35.jl:357-364: deltanet_sequence! into O, then y = O rstd
  * NormWeight silu(z), the out projection's input): the chunked recurrence of
- * vm_deltanet_sequence_chunked with the norm applied in its output kernel,
- * so O never reaches memory. y, z :: (Dv, Hv, T, B) bf16 rows at token
+ * vm_deltanet_sequence_chunked with O (fp32) in the workspace, then the norm
+ * as vm_gated_rms_norm. y, z :: (Dv, Hv, T, B) bf16 rows at token
  * stride *_st and sequence stride *_sb (heads contiguous), as
  * vm_gated_rms_norm; the state and workspace as vm_deltanet_sequence_chunked. */
 int vm_deltanet_sequence_chunked_gated_norm(vm_bf16* y, int64_t y_st, int64_t y_sb,

@@ -496,6 +496,36 @@ def test_deltanet_sequence_chunked(vm, orc, B, T):
         assert err <= 5e-4, name
 
 
+@pytest.mark.parametrize("Hk,Hv,B,T", [(2, 2, 1, 36), (2, 2, 1, 37), (1, 3, 2, 64), (8, 8, 1, 129),
+                                       (2, 8, 1, 191)])
+def test_deltanet_sequence_chunked_groups(vm, orc, Hk, Hv, B, T):
+    """The chunked form at value-head groups of 1, 3 and 4 (phase 1 takes two value
+    heads a workgroup, the last one alone), qk heads that do and do not spread
+    over the XCDs, both sides of the sequential kernel's range (T = 36) and
+    chunk edges: 5e-4 of the largest value, as the tests above."""
+    banner(f"deltanet sequence chunked Hk={Hk} Hv={Hv} B={B} T={T}")
+    rng = np.random.default_rng(Hk * 1000 + Hv * 100 + T)
+    unit = lambda x: (x / np.linalg.norm(x, axis=-1, keepdims=True)).astype(np.float32)
+    q = unit(rng.standard_normal((B, Hk, T, DK))) / np.float32(np.sqrt(DK))
+    k = unit(rng.standard_normal((B, Hk, T, DK)))
+    v = rng.standard_normal((B, Hv, T, DV)).astype(np.float32)
+    beta = rng.uniform(0.05, 0.95, (B, T, Hv)).astype(np.float32)
+    gate = -rng.uniform(0.001, 1.0, (B, T, Hv)).astype(np.float32)
+    s = (0.05 * rng.standard_normal((B, Hv, DV, DK))).astype(np.float32)
+    o_ref, s_ref = orc.deltanet_sequence(q, k, v, beta, gate, s)
+    S = f32dev(s)
+    o = torch.empty((B, Hv, T, DV), dtype=torch.float32, device="cuda")
+    ws = torch.full((vm.deltanet_sequence_workspace_bytes(T, Hv, B),), 255, dtype=torch.uint8,
+                    device="cuda")
+    vm.deltanet_sequence_chunked_({"O": o, "Sp": S}, f32dev(q), f32dev(k), f32dev(v), f32dev(beta),
+                                  f32dev(gate), S, workspace=ws)
+    torch.cuda.synchronize()
+    for got, ref, name in ((o.cpu().numpy(), o_ref, "O"), (S.cpu().numpy(), s_ref, "S")):
+        err = np.abs(got - ref).max() / np.abs(ref).max()
+        print(f"chunked {name}: max err / max |ref| = {err:.2e}")
+        assert err <= 5e-4, name
+
+
 @pytest.mark.parametrize("B,T,off", [(1, 100, 0), (2, 65, 8), (1, 1, 0), (3, 129, 0)])
 def test_deltanet_sequence_chunked_gated_norm(vm, orc, B, T, off):
     """forward(::DeltaNetLayer)'s recurrence and gated norm as one call

@@ -373,53 +373,46 @@ __global__ __launch_bounds__(256) void deltanet_sequence_kernel(DeltaSeqArgs a) 
 // Over a chunk of C tokens (G the in-chunk cumulative log decay, gamma = exp G,
 // D_ij = gamma_i / gamma_j) the recurrence's per-token corrections delta_i =
 // beta_i (v_i - alpha_i S_{i-1}^T k_i) satisfy the lower-triangular system
-//     (I + L) delta = beta V - (beta gamma K) S_0,   L_ij = beta_i D_ij k_i.k_j (i > j)
-// so delta = U - W S_0 with U = (I + L)^-1 beta V, W = (I + L)^-1 beta gamma K;
-// then O = gamma Q S_0 + M delta with M_ij = D_ij q_i.k_j (j <= i), and
-// S_C = gamma_C S_0 + K~^T delta with K~_j = (gamma_C / gamma_j) k_j (exact
-// algebra of the sequential update; fp32 throughout). Three launches:
-// Phase 1 (deltanet_chunk_kernel, chunk-parallel): the Gram K K^T and the
-// products [U | W] = T [beta V | beta gamma K] with T = (I + L)^-1 on the bf16
-// MFMA in split precision (see phase 3), T itself by fp32 forward
-// substitution, and the operands of the state chain (-W, K~^T split, U,
-// gamma_C) written in the operand orders phase 2 loads them in, 16 bytes per
-// lane, so phase 2 reads 1 KB contiguous per wave load.
+//     (I + L) delta = beta (V - gamma K S_0),   L_ij = beta_i D_ij k_i.k_j (i > j)
+// so delta = T R with T = (I + L)^-1 and R = beta V - beta gamma (K S_0); then
+// O = gamma (Q S_0) + M delta with M_ij = D_ij q_i.k_j (j <= i), and
+// S_C = gamma_C S_0 + K^T (e delta) with e_j = gamma_C / gamma_j (exact algebra
+// of the sequential update). Two launches, and the gated norm as a third:
+// Phase 1 (deltanet_chunk_kernel, chunk-parallel): what does not depend on the
+// state: the Gram K K^T and Q K^T once per qk head, then per value head L, T by
+// fp32 forward substitution, M, and the rows' decays.
 // Phase 2 (deltanet_scan_kernel, sequential over chunks): one workgroup per 16
-// state columns of a value head; per chunk 24 split-precision MFMAs per wave
-// (delta, then the state, fp32 accumulators), writing each chunk's start state
-// S_0 and its delta for phase 3, the next chunk's operands loading into a
-// second register set meanwhile. The state and delta pass between the waves
-// through LDS split and transposed ([column][k]), so that a B operand is one
-// 16-byte read.
-// Phase 3 (deltanet_out_kernel, chunk-parallel): Q K^T, M and O = gamma Q S_0 +
-// M delta on the bf16 MFMA (v_mfma_f32_16x16x32_bf16) in split precision:
-// each fp32 operand x is hi = bf16(x) and lo = bf16(x - hi), and a product is
-// hi hi + hi lo + lo hi with fp32 accumulation (about 2^-16 relative per
-// product), then either O (fp32, the operator's output) or, fused, the layer's
-// gated RMSNorm with z (qwen35.jl:360-364) in bf16. The scan writes S_0 and
-// delta already split, in that MFMA's B operand order.
+// state columns of a value head. Four waves carry the state chain (K S_0, T R,
+// the state), four others form and store O beside them and stage the next K.
+// Phase 3, fused form only: the layer's gated RMSNorm with z (qwen35.jl:360-364)
+// on O, gated_rms_norm_*_kernel.
+// Little passes between the phases: T, M and the decays, 33 KB per (chunk, value
+// head), and K and Q split, 64 KB per (chunk, qk head), which the column blocks
+// of all its value heads share in one XCD's L2. (-W, K~^T and U took 98 KB per
+// value head, and S_0 and delta, passed on to an output kernel, another 98 KB.)
+// The products run on the bf16 MFMA (v_mfma_f32_16x16x32_bf16) in split
+// precision: each fp32 operand x is hi = bf16(x) and lo = bf16(x - hi), and a
+// product is hi hi + hi lo + lo hi with fp32 accumulation (about 2^-16
+// relative per product).
 namespace {
 constexpr int DC = 64;   // chunk length
 constexpr int CBW = 16;  // state columns per scan workgroup
-// per (chunk, value head, sequence) unit of the scan's operands, floats
-// (-W and K~^T split into bf16 hi / lo in the A operand order of
-// v_mfma_f32_16x16x32_bf16, 8 bf16 per lane: lane l element j = A[16 tile + l %
-// 16][32 ks + 8 (l / 16) + j]; U fp32 in accumulator order)
-constexpr int UO_W = 0;      // -W:   [w 4][ks 4][hl 2][lane][8] bf16, A[i = r][k = dk]
-constexpr int UO_K = 8192;   // K~^T: [d 8][ks 2][hl 2][lane][8] bf16, A[i = dk][k = r]
-constexpr int UO_U = 16384;  // U:    [cb 8][w 4][lane][4] floats, D[r][dv] tiles
-constexpr int UO_G = 24576;  // gamma_C
-constexpr int UNIT = 24640;  // floats per unit (98 560 B, a multiple of 256)
-// per (chunk, value head, sequence), written by the scan for phase 3, in
-// float-sized units: S_0 and delta split into bf16 hi and lo parts, in the B
-// operand order of v_mfma_f32_16x16x32_bf16 for column block cb and 32-deep k
-// step ks: [cb 8][ks][hl 2][lane 64][8] bf16 with lane l element j =
-// X[32 ks + 8 (l / 16) + j][16 cb + l % 16] (hl 0: hi, 1: lo); ks < 4 for S_0
-// (k = dk), ks < 2 for delta (k = the chunk's token)
-constexpr int S0_UNIT = DN_D * DN_D;
-constexpr int DL_UNIT = DC * DN_D;
+// per (chunk, value head, sequence) unit of phase 1's results, floats. T and M
+// are split into bf16 hi / lo in the A operand order of
+// v_mfma_f32_16x16x32_bf16: [row tile w 4][k step ks 2][hl 2][lane 64][8] with
+// lane l element j = X[16 w + l % 16][32 ks + 8 (l / 16) + j]; the blocks ks >
+// w / 2 lie above the diagonal and are neither written nor read
+constexpr int UO_T = 0;
+constexpr int UO_M = 4096;
+constexpr int UO_SC = 8192;  // [beta 64][beta gamma 64][gamma_C / gamma 64][gamma 64]
+constexpr int UNIT = 8448;   // floats per unit (33 792 B, a multiple of 256)
+// per (chunk, qk head, sequence): K split, [hl 2][token 64][dk 128] bf16 (rows
+// past the sequence's end 0), and Q split in A operand order, [row tile w 4][k
+// step ks 4][hl 2][lane 64][8] bf16 (rows past the end repeat the last)
+constexpr int KQ_Q = 8192;
+constexpr int KQ_UNIT = 16384;  // floats per unit (64 KB)
 
-// the chunk's inclusive cumulative log decay (wave 0, one token per lane; log
+// the chunk's inclusive cumulative log decay (one wave, one token per lane; log
 // decays below -110 are taken as -110: expf underflows to exactly 0 below
 // about -104, so every decay the recurrence applies is unchanged, while the
 // cumulative sums stay finite; a -inf log decay, e.g. from softplus
@@ -438,20 +431,14 @@ __device__ __forceinline__ float chunk_cumsum(const DeltaSeqArgs& q, int b, int 
 }
 }  // namespace
 
-// the (chunk, value head, sequence) workspaces of the three phases
-__host__ __device__ __forceinline__ int64_t dn_units_floats(int NC) { return (int64_t)(NC + 1) * UNIT; }
-__host__ __device__ __forceinline__ int64_t dn_s0_floats(int NC) { return (int64_t)(NC + 1) * S0_UNIT; }
-__host__ __device__ __forceinline__ int64_t dn_dl_floats(int NC) { return (int64_t)(NC + 1) * DL_UNIT; }
-__device__ __forceinline__ float* dn_units(const DeltaChunkArgs& a, int b, int hv, int NC) {
-  return a.ws + ((int64_t)b * a.s.Hv + hv) * dn_units_floats(NC);
+// the workspace: the units of every (sequence, value head, chunk), the K and Q
+// units of every (sequence, qk head, chunk), then the fused form's O (fp32)
+__device__ __forceinline__ float* dn_unit(const DeltaChunkArgs& a, int b, int hv, int NC, int c) {
+  return a.ws + (((int64_t)b * a.s.Hv + hv) * NC + c) * UNIT;
 }
-__device__ __forceinline__ float* dn_s0(const DeltaChunkArgs& a, int b, int hv, int NC) {
-  return a.ws + (int64_t)a.s.B * a.s.Hv * dn_units_floats(NC) +
-         ((int64_t)b * a.s.Hv + hv) * dn_s0_floats(NC);
-}
-__device__ __forceinline__ float* dn_dl(const DeltaChunkArgs& a, int b, int hv, int NC) {
-  return a.ws + (int64_t)a.s.B * a.s.Hv * (dn_units_floats(NC) + dn_s0_floats(NC)) +
-         ((int64_t)b * a.s.Hv + hv) * dn_dl_floats(NC);
+__device__ __forceinline__ uint16_t* dn_kq(const DeltaChunkArgs& a, int b, int hk, int NC, int c) {
+  return reinterpret_cast<uint16_t*>(a.ws + (int64_t)a.s.B * a.s.Hv * NC * UNIT +
+                                     (((int64_t)b * a.s.Hk + hk) * NC + c) * KQ_UNIT);
 }
 
 namespace {
@@ -477,136 +464,132 @@ __device__ __forceinline__ f32x4 mfma_x3(const uint4& ah, const uint4& al, const
   acc = mfma16(ah, bl, acc);
   return mfma16(ah, bh, acc);
 }
-constexpr int KSW = DN_D + 4;  // LDS row of K (floats; 16-byte aligned, banks skewed)
-constexpr int LSW = DC + 4;    // LDS row of L (floats)
-constexpr int TW = DC + 8;     // LDS row of T hi / lo (bf16)
+__device__ __forceinline__ uint4 lds16(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+constexpr int KW = DN_D + 8;  // LDS row of K hi / lo (bf16; 16-byte aligned, banks skewed)
+constexpr int LSW = DC + 4;   // LDS row of L (floats)
+constexpr int TW = DC + 8;    // LDS row of T hi / lo (bf16)
 }  // namespace
 
-// One workgroup per (chunk, value head, sequence). Wave w forms Gram row block
-// w into L (L[i][j] = beta_i gamma_i / gamma_j k_i . k_j below the diagonal),
-// then wave 3 solves (I + L) T = I, lane c for column c, in fp32 (row i + 1 of
-// L read from LDS while row i is reduced), and stores T split into bf16 hi /
-// lo over L, while waves 0-2 write K~^T and gather their operands of the
-// products below. Then waves 0, 1 form U = T (beta V) (value columns 64 w ..)
-// in the scan's accumulator order, and waves 2, 3 form W^T = (beta gamma K)^T
-// T^T (key columns 64 (w - 2) ..): their A operand lane l of tile ct gathers
-// key column 32 (ct / 2) + 4 (ct % 2) + 8 ((l % 16) / 4) + l % 4, so that
-// result tiles 2 h, 2 h + 1, lane l reg r hold W[i][32 h + 8 (l / 16) + 4 (tile
-// % 2) + r]: 8 consecutive keys per lane, the -W operand order of the scan.
-// (three waves per SIMD: the phases are latency-bound, and three workgroups fit a CU's LDS)
+// Phase 1. One workgroup per (chunk, two value heads of a qk head, sequence). Wave w
+// takes rows i = 16 w .. of G = K K^T and P = Q K^T (lane l: row 16 w + l % 16, reg r of tile jt <=
+// w: column 16 jt + 4 (l / 16) + r; tiles above the diagonal are not formed).
+// Then every wave writes its rows of each head's L (LDS) and M (workspace); wave 3 solves (I + L) T = I for the first head and wave 2 for
+// the second, lane c for column c, in fp32 (L's rows read from LDS ahead of
+// their use); T, split, goes through LDS into the operand order.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 void deltanet_chunk_kernel(DeltaChunkArgs a) {
   const DeltaSeqArgs& q = a.s;
-  const int c = blockIdx.x, hv = blockIdx.y, b = blockIdx.z, t = threadIdx.x;
+  const int R = q.Hv / q.Hk, RP = (R + 1) / 2;
+  const int c = blockIdx.x, hk = blockIdx.y / RP, b = blockIdx.z, t = threadIdx.x;
+  const int hv0 = hk * R + 2 * (blockIdx.y % RP);   // the workgroup's value heads
+  const int nr = min(2, hk * R + R - hv0);
   const int lane = t & 63, l16 = lane & 15, r4 = lane >> 4;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // wave-uniform: scalar branches
-  const int hk = hv / (q.Hv / q.Hk);
   const int t0 = c * DC, n = min(DC, q.T - t0);
   const int NC = (q.T + DC - 1) / DC;
-  float* u = dn_units(a, b, hv, NC) + (int64_t)c * UNIT;
-  if (c == 0) {  // unit NC: the identity chunk (all zero, gamma_C = 1), the scan's pad
-    float* id = u + (int64_t)NC * UNIT;
-    for (int i = t; i < UNIT / 4; i += 256)
-      reinterpret_cast<float4*>(id)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    __syncthreads();
-    if (t == 0) id[UO_G] = 1.f;
-  }
-  // K rows, and L, later T (hi, lo) in its place: ~52 KB, three workgroups per CU
-  __shared__ __attribute__((aligned(16))) float Ks[DC * KSW];
-  __shared__ __attribute__((aligned(16))) float LT[DC * TW];
-  static_assert(sizeof(LT) >= DC * LSW * sizeof(float), "L");
-  __shared__ __attribute__((aligned(16))) float Gs[DC], Bs[DC], Es[DC], Ek[DC];
-  uint16_t* const Th = reinterpret_cast<uint16_t*>(LT);
-  uint16_t* const Tl = Th + DC * TW;
+  // K split (rows of KW), then in its place L and later T (hi, lo) of two heads
+  __shared__ __attribute__((aligned(16))) float LT[2][DC * TW];
+  static_assert(sizeof(LT) >= 2 * DC * KW * sizeof(uint16_t), "K hi, lo");
+  static_assert(sizeof(LT[0]) >= DC * LSW * sizeof(float), "L");
+  __shared__ __attribute__((aligned(16))) float Gs[2][DC], Bs[2][DC];
+  uint16_t* const Kh = reinterpret_cast<uint16_t*>(LT);
+  uint16_t* const Kl = Kh + DC * KW;
   const float* kp = q.k + (((int64_t)b * q.Hk + hk) * q.T + t0) * DN_D;
-  {  // K: float4 t + 256 m = (row, column group) ((t + 256 m) / 32, t % 32), all loads in flight at once
-    float4 kv[DC / 8];
+  const float* qp = q.q + (((int64_t)b * q.Hk + hk) * q.T + t0) * DN_D;
+  const int i = 16 * w + l16;  // this lane's row of G, P, L and M
+  uint4 qh[4], ql[4];          // Q[i][32 ks + 8 (l / 16) ..], split
+  uint16_t* const kq = dn_kq(a, b, hk, NC, c);
+  const bool first = blockIdx.y % RP == 0;  // this workgroup writes the qk head's K and Q
+  {
+    f32x4 kv[DC / 8], qv[8];
 #pragma unroll
-    for (int m = 0; m < DC / 8; ++m)
-      kv[m] = *reinterpret_cast<const float4*>(kp + min((t >> 5) + 8 * m, n - 1) * DN_D + 4 * (t & 31));
-    float bt = 0.f;
-    if (t < 64) {  // wave 0: beta, gates, inclusive cumulative sum of the log decay
-      bt = q.beta[((int64_t)b * q.T + t0 + min(t, n - 1)) * q.Hv + hv];
-      const float G = chunk_cumsum(q, b, hv, t0, n, t);
-      Gs[t] = G;
-      Bs[t] = t < n ? bt : 0.f;
-      Es[t] = expf(G);
-      Ek[t] = expf(__shfl(G, DC - 1) - G);  // gamma_C / gamma_t
+    for (int m = 0; m < DC / 8; ++m)  // float4 t + 256 m of the chunk's K
+      kv[m] = *reinterpret_cast<const f32x4*>(kp + min((t >> 5) + 8 * m, n - 1) * DN_D + 4 * (t & 31));
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        qv[2 * ks + u] = *reinterpret_cast<const f32x4*>(qp + (int64_t)min(i, n - 1) * DN_D + 32 * ks +
+                                                         8 * r4 + 4 * u);
+    if (w < nr) {  // wave w: beta, the cumulative log decay and the decays of its value head
+      const int hv = hv0 + w;
+      const float bt = lane < n ? q.beta[((int64_t)b * q.T + t0 + lane) * q.Hv + hv] : 0.f;
+      const float g = chunk_cumsum(q, b, hv, t0, n, lane), eg = expf(g);
+      Gs[w][lane] = g;
+      Bs[w][lane] = bt;
+      float* sc = dn_unit(a, b, hv, NC, c) + UO_SC + lane;
+      sc[0] = bt;
+      sc[64] = bt * eg;
+      sc[128] = expf(__shfl(g, DC - 1) - g);
+      sc[192] = eg;
     }
 #pragma unroll
     for (int m = 0; m < DC / 8; ++m) {  // rows past the end read as 0
       const int r = (t >> 5) + 8 * m;
-      *reinterpret_cast<float4*>(&Ks[r * KSW + 4 * (t & 31)]) = r < n ? kv[m] : make_float4(0.f, 0.f, 0.f, 0.f);
+      uint2 hi, lo;
+      split4(kv[m], hi, lo);
+      if (r >= n) hi = lo = make_uint2(0, 0);
+      *reinterpret_cast<uint2*>(&Kh[r * KW + 4 * (t & 31)]) = hi;
+      *reinterpret_cast<uint2*>(&Kl[r * KW + 4 * (t & 31)]) = lo;
+      if (first) {
+        *reinterpret_cast<uint2*>(kq + 4 * (t + 256 * m)) = hi;
+        *reinterpret_cast<uint2*>(kq + DC * DN_D + 4 * (t + 256 * m)) = lo;
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      split8(qv[2 * ks], qv[2 * ks + 1], qh[ks], ql[ks]);
+      if (first) {
+        uint16_t* const qo = kq + 2 * KQ_Q + (w * 4 + ks) * 1024 + lane * 8;
+        *reinterpret_cast<uint4*>(qo) = qh[ks];
+        *reinterpret_cast<uint4*>(qo + 512) = ql[ks];
+      }
     }
   }
   __syncthreads();
-  {  // Gram tiles (w, jt), jt <= w: lane l reg r = k_i . k_j, i = 16 w + 4 (l / 16) + r, j = 16 jt + l % 16
-    uint4 ah[4], al[4];
+  f32x4 G[4], P[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const float* kr = &Ks[(16 * w + l16) * KSW + 32 * ks + 8 * r4];
-      split8(*reinterpret_cast<const f32x4*>(kr), *reinterpret_cast<const f32x4*>(kr + 4), ah[ks], al[ks]);
-    }
+  for (int jt = 0; jt < 4; ++jt) G[jt] = P[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    const int o = 32 * ks + 8 * r4;
+    const uint4 bh = lds16(&Kh[i * KW + o]), bl = lds16(&Kl[i * KW + o]);
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) {
       if (jt > w) break;
-      f32x4 G = f32x4{0.f, 0.f, 0.f, 0.f};
+      const uint4 ah = lds16(&Kh[(16 * jt + l16) * KW + o]), al = lds16(&Kl[(16 * jt + l16) * KW + o]);
+      G[jt] = mfma_x3(ah, al, bh, bl, G[jt]);
+      P[jt] = mfma_x3(ah, al, qh[ks], ql[ks], P[jt]);
+    }
+  }
+  __syncthreads();  // K read: L takes its place
+  for (int rr = 0; rr < nr; ++rr) {
+    uint16_t* const mo =
+        reinterpret_cast<uint16_t*>(dn_unit(a, b, hv0 + rr, NC, c) + UO_M) + w * 2048;
+    const float Gi = Gs[rr][i], Bi = Bs[rr][i];
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const float* kr = &Ks[(16 * jt + l16) * KSW + 32 * ks + 8 * r4];
-        uint4 bh, bl;
-        split8(*reinterpret_cast<const f32x4*>(kr), *reinterpret_cast<const f32x4*>(kr + 4), bh, bl);
-        G = mfma_x3(ah[ks], al[ks], bh, bl, G);
-      }
-      const int j = 16 * jt + l16;
+    for (int jt = 0; jt < 4; ++jt) {
+      if (jt > (w | 1)) break;
+      const f32x4 Gj = *reinterpret_cast<const f32x4*>(&Gs[rr][16 * jt + 4 * r4]);
+      f32x4 l, m;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = 16 * w + 4 * r4 + r;
-        LT[i * LSW + j] = i > j ? Bs[i] * expf(Gs[i] - Gs[j]) * G[r] : 0.f;
+        const int j = 16 * jt + 4 * r4 + r;
+        const float d = expf(Gi - Gj[r]);
+        l[r] = i > j ? Bi * d * G[jt][r] : 0.f;
+        m[r] = (j <= i && i < n) ? d * P[jt][r] : 0.f;
       }
+      *reinterpret_cast<f32x4*>(&LT[rr][i * LSW + 16 * jt + 4 * r4]) = l;
+      uint2 mh, ml;
+      split4(m, mh, ml);
+      const int l2 = 16 * (2 * (jt & 1) + (r4 >> 1)) + l16;  // operand lane of these 4 columns
+      uint16_t* const d = mo + (jt >> 1) * 1024 + l2 * 8 + 4 * (r4 & 1);
+      *reinterpret_cast<uint2*>(d) = mh;
+      *reinterpret_cast<uint2*>(d + 512) = ml;
     }
   }
   __syncthreads();
-  // the products' operands from V or K (rows j = 32 ks + 8 (l / 16) + e of R),
-  // scaled and split: waves 0, 1 B = beta_j V[j][64 w + 16 ct + l % 16] (rows past
-  // the end: beta = 0), waves 2, 3 A = beta_j gamma_j K[j][key column]
-  const bool uw = w < 2;
-  uint4 rh[2][4], rl[2][4];  // [ks][ct]
-  auto gather = [&]() __attribute__((always_inline)) {
-    const float* vp = q.v + (((int64_t)b * q.Hv + hv) * q.T + t0) * DN_D + 64 * (w & 1) + l16;
-    // gathered key column of tile ct: 64 (w % 2) + 32 (ct / 2) + 4 (ct % 2) + pc
-    const int pc = 64 * (w & 1) + 8 * (l16 >> 2) + (l16 & 3);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int j0 = 32 * ks + 8 * r4;
-      f32x4 s0 = *reinterpret_cast<const f32x4*>(&Bs[j0]), s1 = *reinterpret_cast<const f32x4*>(&Bs[j0 + 4]);
-      if (!uw) {
-        s0 = s0 * *reinterpret_cast<const f32x4*>(&Es[j0]);
-        s1 = s1 * *reinterpret_cast<const f32x4*>(&Es[j0 + 4]);
-      }
-      f32x4 r0[4], r1[4];
-      if (uw) {
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            r0[ct][e] = vp[(int64_t)min(j0 + e, n - 1) * DN_D + 16 * ct];
-            r1[ct][e] = vp[(int64_t)min(j0 + 4 + e, n - 1) * DN_D + 16 * ct];
-          }
-      } else {
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            r0[ct][e] = Ks[(j0 + e) * KSW + pc + 32 * (ct >> 1) + 4 * (ct & 1)];
-            r1[ct][e] = Ks[(j0 + 4 + e) * KSW + pc + 32 * (ct >> 1) + 4 * (ct & 1)];
-          }
-      }
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct) split8(r0[ct] * s0, r1[ct] * s1, rh[ks][ct], rl[ks][ct]);
-    }
-  };
-  if (w == 3) {
+  if (3 - w < nr) {
     // (I + L) T = I: lane c holds column c (rows above c stay 0, T[c][c] = 1).
     // The float4s of L's rows 1 .. 63 (j < i) are read in order through a ring
     // of SD registers, SD ahead of their use (the cursor (pi, pj) is a
@@ -615,26 +598,27 @@ void deltanet_chunk_kernel(DeltaChunkArgs a) {
     // tiles on it are written whole) times x[j] = 0, and a load whose every
     // register is used keeps the allocator from reloading into one in flight.
     constexpr int SD = 12;
+    const float* const L = LT[3 - w];
     float x[DC];
 #pragma unroll
-    for (int i = 0; i < DC; ++i) x[i] = 0.f;
+    for (int k = 0; k < DC; ++k) x[k] = 0.f;
     f32x4 ring[SD];
     int pi = 1, pj = 0;  // next float4 to read: row pi, columns 4 pj ..
 #pragma unroll
     for (int d = 0; d < SD; ++d) {
-      ring[d] = *reinterpret_cast<const f32x4*>(&LT[pi * LSW + 4 * pj]);
+      ring[d] = *reinterpret_cast<const f32x4*>(&L[pi * LSW + 4 * pj]);
       if (4 * (pj + 1) < pi) ++pj; else { ++pi; pj = 0; }
     }
     x[0] = lane == 0 ? 1.f : 0.f;
     int idx = 0;
 #pragma unroll
-    for (int i = 1; i < DC; ++i) {
-      float acc[4] = {i == lane ? 1.f : 0.f, 0.f, 0.f, 0.f};
+    for (int k = 1; k < DC; ++k) {
+      float acc[4] = {k == lane ? 1.f : 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j4 = 0; 4 * j4 < i; ++j4) {
+      for (int j4 = 0; 4 * j4 < k; ++j4) {
         const f32x4 l4 = ring[idx % SD];
         if (pi < DC) {
-          ring[idx % SD] = *reinterpret_cast<const f32x4*>(&LT[pi * LSW + 4 * pj]);
+          ring[idx % SD] = *reinterpret_cast<const f32x4*>(&L[pi * LSW + 4 * pj]);
           if (4 * (pj + 1) < pi) ++pj; else { ++pi; pj = 0; }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -642,461 +626,324 @@ void deltanet_chunk_kernel(DeltaChunkArgs a) {
         for (int e = 0; e < 4; ++e) acc[e] -= l4[e] * x[4 * j4 + e];
         ++idx;
       }
-      x[i] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      x[k] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     }
     // T rows, split: columns (c & ~1, c | 1) as one pair, lane c even stores the
     // hi pair, odd the lo pair (L is dead: every read of it is above)
+    uint16_t* const Tx = reinterpret_cast<uint16_t*>(LT[3 - w]) + ((lane & 1) ? DC * TW : 0);
 #pragma unroll
-    for (int i = 0; i < DC; ++i) {
-      const float xo = __shfl_xor(x[i], 1);
-      const float x0 = (lane & 1) ? xo : x[i], x1 = (lane & 1) ? x[i] : xo;
+    for (int k = 0; k < DC; ++k) {
+      const float xo = xor32<1>(x[k]);
+      const float x0 = (lane & 1) ? xo : x[k], x1 = (lane & 1) ? x[k] : xo;
       const uint32_t hi = pack2(x0, x1);
       const uint32_t lo = pack2(x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xffff0000u));
-      *reinterpret_cast<uint32_t*>(((lane & 1) ? Tl : Th) + i * TW + (lane & ~1)) = (lane & 1) ? lo : hi;
+      *reinterpret_cast<uint32_t*>(Tx + k * TW + (lane & ~1)) = (lane & 1) ? lo : hi;
     }
-  } else {
-    // K~^T split, in operand order: slot f = (tile d, ks) = (f / 128, (f / 64) % 2),
-    // lane f % 64: dk 16 d + l % 16, r = 32 ks + 8 (l / 16) + j
-    uint16_t* const kt = reinterpret_cast<uint16_t*>(u + UO_K);
-    for (int f = t; f < 1024; f += 192) {
-      const int l = f & 63, dk = 16 * (f >> 7) + (l & 15), r0 = 32 * ((f >> 6) & 1) + 8 * (l >> 4);
-      f32x4 v0, v1;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v0[e] = Ek[r0 + e] * Ks[(r0 + e) * KSW + dk];
-        v1[e] = Ek[r0 + 4 + e] * Ks[(r0 + 4 + e) * KSW + dk];
-      }
-      uint4 hi, lo;
-      split8(v0, v1, hi, lo);
-      *reinterpret_cast<uint4*>(kt + ((2 * (f >> 6) + 0) * 64 + l) * 8) = hi;
-      *reinterpret_cast<uint4*>(kt + ((2 * (f >> 6) + 1) * 64 + l) * 8) = lo;
-    }
-    if (t == 0) u[UO_G] = expf(Gs[DC - 1]);
-    gather();
   }
   __syncthreads();
-  if (w == 3) gather();
-  f32x4 acc[4][4];  // [row tile][column tile] (U) or [column tile][row tile] (W^T)
+  for (int rr = 0; rr < nr; ++rr) {
+    uint16_t* const to =
+        reinterpret_cast<uint16_t*>(dn_unit(a, b, hv0 + rr, NC, c) + UO_T) + w * 2048;
+    const uint16_t* const Th = reinterpret_cast<const uint16_t*>(LT[rr]);
 #pragma unroll
-  for (int x = 0; x < 4; ++x)
+    for (int ks = 0; ks < 2; ++ks) {
+      if (ks > (w >> 1)) break;
 #pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int j0 = 32 * ks + 8 * r4;
-    uint4 th[4], tl[4];  // T[16 rt + l % 16][j0 ..]
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      th[rt] = *reinterpret_cast<const uint4*>(&Th[(16 * rt + l16) * TW + j0]);
-      tl[rt] = *reinterpret_cast<const uint4*>(&Tl[(16 * rt + l16) * TW + j0]);
+      for (int hl = 0; hl < 2; ++hl)
+        *reinterpret_cast<uint4*>(to + (ks * 2 + hl) * 512 + lane * 8) =
+            lds16(Th + hl * DC * TW + i * TW + 32 * ks + 8 * r4);
     }
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct)
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        if (uw)
-          acc[rt][ct] = mfma_x3(th[rt], tl[rt], rh[ks][ct], rl[ks][ct], acc[rt][ct]);
-        else
-          acc[ct][rt] = mfma_x3(rh[ks][ct], rl[ks][ct], th[rt], tl[rt], acc[ct][rt]);
-      }
-  }
-  if (uw) {  // U tile (rt, column block 4 w + ct): lane l reg r = U[16 rt + 4 (l / 16) + r][..]
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct)
-        *reinterpret_cast<f32x4*>(u + UO_U + (((4 * w + ct) * 4 + rt) * 64 + lane) * 4) = acc[rt][ct];
-  } else {  // -W, row tile rt, k step ks = 2 (w - 2) + h: tiles 2 h, 2 h + 1 hold
-            // lane l's dk 32 ks + 8 (l / 16) + j, j < 4 and j >= 4
-    uint16_t* const wm = reinterpret_cast<uint16_t*>(u + UO_W);
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        const int ks = 2 * (w - 2) + h;
-        uint4 hi, lo;
-        split8(-acc[2 * h][rt], -acc[2 * h + 1][rt], hi, lo);
-        *reinterpret_cast<uint4*>(wm + (((rt * 4 + ks) * 2 + 0) * 64 + lane) * 8) = hi;
-        *reinterpret_cast<uint4*>(wm + (((rt * 4 + ks) * 2 + 1) * 64 + lane) * 8) = lo;
-      }
   }
 }
 
 namespace {
-// a chunk's operands, split by the step that consumes them: step A (the delta
-// products) and step B (the state products); bf16 hi / lo pairs [.][hl]
-struct ScanOpsA {
-  uint4 w[4][2];  // -W rows 16 w .., k step ks
-  f32x4 u;
-};
-struct ScanOpsB {
-  uint4 k[2][2][2];  // K~^T tiles 2 w + x, k step ks
-  float gl;
-};
-__device__ __forceinline__ void scan_load_a(ScanOpsA& o, const float* unit, int w, int cb,
-                                            int lane) {
-  const uint16_t* wm = reinterpret_cast<const uint16_t*>(unit + UO_W);
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-    for (int hl = 0; hl < 2; ++hl)
-      o.w[ks][hl] = *reinterpret_cast<const uint4*>(wm + (((w * 4 + ks) * 2 + hl) * 64 + lane) * 8);
-  o.u = *reinterpret_cast<const f32x4*>(unit + UO_U + ((cb * 4 + w) * 64 + lane) * 4);
-}
-__device__ __forceinline__ void scan_load_b(ScanOpsB& o, const float* unit, int w, int lane) {
-  const uint16_t* kt = reinterpret_cast<const uint16_t*>(unit + UO_K);
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int hl = 0; hl < 2; ++hl)
-        o.k[x][ks][hl] =
-            *reinterpret_cast<const uint4*>(kt + ((((2 * w + x) * 2 + ks) * 2 + hl) * 64 + lane) * 8);
-  o.gl = unit[UO_G];
-}
-// an accumulator tile (lane (r4, n) rows 16 d + 4 r4 + e, column n) split into
-// the phase-3 B operand order: k step d / 2, lane 16 (2 (d % 2) + r4 / 2) + n,
-// elements 4 (r4 % 2) .. +3 (ks: this tile's k step; blk: the block's base)
-__device__ __forceinline__ void store_split(uint16_t* blk, int ks, int half, const uint2& hi,
-                                            const uint2& lo, int lane) {
-  const int r4 = lane >> 4, n = lane & 15;
-  const int l2 = 16 * (2 * half + (r4 >> 1)) + n;
-  *reinterpret_cast<uint2*>(blk + ((ks * 2 + 0) * 64 + l2) * 8 + 4 * (r4 & 1)) = hi;
-  *reinterpret_cast<uint2*>(blk + ((ks * 2 + 1) * 64 + l2) * 8 + 4 * (r4 & 1)) = lo;
-}
 constexpr int SSW = DN_D + 8;  // LDS row (one state column) of S hi / lo, bf16
-constexpr int DSW = DC + 8;    // LDS row (one state column) of delta hi / lo, bf16
-// the scan's LDS: S and delta split, transposed: X[k][column c] at [c][k]
-struct ScanLds {
-  uint16_t sh[CBW * SSW], sl[CBW * SSW], dh[CBW * DSW], dl[CBW * DSW];
-};
+constexpr int DSW = DC + 8;    // LDS row (one state column) of R, delta, e delta hi / lo, bf16
 // accumulator tile rows k0 + 4 (l / 16) .. +3 of column l % 16, split, into LDS
-__device__ __forceinline__ void lds_put(uint16_t* h, uint16_t* l, int ld, int k0, const uint2& hi,
-                                        const uint2& lo, int lane) {
-  const int o = (lane & 15) * ld + k0 + 4 * (lane >> 4);
-  *reinterpret_cast<uint2*>(h + o) = hi;
-  *reinterpret_cast<uint2*>(l + o) = lo;
+// transposed (X[k][column] at [column][k], hi then lo)
+__device__ __forceinline__ void lds_put(uint16_t* x, int ld, int k0, const f32x4& v, int lane) {
+  uint2 hi, lo;
+  split4(v, hi, lo);
+  uint16_t* const p = x + (lane & 15) * ld + k0 + 4 * (lane >> 4);
+  *reinterpret_cast<uint2*>(p) = hi;
+  *reinterpret_cast<uint2*>(p + CBW * ld) = lo;
 }
-// one chunk: S_0 out for phase 3, delta = U - W S_0 (step A), delta out, then
-// S = gamma_C S_0 + K~^T delta (step B). s0 / dl: this chunk's S_0 and delta
-// blocks of this workgroup's column block (bf16 hi / lo, see S0_UNIT). B
-// operand of k step ks, lane l: X[32 ks + 8 (l / 16) + j][l % 16], one LDS read
-// each of hi and lo.
-__device__ __forceinline__ void scan_chunk(const ScanOpsA& oa, const ScanOpsB& ob, f32x4 (&St)[2],
-                                           ScanLds& sm, uint16_t* s0, uint16_t* dl, int w,
-                                           int lane) {
-  const int row4 = lane >> 4, col = lane & 15;
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {  // rows 16 (2 w + x) ..
-    uint2 hi, lo;
-    split4(St[x], hi, lo);
-    store_split(s0, w, x, hi, lo, lane);
-  }
-  f32x4 dacc = oa.u;
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    const int o = col * SSW + 32 * ks + 8 * row4;
-    dacc = mfma_x3(oa.w[ks][0], oa.w[ks][1], *reinterpret_cast<const uint4*>(&sm.sh[o]),
-                   *reinterpret_cast<const uint4*>(&sm.sl[o]), dacc);
-  }
-  {  // delta rows 16 w ..
-    uint2 hi, lo;
-    split4(dacc, hi, lo);
-    store_split(dl, w >> 1, w & 1, hi, lo, lane);
-    lds_put(sm.dh, sm.dl, DSW, 16 * w, hi, lo, lane);
-  }
-  __syncthreads();
-  f32x4 s0v = St[0] * ob.gl, s1v = St[1] * ob.gl;
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int o = col * DSW + 32 * ks + 8 * row4;
-    const uint4 bh = *reinterpret_cast<const uint4*>(&sm.dh[o]);
-    const uint4 bl = *reinterpret_cast<const uint4*>(&sm.dl[o]);
-    s0v = mfma_x3(ob.k[0][ks][0], ob.k[0][ks][1], bh, bl, s0v);
-    s1v = mfma_x3(ob.k[1][ks][0], ob.k[1][ks][1], bh, bl, s1v);
-  }
-  St[0] = s0v;
-  St[1] = s1v;
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    uint2 hi, lo;
-    split4(St[x], hi, lo);
-    lds_put(sm.sh, sm.sl, SSW, 16 * (2 * w + x), hi, lo, lane);
-  }
-  __syncthreads();
+// the B operand of k step ks from such a buffer: lane l = X[32 ks + 8 (l / 16) ..][l % 16]
+__device__ __forceinline__ void lds_get(const uint16_t* x, int ld, int ks, int lane, uint4& hi,
+                                        uint4& lo) {
+  const uint16_t* const p = x + (lane & 15) * ld + 32 * ks + 8 * (lane >> 4);
+  hi = lds16(p);
+  lo = lds16(p + CBW * ld);
 }
+// a load at a wave-uniform base and a 32-bit byte offset per lane
+template <typename T>
+__device__ __forceinline__ T ld_off(const void* base, uint32_t bytes) {
+  return *reinterpret_cast<const T*>(static_cast<const char*>(base) + bytes);
+}
+// the scan's LDS: K (two chunks) and S (two chunks) split, R, delta and e delta
+struct ScanLds {
+  uint16_t k[2][2 * DC * KW];   // [parity][hi, lo][token][dk]
+  uint16_t s[2][2 * CBW * SSW];
+  uint16_t r[2 * CBW * DSW], d[2 * CBW * DSW], e[2 * CBW * DSW];
+};
 }  // namespace
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void deltanet_scan_kernel(DeltaChunkArgs a) {
+// Phase 2. One workgroup of 8 waves per (16 state columns, value head, sequence);
+// chunk c uses the LDS buffers of parity c % 2. Per chunk three barriers:
+//   chain wave w (0 .. 3): X = K S_0 (rows 16 w), R = beta V - beta gamma X -> LDS | A |
+//     delta = T R (rows 16 w), delta and e delta -> LDS | B |
+//     S = gamma_C S_0 + K^T (e delta) (dk 32 w ..) -> LDS, other parity | C |
+//   wave 4 + w: K of the next chunk into LDS, other parity | A | Q S_0 (rows 16 w) | B |
+//     O = gamma (Q S_0) + M delta, stored | C |
+// Every operand from memory is loaded one or two chunks ahead into registers.
+// The chain's latency (three LDS round trips, three short MFMA chains) bounds a
+// chunk; O's products fill its gaps. K goes through LDS because its rows serve
+// both as they are (K S_0) and transposed (K^T delta).
+// Measured at T = 4096, B = 1, 16 / 32 heads (kernel trace): 128 us, 2.0 us a chunk
+// (1.1 us with every operand in cache and no O), after 49 us of phase 1 and before
+// 25 us of gated norm: 202 us. The three kernels before (-W and U precomputed, S_0
+// and delta passed on to an output kernel) took 86 + 145 + 94 = 325 us.
+template <bool CHAIN>
+__device__ __forceinline__ void scan_body(const DeltaChunkArgs& a, ScanLds& sm, int b, int hv,
+                                          int hk, int cb, int w, int lane) {
   const DeltaSeqArgs& q = a.s;
-  const int HB = q.Hv * q.B;
-  // the 8 column blocks of a head share an XCD (workgroup id mod 8) when HB % 8 == 0
-  const int head = blockIdx.x % HB, cb = blockIdx.x / HB;
-  const int hv = head % q.Hv, b = head / q.Hv;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int row4 = lane >> 4, col = lane & 15;
-  __shared__ __attribute__((aligned(16))) ScanLds sm;
-  const int dv0 = cb * CBW;
-  const int64_t sb = ((int64_t)b * q.Hv + hv) * DN_D * DN_D;
-  f32x4 St[2];  // state tiles d = 2w, 2w + 1: lane l reg e = S[16 d + 4 (l / 16) + e][l % 16]
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    const int d = 2 * w + x;
-    St[x] = *reinterpret_cast<const f32x4*>(q.s_in + sb + (int64_t)(dv0 + col) * DN_D + 16 * d +
-                                            4 * row4);
-    uint2 hi, lo;
-    split4(St[x], hi, lo);
-    lds_put(sm.sh, sm.sl, SSW, 16 * d, hi, lo, lane);
-  }
+  const int r4 = lane >> 4, col = lane & 15;
   const int NC = (q.T + DC - 1) / DC;
-  const float* units = dn_units(a, b, hv, NC);
-  // phase 3's inputs of this column block: chunk c at + c * unit + cb * block
-  uint16_t* s0b = reinterpret_cast<uint16_t*>(dn_s0(a, b, hv, NC) + cb * (S0_UNIT / 8));
-  uint16_t* dlb = reinterpret_cast<uint16_t*>(dn_dl(a, b, hv, NC) + cb * (DL_UNIT / 8));
-  // Two register sets, chunks in pairs, each set reloaded two chunks ahead right
-  // after its chunk; chunk indices past the end read the identity unit (an odd
-  // count pads with it; its S_0 and delta go to the spare slot NC). Branch-free,
-  // so the compiler's waits count exactly.
-  ScanOpsA ax, ay;
-  ScanOpsB bx, by;
-  scan_load_a(ax, units, w, cb, lane);
-  scan_load_b(bx, units, w, lane);
-  scan_load_a(ay, units + (int64_t)min(1, NC) * UNIT, w, cb, lane);
-  scan_load_b(by, units + (int64_t)min(1, NC) * UNIT, w, lane);
-  // every prologue load complete (s_waitcnt vmcnt(0)): the loop is then entered
-  // with no load in flight, and the compiler's count of the loads each wait in
-  // the loop must see is the one its own body implies (else it takes the
-  // prologue's order, where a register the loop reloads early was loaded last).
-  // NC >= 1 (the launch returns before T = 0): a do-while has no guard branch
-  // that the prologue's loads could be sunk past.
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(0x0f70);
-  __builtin_amdgcn_sched_barrier(0);
-  __syncthreads();
-  int c = 0;
-  do {
-    scan_chunk(ax, bx, St, sm, s0b + 2 * (int64_t)c * S0_UNIT, dlb + 2 * (int64_t)c * DL_UNIT, w,
-               lane);
-    const float* u2 = units + (int64_t)min(c + 2, NC) * UNIT;
-    __builtin_amdgcn_sched_barrier(0);  // the reloads issue here, between the chunks
-    scan_load_a(ax, u2, w, cb, lane);
-    scan_load_b(bx, u2, w, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    const int c1 = min(c + 1, NC);
-    scan_chunk(ay, by, St, sm, s0b + 2 * (int64_t)c1 * S0_UNIT, dlb + 2 * (int64_t)c1 * DL_UNIT, w,
-               lane);
-    const float* u3 = units + (int64_t)min(c + 3, NC) * UNIT;
-    __builtin_amdgcn_sched_barrier(0);
-    scan_load_a(ay, u3, w, cb, lane);
-    scan_load_b(by, u3, w, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    c += 2;
-  } while (c < NC);
+  const int dv0 = cb * CBW, i0 = 16 * w + 4 * r4;  // this lane's accumulator rows i0 .. i0 + 3
+  const bool lower = w < 2;                        // rows below token 32: k step 1 is zero
+  const float* const units = dn_unit(a, b, hv, NC, 0);
+  if constexpr (CHAIN) {
+    const float* const vp = q.v + ((int64_t)b * q.Hv + hv) * q.T * DN_D + dv0;
+    const int64_t sb = ((int64_t)b * q.Hv + hv) * DN_D * DN_D;
+    f32x4 St[2];  // state tiles d = 2w, 2w + 1: lane l reg e = S[16 d + 4 (l / 16) + e][l % 16]
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
-    *reinterpret_cast<f32x4*>(q.s_out + sb + (int64_t)(dv0 + col) * DN_D + 16 * (2 * w + x) +
-                              4 * row4) = St[x];
-}
-
-// Phase 3: one workgroup per (chunk, value head, sequence). First each wave w
-// forms rows 16 w .. 16 w + 15 of M and of gamma Q into LDS, split into bf16
-// hi and lo parts: lane l holds q row i = 16 w + l % 16 at columns 32 ks + 8
-// (l / 16) .. +7 (ks < 4), the B operand of P^T = K Q^T, whose result tiles
-// (tile jt: lane l reg r = P[i][16 jt + 4 (l / 16) + r]) are masked and
-// decayed into M. Then wave w forms output columns 32 w .. 32 w + 31 (the
-// scan's column blocks 2 w, 2 w + 1) of all 64 rows: its S_0 and delta
-// operands (the scan's split blocks) are loaded once the first phase is done,
-// and gamma Q and M come from LDS. Each product is hi hi + hi lo + lo hi on
-// v_mfma_f32_16x16x32_bf16 (A lane l = A[l % 16][8 (l / 16) + j], B lane l =
-// B[8 (l / 16) + j][l % 16], D lane l reg r = D[4 (l / 16) + r][l % 16]). The
-// output tile is staged through LDS, so that a thread then holds 32
-// contiguous columns of one row: O, or with NORM y = o rstd norm_w silu(z)
-// (the layer's gated norm, as gated_rms_norm_kernel) in bf16.
-constexpr int OQW = DN_D + 8;  // LDS row of gamma Q hi / lo (bf16; 16-byte aligned, banks skewed)
-constexpr int OMW = DC + 8;    // LDS row of M hi / lo (bf16)
-constexpr int OOW = DN_D + 4;  // LDS row of the output tile (floats)
-template <bool NORM>
-__global__ __launch_bounds__(256) void deltanet_out_kernel(DeltaChunkArgs a) {
-  const DeltaSeqArgs& q = a.s;
-  const int c = blockIdx.x, hv = blockIdx.y, b = blockIdx.z, t = threadIdx.x;
-  const int lane = t & 63, w = t >> 6, l16 = lane & 15, r4 = lane >> 4;
-  const int hk = hv / (q.Hv / q.Hk);
-  const int t0 = c * DC, n = min(DC, q.T - t0);
-  const int NC = (q.T + DC - 1) / DC;
-  __shared__ float Gs[DC];
-  __shared__ __attribute__((aligned(16))) uint16_t Qhl[2][DC * OQW];  // gamma Q [i][dk] hi, lo
-  uint16_t* const Qh = Qhl[0];
-  uint16_t* const Ql = Qhl[1];
-  __shared__ __attribute__((aligned(16))) uint16_t Mh[DC * OMW], Ml[DC * OMW];  // M [i][j]
-  if (t < 64) Gs[t] = chunk_cumsum(q, b, hv, t0, n, t);
-  const float* qp = q.q + (((int64_t)b * q.Hk + hk) * q.T + t0) * DN_D;
-  const float* kp = q.k + (((int64_t)b * q.Hk + hk) * q.T + t0) * DN_D;
-  {
-    const int i = 16 * w + l16;  // this lane's q row
-    f32x4 qv[8];                 // q[i][32 ks + 8 (l / 16) + 4 u .. +3] at qv[2 ks + u]
+    for (int x = 0; x < 2; ++x) {
+      St[x] = *reinterpret_cast<const f32x4*>(q.s_in + sb + (int64_t)(dv0 + col) * DN_D +
+                                              16 * (2 * w + x) + 4 * r4);
+      lds_put(sm.s[0], SSW, 16 * (2 * w + x), St[x], lane);
+    }
+    struct Ops {
+      uint4 t[2][2];
+      f32x4 v, be, bg, ek;
+      float gc;
+    } o0, o1;
+    auto load_rows = [&](Ops& o, int c) __attribute__((always_inline)) {
+      c = min(c, NC - 1);
+      const int n = min(DC, q.T - c * DC);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+      for (int r = 0; r < 4; ++r)
+        o.v[r] = ld_off<float>(vp + (int64_t)c * DC * DN_D, 4 * (min(i0 + r, n - 1) * DN_D + col));
+      const float* sc = units + (int64_t)c * UNIT + UO_SC;
+      o.be = ld_off<f32x4>(sc, 4 * i0);
+      o.bg = ld_off<f32x4>(sc + 64, 4 * i0);
+    };
+    auto load_t = [&](Ops& o, int c) __attribute__((always_inline)) {
+      c = min(c, NC - 1);
+      const uint16_t* tp = reinterpret_cast<const uint16_t*>(units + (int64_t)c * UNIT + UO_T) + w * 2048;
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-        qv[2 * ks + u] = *reinterpret_cast<const f32x4*>(qp + (int64_t)min(i, n - 1) * DN_D + 32 * ks +
-                                                         8 * r4 + 4 * u);
-    uint4 qh[4], ql[4];
+      for (int hl = 0; hl < 2; ++hl) o.t[0][hl] = ld_off<uint4>(tp + hl * 512, 16 * lane);
+      if (!lower) {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) split8(qv[2 * ks], qv[2 * ks + 1], qh[ks], ql[ks]);
-    // P^T tiles: D[j][i] = sum_dk K[j][dk] Q[i][dk], A lane l = K[16 jt + l % 16][dk]
-    f32x4 P[4];
-#pragma unroll
-    for (int jt = 0; jt < 4; ++jt) P[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      uint4 kh[4], kl[4];
-#pragma unroll
-      for (int jt = 0; jt < 4; ++jt) {
-        const float* kr = kp + (int64_t)min(16 * jt + l16, n - 1) * DN_D + 32 * ks + 8 * r4;
-        split8(*reinterpret_cast<const f32x4*>(kr), *reinterpret_cast<const f32x4*>(kr + 4), kh[jt],
-               kl[jt]);
+        for (int hl = 0; hl < 2; ++hl) o.t[1][hl] = ld_off<uint4>(tp + 1024 + hl * 512, 16 * lane);
       }
+      const float* sc = units + (int64_t)c * UNIT + UO_SC;
+      o.ek = ld_off<f32x4>(sc + 128, 4 * i0);
+      o.gc = sc[192 + DC - 1];
+    };
+    uint4 kx[4][2];  // K rows 16 w + l % 16 of the coming chunk, A operands of X
+    auto read_kx = [&](const uint16_t* k) __attribute__((always_inline)) {
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt) P[jt] = mfma_x3(kh[jt], kl[jt], qh[ks], ql[ks], P[jt]);
-    }
-    __syncthreads();  // Gs
-    // M = P D on j <= i < n, j < n (rows or keys past the chunk: 0); lane l reg r
-    // of tile jt is (i, j = 16 jt + 4 (l / 16) + r)
-    const float Gi = Gs[i];
+      for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-    for (int jt = 0; jt < 4; ++jt) {
-      f32x4 m;
+        for (int hl = 0; hl < 2; ++hl)
+          kx[ks][hl] = lds16(k + hl * DC * KW + (16 * w + col) * KW + 32 * ks + 8 * r4);
+    };
+    auto chunk = [&](Ops& o, int c, int p) __attribute__((always_inline)) {
+      const uint16_t* const kb = sm.k[p];
+      f32x4 xa = {0.f, 0.f, 0.f, 0.f}, xb = xa;
+      uint4 sh[4], sl[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int j = 16 * jt + 4 * r4 + r;
-        m[r] = (j <= i && i < n) ? P[jt][r] * expf(Gi - Gs[j]) : 0.f;
-      }
-      uint2 mh, ml;
-      split4(m, mh, ml);
-      *reinterpret_cast<uint2*>(&Mh[i * OMW + 16 * jt + 4 * r4]) = mh;
-      *reinterpret_cast<uint2*>(&Ml[i * OMW + 16 * jt + 4 * r4]) = ml;
-    }
-    const float gi = i < n ? expf(Gi) : 0.f;  // gamma_i (rows past the chunk: 0)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      uint4 gh, gl;
-      split8(qv[2 * ks] * gi, qv[2 * ks + 1] * gi, gh, gl);
-      *reinterpret_cast<uint4*>(&Qh[i * OQW + 32 * ks + 8 * r4]) = gh;
-      *reinterpret_cast<uint4*>(&Ql[i * OQW + 32 * ks + 8 * r4]) = gl;
-    }
-  }
-  // this wave's B operands, column blocks 2 w + x: S_0 (ks < 4) and delta (ks < 2)
-  const uint16_t* s0 = reinterpret_cast<const uint16_t*>(dn_s0(a, b, hv, NC) + (int64_t)c * S0_UNIT) +
-                       2 * (2 * w) * (S0_UNIT / 8);
-  const uint16_t* dl = reinterpret_cast<const uint16_t*>(dn_dl(a, b, hv, NC) + (int64_t)c * DL_UNIT) +
-                       2 * (2 * w) * (DL_UNIT / 8);
-  uint4 sb[2][4][2], db[2][2][2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-      for (int hl = 0; hl < 2; ++hl)
-        sb[x][ks][hl] = *reinterpret_cast<const uint4*>(s0 + 2 * x * (S0_UNIT / 8) + ((ks * 2 + hl) * 64 + lane) * 8);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int hl = 0; hl < 2; ++hl)
-        db[x][ks][hl] = *reinterpret_cast<const uint4*>(dl + 2 * x * (DL_UNIT / 8) + ((ks * 2 + hl) * 64 + lane) * 8);
-  }
-  __syncthreads();
-  // O = gamma Q S_0 + M delta: row tile rt, column block 2 w + x
-  f32x4 O[4][2];
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-    for (int x = 0; x < 2; ++x) O[rt][x] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    uint4 ah[4], al[4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      ah[rt] = *reinterpret_cast<const uint4*>(&Qh[(16 * rt + l16) * OQW + 32 * ks + 8 * r4]);
-      al[rt] = *reinterpret_cast<const uint4*>(&Ql[(16 * rt + l16) * OQW + 32 * ks + 8 * r4]);
-    }
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+      for (int ks = 0; ks < 4; ++ks) lds_get(sm.s[p], SSW, ks, lane, sh[ks], sl[ks]);
+      // K^T operands of the state product: lane l = K[32 ks + 8 (l / 16) + j][16 d + l % 16]
+      uint2 kt[2][2][2][2];  // [x][ks][hl][j / 4]
 #pragma unroll
       for (int x = 0; x < 2; ++x)
-        O[rt][x] = mfma_x3(ah[rt], al[rt], sb[x][ks][0], sb[x][ks][1], O[rt][x]);
-  }
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    uint4 ah[4], al[4];
+        for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      ah[rt] = *reinterpret_cast<const uint4*>(&Mh[(16 * rt + l16) * OMW + 32 * ks + 8 * r4]);
-      al[rt] = *reinterpret_cast<const uint4*>(&Ml[(16 * rt + l16) * OMW + 32 * ks + 8 * r4]);
-    }
+          for (int hl = 0; hl < 2; ++hl)
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+            for (int h = 0; h < 2; ++h)
+              kt[x][ks][hl][h] = lds_read_tr16(kb + hl * DC * KW +
+                                               (32 * ks + 8 * r4 + 4 * h + (col >> 2)) * KW +
+                                               16 * (2 * w + x) + 4 * (col & 3));
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
-        O[rt][x] = mfma_x3(ah[rt], al[rt], db[x][ks][0], db[x][ks][1], O[rt][x]);
-  }
-  // lane l reg r of O[rt][x] = O[16 rt + 4 (l / 16) + r][32 w + 16 x + l % 16]: the
-  // tile goes through LDS (the gamma Q and M rows, free once every wave is past
-  // its products) so that a thread then holds 32 contiguous columns of one row
-  __syncthreads();
-  float* Os = reinterpret_cast<float*>(&Qhl[0][0]);  // 2 x 17 KB >= 64 rows of OOW floats
-  static_assert(sizeof(Qhl) >= DC * OOW * sizeof(float), "output tile");
+      for (int ks = 0; ks < 2; ++ks) {
+        xa = mfma_x3(kx[ks][0], kx[ks][1], sh[ks], sl[ks], xa);
+        xb = mfma_x3(kx[2 + ks][0], kx[2 + ks][1], sh[2 + ks], sl[2 + ks], xb);
+      }
+      lds_put(sm.r, DSW, 16 * w, o.be * o.v - o.bg * (xa + xb), lane);
+      load_rows(o, c + 2);
+      __syncthreads();  // A
+      f32x4 d = {0.f, 0.f, 0.f, 0.f};
+      uint4 rh[2], rl[2];
 #pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
+      for (int ks = 0; ks < 2; ++ks) lds_get(sm.r, DSW, ks, lane, rh[ks], rl[ks]);
+      d = mfma_x3(o.t[0][0], o.t[0][1], rh[0], rl[0], d);
+      if (!lower) d = mfma_x3(o.t[1][0], o.t[1][1], rh[1], rl[1], d);
+      lds_put(sm.e, DSW, 16 * w, d * o.ek, lane);
+      lds_put(sm.d, DSW, 16 * w, d, lane);
+      const float gc = o.gc;
+      load_t(o, c + 2);
+      __syncthreads();  // B
+      uint4 eh[2], el[2];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+      for (int ks = 0; ks < 2; ++ks) lds_get(sm.e, DSW, ks, lane, eh[ks], el[ks]);
+      read_kx(sm.k[p ^ 1]);  // staged before A
+      St[0] = St[0] * gc;
+      St[1] = St[1] * gc;
 #pragma unroll
-      for (int x = 0; x < 2; ++x) Os[(16 * rt + 4 * r4 + r) * OOW + 32 * w + 16 * x + l16] = O[rt][x][r];
-  __syncthreads();
-  const int row = t >> 2, c0 = 32 * (t & 3);  // thread t: row t / 4, columns c0 .. c0 + 31
-  float o[32];
+      for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const f32x4 v = *reinterpret_cast<const f32x4*>(&Os[row * OOW + c0 + 4 * j]);
-    o[4 * j] = v[0]; o[4 * j + 1] = v[1]; o[4 * j + 2] = v[2]; o[4 * j + 3] = v[3];
-  }
-  const int64_t tok = t0 + row;
-  if constexpr (!NORM) {
-    if (row < n) {
-      float* op = q.o + (((int64_t)b * q.Hv + hv) * q.T + tok) * DN_D + c0;
+        for (int x = 0; x < 2; ++x)
+          St[x] = mfma_x3(make_uint4(kt[x][ks][0][0].x, kt[x][ks][0][0].y, kt[x][ks][0][1].x, kt[x][ks][0][1].y),
+                          make_uint4(kt[x][ks][1][0].x, kt[x][ks][1][0].y, kt[x][ks][1][1].x, kt[x][ks][1][1].y),
+                          eh[ks], el[ks], St[x]);
+      }
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        *reinterpret_cast<float4*>(op + 4 * j) = make_float4(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
-    }
+      for (int x = 0; x < 2; ++x) lds_put(sm.s[p ^ 1], SSW, 16 * (2 * w + x), St[x], lane);
+      __syncthreads();  // C
+    };
+    load_rows(o0, 0);
+    load_t(o0, 0);
+    load_rows(o1, 1);
+    load_t(o1, 1);
+    __syncthreads();
+    read_kx(sm.k[0]);
+    int c = 0;
+    do {
+      chunk(o0, c, 0);
+      if (c + 1 >= NC) break;
+      chunk(o1, c + 1, 1);
+      c += 2;
+    } while (c < NC);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+      *reinterpret_cast<f32x4*>(q.s_out + sb + (int64_t)(dv0 + col) * DN_D + 16 * (2 * w + x) +
+                                4 * r4) = St[x];
   } else {
-    const GatedNormArgs& g = a.g;
-    float ss = 0.f;
+    const uint16_t* const kq = dn_kq(a, b, hk, NC, 0);
+    float* const op = q.o + ((int64_t)b * q.Hv + hv) * q.T * DN_D + dv0 + col;
+    struct OpsM {
+      uint4 m[2][2];
+      f32x4 g;
+    } o0, o1;
+    f32x4 k0[8], k1[8];  // 8 bf16 each
+    uint4 q0[4][2], q1[4][2];
+    // K: 16-byte pieces t + 256 u of the chunk's [hl][token][dk]
+    auto load_k = [&](f32x4 (&k)[8], int c) __attribute__((always_inline)) {
+      const uint16_t* p = kq + (int64_t)min(c, NC - 1) * (2 * KQ_UNIT);
 #pragma unroll
-    for (int j = 0; j < 32; ++j) ss += o[j] * o[j];
-    ss += __shfl_xor(ss, 1);  // the row's four threads
-    ss += __shfl_xor(ss, 2);
-    const float rstd = 1.0f / sqrtf(ss / (float)DN_D + g.eps);
-    if (row < n) {
-      const uint16_t* z = g.z + (int64_t)b * g.z_sb + tok * g.z_st + hv * DN_D + c0;
-      uint16_t* y = g.y + (int64_t)b * g.y_sb + tok * g.y_st + hv * DN_D + c0;
-      if (((reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(y) |
-            reinterpret_cast<uintptr_t>(g.norm_w)) & 15u) == 0) {
+      for (int u = 0; u < 8; ++u) k[u] = ld_off<f32x4>(p + 2048 * u, 16 * (64 * w + lane));
+    };
+    auto stage_k = [&](const f32x4 (&v)[8], uint16_t* k) __attribute__((always_inline)) {
+      uint16_t* const p = k + (4 * w + (lane >> 4)) * KW + 8 * (lane & 15);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float zf[8], wf[8], yv[8];
-          unpack8(*reinterpret_cast<const uint4*>(z + 8 * j), zf);
-          unpack8(*reinterpret_cast<const uint4*>(g.norm_w + c0 + 8 * j), wf);
+      for (int u = 0; u < 8; ++u) *reinterpret_cast<f32x4*>(p + 16 * u * KW) = v[u];
+    };
+    auto load_q = [&](uint4 (&q)[4][2], int c) __attribute__((always_inline)) {
+      const uint16_t* p = kq + (int64_t)min(c, NC - 1) * (2 * KQ_UNIT) + 2 * KQ_Q + w * 4096;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) yv[e] = o[8 * j + e] * rstd * wf[e] * accurate_silu(zf[e]);
-          *reinterpret_cast<uint4*>(y + 8 * j) = pack8(yv);
-        }
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int hl = 0; hl < 2; ++hl) q[ks][hl] = ld_off<uint4>(p + (ks * 2 + hl) * 512, 16 * lane);
+    };
+    auto load_m = [&](OpsM& o, int c) __attribute__((always_inline)) {
+      c = min(c, NC - 1);
+      const float* u = units + (int64_t)c * UNIT;
+      const uint16_t* mp = reinterpret_cast<const uint16_t*>(u + UO_M) + w * 2048;
+#pragma unroll
+      for (int hl = 0; hl < 2; ++hl) o.m[0][hl] = ld_off<uint4>(mp + hl * 512, 16 * lane);
+      if (!lower) {
+#pragma unroll
+        for (int hl = 0; hl < 2; ++hl) o.m[1][hl] = ld_off<uint4>(mp + 1024 + hl * 512, 16 * lane);
+      }
+      o.g = ld_off<f32x4>(u + UO_SC + 192, 4 * i0);
+    };
+    // qc, o: chunk c's operands; kn: K of chunk c + 1
+    auto chunk = [&](f32x4 (&kn)[8], uint4 (&qc)[4][2], OpsM& o, int c, int p) __attribute__((always_inline)) {
+      f32x4 oa = {0.f, 0.f, 0.f, 0.f}, ob = oa;
+      stage_k(kn, sm.k[p ^ 1]);
+      load_k(kn, c + 3);
+      __syncthreads();  // A
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        uint4 sh, sl;
+        lds_get(sm.s[p], SSW, ks, lane, sh, sl);
+        oa = mfma_x3(qc[ks][0], qc[ks][1], sh, sl, oa);
+        lds_get(sm.s[p], SSW, 2 + ks, lane, sh, sl);
+        ob = mfma_x3(qc[2 + ks][0], qc[2 + ks][1], sh, sl, ob);
+      }
+      load_q(qc, c + 2);
+      oa = (oa + ob) * o.g;
+      __syncthreads();  // B
+      uint4 dh, dl;
+      lds_get(sm.d, DSW, 0, lane, dh, dl);
+      oa = mfma_x3(o.m[0][0], o.m[0][1], dh, dl, oa);
+      if (!lower) {
+        lds_get(sm.d, DSW, 1, lane, dh, dl);
+        oa = mfma_x3(o.m[1][0], o.m[1][1], dh, dl, oa);
+      }
+      float* const oc = op + ((int64_t)c * DC + i0) * DN_D;
+      const int n = q.T - c * DC;
+      if (n >= DC) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) oc[r * DN_D] = oa[r];
       } else {
 #pragma unroll
-        for (int j = 0; j < 32; ++j)
-          y[j] = f2bf(o[j] * rstd * bf2f(g.norm_w[c0 + j]) * accurate_silu(bf2f(z[j])));
+        for (int r = 0; r < 4; ++r)
+          if (i0 + r < n) oc[r * DN_D] = oa[r];
       }
-    }
+      load_m(o, c + 2);
+      __syncthreads();  // C
+    };
+    load_k(k0, 0);
+    stage_k(k0, sm.k[0]);
+    load_k(k0, 1);
+    load_k(k1, 2);
+    load_q(q0, 0);
+    load_q(q1, 1);
+    load_m(o0, 0);
+    load_m(o1, 1);
+    __syncthreads();
+    int c = 0;
+    do {
+      chunk(k0, q0, o0, c, 0);
+      if (c + 1 >= NC) break;
+      chunk(k1, q1, o1, c + 1, 1);
+      c += 2;
+    } while (c < NC);
+  }
+}
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void deltanet_scan_kernel(DeltaChunkArgs a) {
+  const DeltaSeqArgs& q = a.s;
+  // a qk head's column blocks (of its R value heads) share an XCD (workgroup id
+  // mod 8) when the (qk head, sequence) groups divide over the 8 XCDs
+  const int R = q.Hv / q.Hk, R8 = R * (DN_D / CBW), id = blockIdx.x;
+  const bool xcd = (q.Hk * q.B) % 8 == 0;
+  const int grp = xcd ? (id & 7) + 8 * ((id >> 3) / R8) : id / R8;
+  const int mem = xcd ? (id >> 3) % R8 : id % R8;
+  const int hk = grp % q.Hk, b = grp / q.Hk;
+  const int hv = hk * R + mem / (DN_D / CBW), cb = mem % (DN_D / CBW);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ __attribute__((aligned(16))) ScanLds sm;
+  if (w < 4) {
+    scan_body<true>(a, sm, b, hv, hk, cb, w, lane);
+  } else {
+    scan_body<false>(a, sm, b, hv, hk, cb, w - 4, lane);
   }
 }
 
@@ -1208,8 +1055,10 @@ __global__ __launch_bounds__(256) void gated_rms_norm_kernel(GatedNormArgs a) {
   const float w0 = bf2f(a.norm_w[2 * lane]), w1 = bf2f(a.norm_w[2 * lane + 1]);
   const float y0 = o.x * rstd * w0 * accurate_silu(bf2f(z[0]));
   const float y1 = o.y * rstd * w1 * accurate_silu(bf2f(z[1]));
-  *reinterpret_cast<uint32_t*>(a.y + (int64_t)b * a.y_sb + (int64_t)t * a.y_st + hv * DN_D +
-                               2 * lane) = pack2(y0, y1);
+  uint16_t* y = a.y + (int64_t)b * a.y_sb + (int64_t)t * a.y_st + hv * DN_D + 2 * lane;
+  const uint32_t yp = pack2(y0, y1);
+  y[0] = (uint16_t)yp;  // y may be 2-byte aligned
+  y[1] = (uint16_t)(yp >> 16);
 }
 
 // The same, vectorised for aligned z and y (16-byte aligned, strides of whole
@@ -1539,26 +1388,38 @@ hipError_t launch_deltanet_sequence(const DeltaSeqArgs& a, hipStream_t st) {
 }
 
 size_t deltanet_chunk_workspace_bytes(int T, int Hv, int B) {
-  const int NC = (T + DC - 1) / DC;  // each per (b, hv): the units (+ the identity), S_0, delta
-  return (size_t)((dn_units_floats(NC) + dn_s0_floats(NC) + dn_dl_floats(NC)) * Hv * B) *
-         sizeof(float);
+  // per (b, hv): the units, the K and Q units (Hk <= Hv) and the fused form's O
+  const size_t NC = (T + DC - 1) / DC;
+  return (NC * (UNIT + KQ_UNIT) + (size_t)T * DN_D) * Hv * B * sizeof(float);
 }
 
-hipError_t launch_deltanet_sequence_chunked(const DeltaChunkArgs& a, hipStream_t st) {
+// Up to SEQ_T tokens the sequential kernel is the faster form: it takes 2 us + 0.6
+// us a token whatever the batch, the two chunked launches 24 us (B = 1, Hv = 32)
+// to 39 us (B = 4) for a chunk of any length. Measured at B = 1 / 4, T = 32: 21.3 /
+// 23.7 us sequential, 23.9 / 38.5 chunked; T = 40: 26.0 / 30.0 and 24.1 / 38.9.
+constexpr int SEQ_T = 36;
+hipError_t launch_deltanet_sequence_chunked(const DeltaChunkArgs& args, hipStream_t st) {
+  DeltaChunkArgs a = args;
   const DeltaSeqArgs& q = a.s;
   if (q.B == 0 || q.T == 0) return launch_deltanet_sequence(q, st);  // state copy / no-op
   const int NC = (q.T + DC - 1) / DC;
-  hipLaunchKernelGGL(deltanet_chunk_kernel, dim3(NC, q.Hv, q.B), dim3(256), 0, st, a);
+  if (a.g.y) {
+    a.s.o = a.ws + (int64_t)q.B * NC * ((int64_t)q.Hv * UNIT + (int64_t)q.Hk * KQ_UNIT);
+    a.g.o = a.s.o;
+  }
+  const int R = q.Hv / q.Hk;  // value heads per qk head, two a workgroup
+  if (q.T <= SEQ_T) {
+    hipError_t e = launch_deltanet_sequence(a.s, st);
+    if (e != hipSuccess || !a.g.y) return e;
+    return launch_gated_rms_norm(a.g, st);
+  }
+  hipLaunchKernelGGL(deltanet_chunk_kernel, dim3(NC, q.Hk * ((R + 1) / 2), q.B), dim3(256), 0, st, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(deltanet_scan_kernel, dim3(q.Hv * q.B * (DN_D / CBW)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(deltanet_scan_kernel, dim3(q.Hv * q.B * (DN_D / CBW)), dim3(512), 0, st, a);
   e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (a.g.y)
-    hipLaunchKernelGGL(deltanet_out_kernel<true>, dim3(NC, q.Hv, q.B), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL(deltanet_out_kernel<false>, dim3(NC, q.Hv, q.B), dim3(256), 0, st, a);
-  return hipGetLastError();
+  if (e != hipSuccess || !a.g.y) return e;
+  return launch_gated_rms_norm(a.g, st);
 }
 
 namespace {

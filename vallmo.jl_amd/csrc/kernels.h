@@ -459,8 +459,8 @@ int linear_dn_decode_run(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ld
 struct DeltaChunkArgs {
   DeltaSeqArgs s;
   float* ws;
-  // g.y set: the gated RMSNorm with z (qwen35.jl:360-364) is fused into the
-  // output phase, which writes y (bf16) instead of s.o; g.o is unused
+  // g.y set: the gated RMSNorm with z (qwen35.jl:360-364) follows, O in the
+  // workspace; s.o and g.o are unused
   GatedNormArgs g;
 };
 size_t deltanet_chunk_workspace_bytes(int T, int Hv, int B);

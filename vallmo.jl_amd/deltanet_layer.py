@@ -172,8 +172,7 @@ def forward(l: DeltaNetLayer, c: DeltaNetConfig, xn, T: int, B: int, *, eps: flo
                             Hk=c.Hk, Hv=c.Hv, Sp=l.conv_state,
                             S=l.conv_state if offset > 0 else None)
     y = torch.empty((B, T, c.Hv, c.Dv), dtype=torch.bfloat16, device=xn.device)
-    # the recurrence in place on S with the gated norm fused into its output
-    # kernel (:357-364: O never reaches memory)
+    # the recurrence in place on S and its gated norm (:357-364)
     ops.deltanet_sequence_chunked_gated_norm_({"Y": y, "Sp": l.S}, z.unflatten(-1, (c.Hv, c.Dv)),
                                               l.gnorm_w, p["Q"], p["K"], p["V"], p["Beta"],
                                               p["Gate"], l.S, eps=eps)

@@ -725,15 +725,15 @@ def deltanet_sequence_(outs, Q, K, V, Beta, Gate, S):
 
 
 def deltanet_sequence_workspace_bytes(T: int, Hv: int, B: int) -> int:
-    """Workspace of deltanet_sequence_chunked_ (about 197 KB per 64-token chunk per
-    value head and sequence: the scan's operands, each chunk's start state and
-    its delta)."""
+    """Workspace of deltanet_sequence_chunked_ (about 132 KB per 64-token chunk per
+    value head and sequence: the scan's operands and, for the form with the gated
+    norm, O)."""
     return int(_lib.load().vm_deltanet_sequence_workspace_bytes(T, Hv, B))
 
 
 def deltanet_sequence_chunked_(outs, Q, K, V, Beta, Gate, S, *, workspace=None):
-    """deltanet_sequence! computed per 64-token chunk (a triangular solve and fp32
-    MFMA products, the chunks' state carried by one scan): the same operator and
+    """deltanet_sequence! computed per 64-token chunk (a triangular solve and
+    split-precision MFMA products, the chunks' state carried by one scan): the same operator and
     arguments as deltanet_sequence_ (deltanet_recurrent.jl:174-198), results
     equal to fp32 rounding. workspace: a uint8 GPU tensor of at least
     deltanet_sequence_workspace_bytes(T, Hv, B), 256-byte aligned (allocated
@@ -759,9 +759,8 @@ def deltanet_sequence(Q, K, V, Beta, Gate, S, *, Sp=None) -> dict:
 def deltanet_sequence_chunked_gated_norm_(outs, Z, NormWeight, Q, K, V, Beta, Gate, S, *, eps,
                                           workspace=None):
     """forward(::DeltaNetLayer)'s recurrence and gated norm in one call
-    (src/llm/qwen35.jl:357-364): deltanet_sequence! in its chunked form with
-    y = O rstd NormWeight silu(Z) applied in the output kernel, so O never
-    reaches memory. outs "Y" :: (Dv, Hv, T, B) bf16 (torch (B, T, Hv, Dv), token
+    (src/llm/qwen35.jl:357-364): deltanet_sequence! in its chunked form (O, fp32,
+    in the workspace), then y = O rstd NormWeight silu(Z). outs "Y" :: (Dv, Hv, T, B) bf16 (torch (B, T, Hv, Dv), token
     and sequence dims may be strided, heads contiguous), "Sp" the state out
     (may be S); Z like Y; Q, K, V, Beta, Gate, S as deltanet_sequence_chunked_."""
     Y, Sp = _out(outs, "Y"), _out(outs, "Sp")
