@@ -194,6 +194,31 @@ def test_linear_narrow_misaligned_view(vm, orc):
     assert mx <= TOL_MAX and mn <= TOL_MEAN
 
 
+@pytest.mark.parametrize("M,N,K", [(2560, 1, 64), (2564, 8, 320), (2560, 9, 4096), (4604, 16, 192),
+                                   (10240, 17, 2560), (12352, 32, 2560), (24576, 5, 448)])
+def test_linear_rows(vm, orc, M, N, K):
+    """The kernel that cuts the rows over the CUs (K whole): 1 to 12 row pieces a
+    workgroup, a last workgroup that is not full, the batch at its 8-column
+    edges, runs of no, one and many 64-k groups per wave; y a view at 8-byte
+    alignment whose neighbours stay, a second call bitwise equal, every element
+    within the narrow product's bar."""
+    banner(f"linear rows M={M} N={N} K={K}")
+    x = normal_bf16((N, K), 760 + N + K)
+    W = normal_bf16((M, K), 761 + M, scale=K ** -0.5)
+    xd, Wd = to_dev(x), to_dev(W)
+    buf = torch.full((N, M + 24), 3.0, dtype=torch.bfloat16, device="cuda")
+    y = buf[:, 16:16 + M]
+    vm.linear_({"y": y}, xd, Wd)
+    y2 = vm.linear(xd, Wd)["y"]
+    torch.cuda.synchronize()
+    ref = orc.linear(x, W).astype(np.float64)
+    over = float((np.abs(dev_f32(y) - ref) / _narrow_bar(x, W, ref)).max())
+    print(f"worst |err|/bar {over:.3f}")
+    assert over <= 1.0
+    assert torch.equal(y.contiguous().view(torch.int16), y2.view(torch.int16))
+    assert bool((buf[:, :16] == 3.0).all()) and bool((buf[:, 16 + M:] == 3.0).all())
+
+
 def _silu_mul_bar(orc, x, W, I):
     """The oracle's mid (orc.linear's fp32 gate-up rounded to bf16, as the
     reference stores gu, then orc.silu_mul, rounded) and a per-element bar:
@@ -218,7 +243,8 @@ def _silu_mul_bar(orc, x, W, I):
 
 
 @pytest.mark.parametrize("I,N,K", [(9216, 32, 2560), (9216, 1, 2560), (1000, 20, 640),
-                                   (1024, 7, 512), (512, 40, 256)])
+                                   (1024, 7, 512), (512, 40, 256), (12288, 9, 192),
+                                   (12296, 3, 256)])
 def test_linear_silu_mul(vm, orc, I, N, K):
     """linear! + silu .* mul in one call (the MLP's first half, qwen35.jl:234-243):
     at N <= 32 the stream-K GEMV's fp32 partials summed by the silu kernel (I =

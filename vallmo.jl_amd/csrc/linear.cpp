@@ -265,6 +265,45 @@ bool gemv_shape(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy) {
   const bool narrow = N <= 16 || (N <= 32 && M <= 4096);
   return narrow && K % 64 == 0 && M % 4 == 0 && ldw % 8 == 0 && ldx % 8 == 0 && ldy % 4 == 0;
 }
+// Of these, and of the wide ones at N = 17 .. 32, the problems below run with K
+// whole, their rows cut over the CUs (launch_gemv_rows), 0 for the others: no
+// partials, no reduce launch, and less batch traffic than the split kernel.
+// Measured as above, at N = 1 / 8 / 32, split kernel or GEMM library against it:
+// 18432 x 2560 25.2 / 26.2 / 23.3 -> 18.5 / 18.7 / 20.5 us; 10240 x 2560 13.5 /
+// 15.4 / 19.0 -> 11.2 / 12.3 / 14.5; 4608 x 2560 (rows that fill 192 of 256 CUs)
+// 9.4 / 10.2 / 12.0 -> 7.1 / 7.7 / 10.5; 2560 x 4096 10.2 / 11.0 / 11.4 -> 7.9 /
+// 8.1 / 10.1. Deep products of few rows stay split: 2560 x 9216 13.8 / 14.1 /
+// 15.3 against 15.8 / 15.8 / 19.4, 4096 x 9216 at N = 32 19.0 against 23.5; and so
+// do few rows, where the batch tile outweighs the weights (2048 x 2560 at N = 32
+// 7.5 against 7.2).
+int rows_shape(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy) {
+  if (N < 1 || N > 32 || M < 2560 || K <= 0 || K % 64 != 0 || M % 4 != 0 || ldw % 8 != 0 ||
+      ldx % 8 != 0 || ldy % 4 != 0)
+    return 0;
+  const int rw = gemv_rows_plan(M);
+  return K <= 4096 || rw >= 40 ? rw : 0;
+}
+int run_gemv_rows(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const uint16_t* w,
+                  int64_t ldw, int M, int N, int K, int rw, bool silu, hipStream_t st,
+                  const char* what, char* err, size_t errn) {
+  GemvRowsArgs r{};
+  r.w = w;
+  r.w_st = ldw;
+  r.x = x;
+  r.x_st = ldx;
+  r.y = y;
+  r.y_st = ldy;
+  r.M = M;
+  r.N = N;
+  r.K = K;
+  r.rw = rw;
+  const hipError_t e = launch_gemv_rows(r, silu, st);
+  if (e != hipSuccess) {
+    snprintf(err, errn, "%s: %s", what, hipGetErrorString(e));
+    return (int)e;
+  }
+  return VM_OK;
+}
 bool gemv_aligned(const void* y, const void* x, const void* w) {
   return ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0) && ((uintptr_t)y % 8 == 0);
 }
@@ -386,6 +425,8 @@ int linear_run(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const u
                "(vm_linear_workspace_bytes)", workspace_bytes, need);
       return VM_E_SCRATCH;
     }
+    if (const int rw = rows_shape(M, N, K, ldw, ldx, ldy))
+      return run_gemv_rows(y, ldy, x, ldx, w, ldw, M, N, K, rw, false, st, "linear", err, errn);
     GemvArgs a{};
     a.w = w;
     a.w_st = ldw;
@@ -415,6 +456,8 @@ int linear_run(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const u
              workspace_bytes, p->workspace);
     return VM_E_SCRATCH;
   }
+  if (const int rw = rows_shape(M, N, K, ldw, ldx, ldy))
+    return run_gemv_rows(y, ldy, x, ldx, w, ldw, M, N, K, rw, false, st, "linear", err, errn);
   hipblasLtHandle_t h;
   {
     int dev = 0;
@@ -482,7 +525,10 @@ int linear_add_norm_run(uint16_t* yn, int64_t yn_st, uint16_t* x, int64_t x_st, 
   na.offset = offset;
   na.eps = eps;
   uint16_t* h = static_cast<uint16_t*>(workspace);  // the bf16 y when one is formed
-  if (gemv_shape(M, N, K, ldw, lda, M) && gemv_aligned(h, a, w)) {
+  // (a problem of rows_shape takes linear_run's kernel, so that the pair stays bit
+  // for bit the two calls)
+  if (gemv_shape(M, N, K, ldw, lda, M) && gemv_aligned(h, a, w) &&
+      !rows_shape(M, N, K, ldw, lda, M)) {
     GemvArgs g{};
     g.w = w;
     g.w_st = ldw;
@@ -512,7 +558,7 @@ int linear_add_norm_run(uint16_t* yn, int64_t yn_st, uint16_t* x, int64_t x_st, 
     }
     return VM_OK;
   }
-  // the GEMM library's path: y into the workspace after the plan's own space
+  // linear!: y into the workspace after the plan's own space
   size_t lin = 0;
   rc = linear_workspace(M, N, K, ldw, lda, M, &lin, err, errn);
   if (rc != VM_OK) return rc;
@@ -569,7 +615,15 @@ int linear_silu_mul_run(uint16_t* mid, int64_t mid_st, const uint16_t* x, int64_
              "(vm_linear_silu_mul_workspace_bytes)", workspace_bytes, need);
     return VM_E_SCRATCH;
   }
-  if (sk_shape(M, N, K, ldw, ldx) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0) {
+  const bool decode = sk_shape(M, N, K, ldw, ldx) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
+  const int rw = decode ? gemv_rows_plan(M) : 0;
+  if (rw > 0) {
+    // one launch (gate-up 18432 x 2560 and the silu
+    // at N = 8: 18.4 us against 19.0 + 4.1 us for the stream-K GEMV and its consumer)
+    return run_gemv_rows(mid, mid_st, x, ldx, w, ldw, I, N, K, rw, true, st, "linear_silu_mul", err,
+                         errn);
+  }
+  if (decode) {
     GemvSkArgs g{};
     g.w = w;
     g.w_st = ldw;

@@ -771,6 +771,190 @@ __global__ __launch_bounds__(RT) void silu_mul_sk_kernel(SiluMulSkArgs a) {
 
 }  // namespace
 
+// ---- y = W^T x, or mid = silu(gate) .* up, for a decode batch (N <= 32 columns)
+// with the rows cut over the CUs and K whole: workgroup b owns rows [b RW, (b +
+// 1) RW) of y, or RW / 2 gate rows and the same up rows, so nothing passes through
+// memory between launches: no partials, no reduce or silu launch (4 us each, a
+// tenth of an MLP at decode, for kernels that move next to nothing). HBM-bound:
+// each weight byte is read once, 8 rows x 128 bytes per 1-KB direct load, by one
+// of four waves that split K in contiguous runs and add their sums through LDS
+// in wave order (bitwise repeatable). Where it is used, and its times against
+// the other kernels: rows_shape and linear_silu_mul_run in linear.cpp.
+constexpr int GR_RING = 78 * 1024;  // bf16 of the four waves' rings (156 KB)
+constexpr int GR_MAX = 12;         // row pieces (8 rows) per workgroup, at most
+
+__device__ __forceinline__ void gr_read(lm_u32x4& o, uint32_t addr) {
+  asm volatile("ds_read_b128 %0, %1" : "=v"(o) : "v"(addr));
+}
+
+// wait until at most `left` groups of PER loads, issued after the one about to be
+// multiplied, are still out (left <= NS - 1 <= 3)
+template <int PER, int NS>
+__device__ __forceinline__ void gr_wait(int left) {
+  if (left >= NS - 1) wait_vmcnt<PER * (NS - 1)>();
+  else if (NS > 3 && left == 2) wait_vmcnt<PER * 2>();
+  else if (NS > 2 && left == 1) wait_vmcnt<PER>();
+  else wait_vmcnt<0>();
+}
+
+// NR: 8-row pieces per workgroup. The batch comes in nx = 1, 2 or 4 pieces of 8
+// columns, as many as exist: batch column j reads column j % (8 nx), columns from
+// N on are computed and not used
+template <int NR, bool SILU>
+__device__ __forceinline__ void gemv_rows(const GemvRowsArgs& a) {
+  constexpr int T = (NR + 3) / 4;     // 32-row MFMA tiles
+  constexpr int SL = (NR + 4) * 512;  // bf16 per slot: NR row pieces, the batch tile
+  constexpr int NS = GR_RING / 4 / SL < 4 ? GR_RING / 4 / SL : 4;
+  static_assert(NS >= 2 && (NR + 4) * (NS - 1) < 64, "ring");
+  static_assert(4 * T * 16 * 64 * 4 <= GR_RING * 2, "reduction space");
+  __shared__ __attribute__((aligned(16))) uint16_t ring_all[GR_RING];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, j = lane & 31, h = lane >> 5;
+  const int cl = lane >> 3, p = lane & 7, chunk = 8 * (p ^ cl);
+  uint16_t* const ring = ring_all + wv * (NS * SL);
+  // local row r of the workgroup: SILU: gate rows r < RW / 2, then the up rows
+  const int hr = a.rw / 2;
+  auto row_of = [&](int r) __attribute__((always_inline)) {
+    if constexpr (SILU) {
+      const int i = min((int)blockIdx.x * hr + (r < hr ? r : r - hr), a.M - 1);
+      return r < hr ? i : a.M + i;
+    } else {
+      return min((int)blockIdx.x * a.rw + r, a.M - 1);
+    }
+  };
+  const uint16_t* wp[NR];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) wp[i] = a.w + (int64_t)row_of(min(8 * i + cl, a.rw - 1)) * a.w_st + chunk;
+  const int nx = a.N <= 8 ? 1 : a.N <= 16 ? 2 : 4;
+  const uint16_t* xp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xp[i] = a.x + (int64_t)min(8 * i + cl, a.N - 1) * a.x_st + chunk;
+  const int G = a.K / 64, per = (G + 3) / 4;
+  const int g0 = min(wv * per, G), n = min(g0 + per, G) - g0;
+  auto issue = [&](int g, uint16_t* slot) __attribute__((always_inline)) {
+    const int k = 64 * (g0 + g);
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      __builtin_amdgcn_global_load_lds(wp[i] + k, (__attribute__((address_space(3))) void*)(slot + 512 * i),
+                                       16, 0, 2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // the batch stays in L2: default cache policy
+      if (i < nx)
+        __builtin_amdgcn_global_load_lds(
+            xp[i] + k, (__attribute__((address_space(3))) void*)(slot + 512 * (NR + i)), 16, 0, 0);
+  };
+  f32x16 acc[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+#pragma unroll
+  for (int g = 0; g < NS; ++g)
+    if (g < n) issue(g, ring + g * SL);
+  int s = 0;
+  for (int g = 0; g < n; ++g) {
+    uint16_t* const slot = ring + s * SL;
+    const int left = n - 1 - g;  // groups issued after this one, at most NS - 1 of them out
+    if (nx == 1) gr_wait<NR + 1, NS>(left);
+    else if (nx == 2) gr_wait<NR + 2, NS>(left);
+    else gr_wait<NR + 4, NS>(left);
+    const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)slot;
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      // operands from asm (a compiler-visible read would drain every load in
+      // flight); tile rows past the pieces repeat the last one, and are unused
+      const uint32_t q = 8 * ((2 * st + h) ^ (j & 7));
+      lm_u32x4 o[T + 1];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const int r = min(32 * t + j, 8 * NR - 8 + (j & 7));
+        gr_read(o[t], base + 2u * (64 * r + q));
+      }
+      gr_read(o[T], base + 2u * (512 * NR + 64 * (j & (8 * nx - 1)) + q));
+      lm_take<0, T + 1>(o);
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+        acc[t] = mfma32(__builtin_bit_cast(uint4, o[t]), __builtin_bit_cast(uint4, o[T]), acc[t]);
+    }
+    if (g + NS < n) issue(g + NS, slot);  // every read of the slot is in
+    s = s + 1 == NS ? 0 : s + 1;
+  }
+  // the four waves' sums: wave w's tile t, register r, lane l at [w][t][r][l]
+  float* const red = reinterpret_cast<float*>(ring_all);
+  __syncthreads();  // every wave is done with its ring
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[((wv * T + t) * 16 + r) * 64 + lane] = acc[t][r];
+  __syncthreads();
+  // local rows r .. r + 3 (r % 4 == 0) of batch column c
+  auto sum4 = [&](int r, int c, float (&v)[4]) __attribute__((always_inline)) {
+    const float* src = red + ((r >> 5) * 16 + 4 * ((r >> 3) & 3)) * 64 + 32 * ((r >> 2) & 1) + c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float x = src[e * 64];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) x += src[(w * T * 16 + e) * 64];
+      v[e] = x;
+    }
+  };
+  const int rows = SILU ? hr : a.rw;
+  for (int i = threadIdx.x; i < rows / 4 * 32; i += 256) {
+    const int r = 4 * (i >> 5), c = i & 31, row = (int)blockIdx.x * rows + r;
+    if (c >= a.N || row >= a.M) continue;
+    float v[4];
+    sum4(r, c, v);
+    if constexpr (SILU) {
+      // gate and up rounded to bf16 first, as the reference stores them in gu
+      float u[4], m[4];
+      sum4(hr + r, c, u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float gf = bf2f(f2bf(v[e])), uf = bf2f(f2bf(u[e]));
+        m[e] = gf / (1.0f + __expf(-gf)) * uf;
+      }
+      *reinterpret_cast<uint2*>(a.y + (int64_t)c * a.y_st + row) =
+          make_uint2(pack2(m[0], m[1]), pack2(m[2], m[3]));
+    } else {
+      *reinterpret_cast<uint2*>(a.y + (int64_t)c * a.y_st + row) =
+          make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+    }
+  }
+}
+
+template <int NR, bool SILU>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void gemv_rows_kernel(GemvRowsArgs a) {
+  gemv_rows<NR, SILU>(a);
+}
+
+template <bool SILU>
+static void launch_gemv_rows_t(const GemvRowsArgs& a, int wgs, hipStream_t st) {
+#define VM_ROWS(nr) \
+  case nr: hipLaunchKernelGGL((gemv_rows_kernel<nr, SILU>), dim3(wgs), dim3(256), 0, st, a); break;
+  switch (a.rw / 8) {
+    VM_ROWS(1) VM_ROWS(2) VM_ROWS(3) VM_ROWS(4) VM_ROWS(5) VM_ROWS(6)
+    VM_ROWS(7) VM_ROWS(8) VM_ROWS(9) VM_ROWS(10) VM_ROWS(11) VM_ROWS(12)
+  }
+#undef VM_ROWS
+}
+
+// rows per workgroup, one workgroup per CU (a multiple of 8; of the packed gate-up:
+// RW / 2 gate and as many up rows), 0 where they are more than a workgroup takes
+int gemv_rows_plan(int M) {
+  const int cus = max(1, lm_head_waves() / 4);
+  const int rw = 8 * ((M + 8 * cus - 1) / (8 * cus));
+  return rw <= 8 * GR_MAX ? rw : 0;
+}
+
+hipError_t launch_gemv_rows(const GemvRowsArgs& a, bool silu, hipStream_t st) {
+  const int rows = silu ? a.rw / 2 : a.rw;
+  const int wgs = (a.M + rows - 1) / rows;
+  if (wgs == 0 || a.N == 0) return hipSuccess;
+  if (silu) launch_gemv_rows_t<true>(a, wgs, st);
+  else launch_gemv_rows_t<false>(a, wgs, st);
+  return hipGetLastError();
+}
+
 GemvSkPlan gemv_sk_plan(int M, int K) {
   GemvSkPlan p;
   p.G = K / 64;
