@@ -101,6 +101,16 @@ def test_fused_prefill_small_ragged(vm, orc):
     assert mx <= TOL_MAX and mn <= TOL_MEAN and kmx <= TOL_MAX and kmn <= TOL_MEAN and ok
 
 
+@pytest.mark.parametrize("ctx", [33, 34, 36, 38, 68, 97])
+def test_fused_prefill_cache_ends_in_tile(vm, orc, ctx):
+    """The attended keys end with the cache, 1 to 6 rows into a 32-key tile: the
+    tile's other rows re-read the cache's last one, which lies before the 1-KB
+    pieces the loads' immediate offsets step over."""
+    (mx, mn), (kmx, kmn), ok, _ = _fused(vm, orc, 2, ctx, ctx, np.array([0, 5], np.int32),
+                                         np.array([ctx, ctx - 5], np.int32), 57)
+    assert mx <= TOL_MAX and mn <= TOL_MEAN and kmx <= TOL_MAX and kmn <= TOL_MEAN and ok
+
+
 def test_config2_prefill_full_size(vm, orc):
     """causal prefill, B=1, T=4096, offset 0; every query row
     re-evaluated by the oracle, every appended K/V row checked."""

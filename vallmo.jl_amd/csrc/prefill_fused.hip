@@ -222,15 +222,20 @@ __global__ __launch_bounds__(64 * VT_WAVES) void vt_transpose_kernel(VtArgs a) {
   }
 }
 
+// The offsets are unsigned: the bias keeps the least of them (row 0 in piece 3) from
+// wrapping to 4 GB past the cache.
+constexpr uint32_t K_BIAS = 3 * 1024;
+
 struct FCtx {
-  const uint16_t* kbase;
+  const uint16_t* kbase;   // K rows of (b, hk), less K_BIAS bytes
   const uint16_t* vtbase;  // V^T tiles of (b, hk): 16 KB each
   int64_t kv_st;
   int krow_max;   // last cache row that may be read
   int n_tiles;
   uint32_t row_bytes;   // cache row stride in bytes
   // per-lane byte offsets of this wave's 4 one-KB pieces of a tile, less 1 KB per
-  // piece (the load's immediate offset adds it back, and moves the LDS side too)
+  // piece (the load's immediate offset adds it back, and moves the LDS side too) and
+  // plus K_BIAS, which kbase is less: a clamped row can lie before 1024 i
   uint32_t dma_boff[4];
   uint32_t dma_clamp[4];  // the same for the tile that reaches past the cache
   int t_part;             // that tile, or -1
@@ -302,7 +307,7 @@ __device__ __forceinline__ ItemGeo item_geo(const PrefillArgs& a, const FItem& i
 
 __device__ __forceinline__ void init_fctx(FCtx& c, const PrefillArgs& a, const ItemGeo& ig,
                                           int wave, int lane) {
-  c.kbase = a.k + (int64_t)ig.b * a.kv_sb + (int64_t)ig.hk * a.kv_sh;
+  c.kbase = a.k + (int64_t)ig.b * a.kv_sb + (int64_t)ig.hk * a.kv_sh - K_BIAS / 2;
   c.vtbase = a.vt + ((int64_t)ig.b * a.Hk + ig.hk) * a.vt_tiles * FT;
   c.kv_st = a.kv_st;
   c.krow_max = a.Lk - 1;  // rows up to here are readable (past k_len: masked)
@@ -319,8 +324,8 @@ __device__ __forceinline__ void init_fctx(FCtx& c, const PrefillArgs& a, const I
   for (int i = 0; i < 4; ++i) {
     const int r = 2 * (4 * wave + i) + (lane >> 5);
     const uint32_t chunk = (uint32_t)(((lane & 31) ^ fswz(r)) * 16);
-    c.dma_boff[i] = (uint32_t)r * c.row_bytes + chunk - 1024u * i;
-    c.dma_clamp[i] = (uint32_t)min(r, max(last, 0)) * c.row_bytes + chunk - 1024u * i;
+    c.dma_boff[i] = (uint32_t)r * c.row_bytes + chunk + (K_BIAS - 1024u * i);
+    c.dma_clamp[i] = (uint32_t)min(r, max(last, 0)) * c.row_bytes + chunk + (K_BIAS - 1024u * i);
   }
 }
 
