@@ -190,6 +190,37 @@ def test_decode_splits_agree(vm):
         assert mx <= 4e-3
 
 
+@pytest.mark.parametrize("Dh,causal,B,H,Hk,L,Lk", [
+    (128, True, 2, 8, 2, 65, 65), (128, False, 1, 4, 4, 33, 31), (64, True, 1, 16, 2, 129, 160),
+    (128, True, 2, 8, 1, 40, 33), (64, False, 3, 8, 8, 128, 97),
+    (128, True, 8, 80, 8, 32, 96), (64, True, 9, 65, 5, 20, 50), (128, False, 8, 64, 8, 16, 64)])
+def test_attention_key_groups(vm, orc, Dh, causal, B, H, Hk, L, Lk):
+    """attention! at D = 128 and 64 on both sides of the key-group rule (few query
+    blocks: two groups of waves split the keys; many: one): one key tile, an odd
+    count, more queries than keys (causal rows before the first key give 0),
+    ragged lengths with a sequence of no keys."""
+    banner(f"attention_ key groups D={Dh} causal={causal} B={B} H={H}/{Hk} L={L} Lk={Lk}")
+    q_bits = normal_bf16((B, H, L, Dh), 428)
+    k_bits = normal_bf16((B, Hk, Lk, Dh), 429)
+    v_bits = normal_bf16((B, Hk, Lk, Dh), 430)
+    kl = np.full(B, Lk, np.int32)
+    ql = np.full(B, L, np.int32)
+    if B > 1:
+        kl[-1], ql[-1] = 0, L // 2
+    O = torch.full((B, H, L, Dh), 7.0, dtype=torch.bfloat16, device="cuda")
+    vm.attention_({"O": O}, to_dev(q_bits), to_dev(k_bits), to_dev(v_bits), causal=causal,
+                  k_lengths=i32(kl), q_lengths=i32(ql))
+    torch.cuda.synchronize()
+    ref = orc.attention(bf16_to_f32(q_bits), bf16_to_f32(k_bits), bf16_to_f32(v_bits),
+                        causal=causal, k_lengths=kl, q_lengths=ql)
+    got = dev_f32(O)
+    fin = ~np.isnan(ref)
+    mx, mn = maxmean(got[fin], ref[fin])
+    print(f"max {mx:.3e} mean {mn:.3e}")
+    assert mx <= TOL_MAX and mn <= TOL_MEAN
+    assert (got[~fin] == 7.0).all()
+
+
 def _decode_bound(ref, v):
     """The bf16 rounding of the result (half an ulp: 2^-8 of the result's power of
     two) plus what the fp32 products leave: p is held to 2^-17 of itself (its two

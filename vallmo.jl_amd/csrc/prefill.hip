@@ -3,8 +3,9 @@
 // for CDNA4) on already-normalised q. The gated layer path with its fused
 // prologue and epilogue is prefill_fused.hip.
 //
-// Workgroup = 4 waves = 128 query rows of one (head, sequence); wave w owns 32
-// rows. Per 32-key tile, all on 32x32x16 bf16 MFMA with fp32 accumulate:
+// Workgroup = 128 query rows of one (head, sequence): four waves of 32 rows, or
+// eight in two groups that split the keys (see the key groups below). Per 32-key
+// tile, all on 32x32x16 bf16 MFMA with fp32 accumulate:
 //   S^T[key][row] = K[key][:] . Q[row][:]         A = K (LDS, ds_read_b128),
 //                                                 B = Q (registers, loaded once)
 //   O^T[d][row]  += V^T[d][key] . P^T[key][row]   A = V^T (LDS, ds_read_b64_tr_b16),
@@ -71,21 +72,31 @@ __device__ __forceinline__ void lds_barrier() {
 // 64 banks of 4 bytes).
 __device__ __forceinline__ int swz_pf(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
+// Key groups: NG groups of four waves share the workgroup's 128 rows, group g
+// taking the key tiles g, g + NG, ... (its j-th tile is tile NG j + g) through a ring
+// of its own; the groups' sums are merged through LDS at the end. At D = 256 one
+// group's ring and registers fill the CU (NG = 1). At D = 128 and 64 a CU holds two
+// and three workgroups of one group, or one of two: either way two waves or more
+// on a SIMD, one's softmax under the other's MFMAs. launch_prefill chooses.
+// waves per SIMD to compile for
+template <int D, int NG> constexpr int pf_waves() { return D == 256 ? 1 : NG == 2 || D == 128 ? 2 : 3; }
+
 struct PrefillCtx {
   const uint16_t* kbase;   // K rows of (b, hk)
   const uint16_t* vbase;
   int64_t kv_st;
-  int k_len, off, row, wrow0, wrow1, q_len, lane, wave;
+  int k_len, off, row, wrow0, wrow1, q_len, lane, wave, grp;
   int krow_max;            // last row that may be read (finite data)
   int dma_off[4];          // per-lane element offsets of this wave's DMA slots
 };
 
-// Issue this wave's share (SPW K + SPW V instructions of 1 KB) of tile `jt`.
-template <int D>
+// Issue this wave's share (SPW K + SPW V instructions of 1 KB) of its group's tile
+// `jt`.
+template <int D, int NG>
 __device__ __forceinline__ void issue_tile(const PrefillCtx& c, int jt, uint16_t* kd,
                                            uint16_t* vd) {
   using Sh = PfShape<D>;
-  const int row0 = jt * PF_BN;
+  const int row0 = (NG * jt + c.grp) * PF_BN;
   if (row0 + PF_BN - 1 <= c.krow_max) {
     // whole tile in range: uniform tile base + precomputed per-lane offsets
     const uint16_t* kt = c.kbase + (int64_t)row0 * c.kv_st;
@@ -143,7 +154,7 @@ __device__ __forceinline__ f32x16 qk_tile(const uint16_t* kb, const uint4 (&qop)
 template <bool CAUSAL>
 __device__ __forceinline__ void mask_tile(const PrefillCtx& c, int jt, f32x16& s) {
   const int lim = CAUSAL ? min(c.k_len - 1, c.row + c.off) : c.k_len - 1;
-  const int key0 = jt * PF_BN + 4 * (c.lane >> 5);
+  const int key0 = jt * PF_BN + 4 * (c.lane >> 5);  // jt: the tile itself
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int key = key0 + 8 * (j >> 2) + (j & 3);
@@ -154,7 +165,7 @@ __device__ __forceinline__ void mask_tile(const PrefillCtx& c, int jt, f32x16& s
 // One pipelined iteration on ring slot SLOT = jt % 4: wait for tile jt+1, issue
 // tile jt+3, then QK(jt+1) on the matrix cores while the VALU runs softmax(jt),
 // then PV(jt). `sc` holds S^T of tile jt on entry and of tile jt+1 on exit.
-template <bool CAUSAL, int SLOT, int D>
+template <bool CAUSAL, int SLOT, int D, int NG>
 __device__ __forceinline__ void tile_step(const PrefillCtx& c, int jt, int n_tiles, int my_tiles,
                                           uint16_t* const (&K)[4], uint16_t* const (&V)[4],
                                           const uint4 (&qop)[16], f32x16 (&acc)[8], f32x16& sc,
@@ -167,12 +178,13 @@ __device__ __forceinline__ void tile_step(const PrefillCtx& c, int jt, int n_til
   else
     wait_vmcnt<0>();
   lds_barrier();
-  if (jt + 3 < n_tiles) issue_tile<D>(c, jt + 3, K[(SLOT + 3) & 3], V[(SLOT + 3) & 3]);
+  if (jt + 3 < n_tiles) issue_tile<D, NG>(c, jt + 3, K[(SLOT + 3) & 3], V[(SLOT + 3) & 3]);
   if (jt >= my_tiles) return;
 
-  const bool need_mask = (jt * PF_BN + PF_BN > c.k_len) ||
-                         (CAUSAL && jt * PF_BN + PF_BN - 1 > c.off + c.wrow0);
-  if (need_mask) mask_tile<CAUSAL>(c, jt, sc);
+  const int tile = NG * jt + c.grp;
+  const bool need_mask = (tile * PF_BN + PF_BN > c.k_len) ||
+                         (CAUSAL && tile * PF_BN + PF_BN - 1 > c.off + c.wrow0);
+  if (need_mask) mask_tile<CAUSAL>(c, tile, sc);
 
   // S^T of the next tile (its slot is resident; past this wave's last tile the
   // result is simply unused)
@@ -224,9 +236,11 @@ __device__ __forceinline__ void tile_step(const PrefillCtx& c, int jt, int n_til
   sc = sn;
 }
 
-// Ring of 4 tile slots; tiles 0..2 are issued by the caller.
-template <bool CAUSAL, int D>
-__device__ __forceinline__ void tile_loop(const PrefillCtx& c, int n_tiles, int my_tiles,
+// Ring of 4 tile slots; tiles 0..2 are issued by the caller. n_loop: the steps
+// (barriers) of the workgroup, those of the group with most tiles; n_tiles: this
+// group's tiles.
+template <bool CAUSAL, int D, int NG>
+__device__ __forceinline__ void tile_loop(const PrefillCtx& c, int n_loop, int n_tiles, int my_tiles,
                                           uint16_t* const (&K)[4], uint16_t* const (&V)[4],
                                           const uint4 (&qop)[16], f32x16 (&acc)[8],
                                           float& m_run, float& l_part, const int (&koff)[8],
@@ -241,28 +255,32 @@ __device__ __forceinline__ void tile_loop(const PrefillCtx& c, int n_tiles, int 
   lds_barrier();
   f32x16 sc;
   if (my_tiles > 0) sc = qk_tile<D>(K[0], qop, koff);
-  for (int jt = 0; jt < n_tiles; jt += 4) {
-    tile_step<CAUSAL, 0, D>(c, jt, n_tiles, my_tiles, K, V, qop, acc, sc, m_run, l_part,
+  for (int jt = 0; jt < n_loop; jt += 4) {
+    tile_step<CAUSAL, 0, D, NG>(c, jt, n_tiles, my_tiles, K, V, qop, acc, sc, m_run, l_part,
                                  koff, voff);
-    if (jt + 1 < n_tiles)
-      tile_step<CAUSAL, 1, D>(c, jt + 1, n_tiles, my_tiles, K, V, qop, acc, sc, m_run,
+    if (jt + 1 < n_loop)
+      tile_step<CAUSAL, 1, D, NG>(c, jt + 1, n_tiles, my_tiles, K, V, qop, acc, sc, m_run,
                                    l_part, koff, voff);
-    if (jt + 2 < n_tiles)
-      tile_step<CAUSAL, 2, D>(c, jt + 2, n_tiles, my_tiles, K, V, qop, acc, sc, m_run,
+    if (jt + 2 < n_loop)
+      tile_step<CAUSAL, 2, D, NG>(c, jt + 2, n_tiles, my_tiles, K, V, qop, acc, sc, m_run,
                                    l_part, koff, voff);
-    if (jt + 3 < n_tiles)
-      tile_step<CAUSAL, 3, D>(c, jt + 3, n_tiles, my_tiles, K, V, qop, acc, sc, m_run,
+    if (jt + 3 < n_loop)
+      tile_step<CAUSAL, 3, D, NG>(c, jt + 3, n_tiles, my_tiles, K, V, qop, acc, sc, m_run,
                                    l_part, koff, voff);
   }
 }
 
-template <bool CAUSAL, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <bool CAUSAL, int D, int NG>
+__global__ __launch_bounds__(256 * NG)
+__attribute__((amdgpu_waves_per_eu(pf_waves<D, NG>())))
 void prefill_kernel(PrefillArgs a) {
   using Sh = PfShape<D>;
   constexpr int TILE = Sh::TILE;
-  __shared__ __attribute__((aligned(1024))) uint16_t K0[TILE], K1[TILE], K2[TILE], K3[TILE];
-  __shared__ __attribute__((aligned(1024))) uint16_t V0[TILE], V1[TILE], V2[TILE], V3[TILE];
+  __shared__ __attribute__((aligned(1024))) uint16_t K0s[NG][TILE], K1s[NG][TILE], K2s[NG][TILE], K3s[NG][TILE];
+  __shared__ __attribute__((aligned(1024))) uint16_t V0s[NG][TILE], V1s[NG][TILE], V2s[NG][TILE], V3s[NG][TILE];
+  const int grp = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  uint16_t *const K0 = K0s[grp], *const K1 = K1s[grp], *const K2 = K2s[grp], *const K3 = K3s[grp];
+  uint16_t *const V0 = V0s[grp], *const V1 = V1s[grp], *const V2 = V2s[grp], *const V3 = V3s[grp];
   uint16_t* const K[4] = {K0, K1, K2, K3};
   uint16_t* const V[4] = {V0, V1, V2, V3};
 
@@ -276,7 +294,7 @@ void prefill_kernel(PrefillArgs a) {
   const int b = hb / a.H, h = hb % a.H;
   const int hk = h / (a.H / a.Hk);
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = (tid >> 6) & 3, lane = tid & 63;
   const int l32 = lane & 31, h2 = lane >> 5;
   const int r0 = qt * PF_BM;
   const int row = r0 + 32 * wave + l32;  // query row in the chunk
@@ -298,7 +316,10 @@ void prefill_kernel(PrefillArgs a) {
   const int k_len = a.k_lengths ? max(0, min(a.k_lengths[b], a.Lk)) : a.Lk;
   const int off = k_len - q_len;  // queries are the suffix of keys
   const int kend = CAUSAL ? min(k_len, off + r0 + PF_BM) : k_len;
-  const int n_tiles = kend > 0 ? (kend + PF_BN - 1) / PF_BN : 0;
+  const int all_tiles = kend > 0 ? (kend + PF_BN - 1) / PF_BN : 0;
+  // the group's share of the first n tiles
+  auto share = [&](int n) __attribute__((always_inline)) { return max(0, (n - grp + NG - 1) / NG); };
+  const int n_tiles = share(all_tiles), n_loop = (all_tiles + NG - 1) / NG;
 
   PrefillCtx c;
   c.kbase = a.k + (int64_t)b * a.kv_sb + (int64_t)hk * a.kv_sh;
@@ -306,7 +327,7 @@ void prefill_kernel(PrefillArgs a) {
   c.kv_st = a.kv_st;
   c.k_len = k_len; c.off = off; c.row = row; c.q_len = q_len;
   c.wrow0 = r0 + 32 * wave; c.wrow1 = c.wrow0 + 31;
-  c.lane = lane; c.wave = wave;
+  c.lane = lane; c.wave = wave; c.grp = grp;
   c.krow_max = max(0, k_len - 1);  // rows past k_len are masked; read finite data
 #pragma unroll
   for (int i = 0; i < Sh::SPW; ++i) {
@@ -316,12 +337,13 @@ void prefill_kernel(PrefillArgs a) {
 
   // the first three tiles go out before the q operand is formed so their
   // latency overlaps it
-  if (n_tiles > 0) issue_tile<D>(c, 0, K0, V0);
-  if (n_tiles > 1) issue_tile<D>(c, 1, K1, V1);
-  if (n_tiles > 2) issue_tile<D>(c, 2, K2, V2);
+  if (n_tiles > 0) issue_tile<D, NG>(c, 0, K0, V0);
+  if (n_tiles > 1) issue_tile<D, NG>(c, 1, K1, V1);
+  if (n_tiles > 2) issue_tile<D, NG>(c, 2, K2, V2);
   // tiles this wave computes (causal: keys <= off + its last row)
   int my_tiles = c.wrow0 < q_len ? n_tiles : 0;
-  if (CAUSAL && my_tiles > 0) my_tiles = max(0, min(n_tiles, (off + c.wrow1) / PF_BN + 1));
+  if (CAUSAL && my_tiles > 0)
+    my_tiles = off + c.wrow1 < 0 ? 0 : min(n_tiles, share((off + c.wrow1) / PF_BN + 1));
 
   // ---- Q operand: lane holds q[row][16kk + 8*h2 + j], pre-scaled by 1/16 at
   // D = 256 (a power of two: exact in bf16)
@@ -364,7 +386,42 @@ void prefill_kernel(PrefillArgs a) {
     for (int j = 0; j < 16; ++j) acc[i][j] = 0.f;
   float l_part = 0.f, m_run = -INFINITY;
 
-  tile_loop<CAUSAL, D>(c, n_tiles, my_tiles, K, V, qop, acc, m_run, l_part, koff, voff);
+  tile_loop<CAUSAL, D, NG>(c, n_loop, n_tiles, my_tiles, K, V, qop, acc, m_run, l_part, koff, voff);
+
+  // ---- the second group's sums into the first's, lane by lane (the same rows and
+  // columns): O, then m and l, through the tiles' LDS (every tile has been read)
+  if constexpr (NG > 1) {
+    static_assert(NG == 2 && sizeof(K0s) >= 32 * D * sizeof(float) && Sh::DT * 1024 <= TILE * 4,
+                  "one wave's O per slot array");
+    uint16_t* const slots[4] = {K0s[0], K1s[0], K2s[0], K3s[0]};
+    float* const o1 = reinterpret_cast<float*>(wave == 0 ? slots[0] : wave == 1 ? slots[1] : wave == 2 ? slots[2] : slots[3]);
+    float* const ml = reinterpret_cast<float*>(V0s[0]) + 128 * wave;
+    lds_barrier();
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < Sh::DT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<f32x4*>(o1 + ((4 * i + j) * 64 + lane) * 4) =
+              f32x4{acc[i][4 * j], acc[i][4 * j + 1], acc[i][4 * j + 2], acc[i][4 * j + 3]};
+      ml[lane] = m_run;
+      ml[64 + lane] = l_part;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float m1 = ml[lane], mm = fmaxf(m_run, m1);
+    const float a0 = m_run == mm ? 1.0f : fast_exp2(m_run - mm);
+    const float a1 = m1 == mm ? 1.0f : fast_exp2(m1 - mm);
+    l_part = l_part * a0 + ml[64 + lane] * a1;
+#pragma unroll
+    for (int i = 0; i < Sh::DT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 o = *reinterpret_cast<const f32x4*>(o1 + ((4 * i + j) * 64 + lane) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][4 * j + e] = acc[i][4 * j + e] * a0 + o[e] * a1;
+      }
+  }
 
   // ---- epilogue: normalise and store (row-major d within each row)
   if (row >= q_len) return;
@@ -387,22 +444,38 @@ void prefill_kernel(PrefillArgs a) {
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st) {
   const int64_t nwg = (int64_t)a.n_qt * a.H * a.B;
   if (nwg == 0) return hipSuccess;
-  dim3 grid((unsigned)nwg), block(256);
+  // Two key groups halve the walk over the keys that a query block makes alone; one
+  // leaves the CU to two independent blocks (three at D = 64), whose waves do not
+  // meet at one barrier. Causal blocks differ in length, so the longest walk
+  // decides while blocks are few: two groups against one, T = 4096, 16 heads (512
+  // blocks) 104 : 122 us at D = 128, 60 : 77 at D = 64; T = 2048 (256 blocks) 41 :
+  // 54; 576 blocks 86 : 86; 768 blocks 83 : 70. Without the mask all are as long,
+  // and one group wins once every CU has two blocks: 512 blocks 158 : 153. Before
+  // (one group, one block per CU at a time): 131 us causal, 231 without the mask.
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  const bool two = a.causal ? 4 * nwg <= 9 * cus : nwg < 2 * cus;
+  const dim3 grid((unsigned)nwg);
+#define VM_PREFILL(causal, d, ng) \
+  hipLaunchKernelGGL((prefill_kernel<causal, d, ng>), grid, dim3(256 * ng), 0, st, a)
+#define VM_PREFILL_D(d)                         \
+  if (a.causal && two) VM_PREFILL(true, d, 2);  \
+  else if (a.causal) VM_PREFILL(true, d, 1);    \
+  else if (two) VM_PREFILL(false, d, 2);        \
+  else VM_PREFILL(false, d, 1);
   if (a.D == 128) {
-    if (a.causal)
-      hipLaunchKernelGGL((prefill_kernel<true, 128>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((prefill_kernel<false, 128>), grid, block, 0, st, a);
+    VM_PREFILL_D(128)
   } else if (a.D == 64) {
-    if (a.causal)
-      hipLaunchKernelGGL((prefill_kernel<true, 64>), grid, block, 0, st, a);
-    else
-      hipLaunchKernelGGL((prefill_kernel<false, 64>), grid, block, 0, st, a);
+    VM_PREFILL_D(64)
   } else if (a.causal) {
-    hipLaunchKernelGGL((prefill_kernel<true, 256>), grid, block, 0, st, a);
+    VM_PREFILL(true, 256, 1);
   } else {
-    hipLaunchKernelGGL((prefill_kernel<false, 256>), grid, block, 0, st, a);
+    VM_PREFILL(false, 256, 1);
   }
+#undef VM_PREFILL_D
+#undef VM_PREFILL
   return hipGetLastError();
 }
 
