@@ -146,6 +146,7 @@ int vm_knorm_rope_append(vm_bf16* k_cache, int64_t kc_st, int64_t kc_sh, int64_t
  * scratch holds one fp32 partial (G*D values + G (max, sum) pairs) per wave
  * and per (b, hk) segment, then a snapshot of the partition (1 + 2B int32
  * in whole 256-byte blocks) that the merge reads instead of lengths.
+ * D = 128 and 64 run the same way (chunks of whole ring slots, 4096 / D tokens).
  *
  * Other shapes run a generic kernel with the reference's split: n_splits
  * tile-aligned key ranges per (b, hk) (n_splits = 0: about four workgroups
@@ -368,10 +369,11 @@ int vm_linear_add_rms_norm(vm_bf16* y, int64_t y_st, vm_bf16* x, int64_t x_st, c
  *                              rows I .. 2I-1; x :: (K, N)), rounded to bf16
  *   mid = silu(gate) .* up    fp32 from the bf16 gate and up, one rounding
  * for callers that want the bf16 gu never written. At N <= 32 (a decode
- * batch; K a multiple of 64, aligned columns) the projection runs a stream-K
- * GEMV whose fp32 partials the silu kernel adds in a fixed order (bitwise
- * repeatable; the same rounding points as the two calls, the sums in another
- * order). Otherwise it is linear! + silu .* mul. I a multiple of 8; mid a
+ * batch; K a multiple of 64, aligned columns) one launch does both while a CU's
+ * share of the 2I rows is at most 96, each workgroup holding its gate rows and
+ * the same up rows; above that a stream-K GEMV runs whose fp32 partials the
+ * silu kernel adds in a fixed order. Both are bitwise repeatable, with the same
+ * rounding points as the two calls and the sums in another order. Otherwise it is linear! + silu .* mul. I a multiple of 8; mid a
  * 16-byte aligned (I, N) with an element column stride (a multiple of 8);
  * workspace (256-byte aligned) of vm_linear_silu_mul_workspace_bytes bytes
  * ((size_t)-1 on a bad shape).                                              */

@@ -618,8 +618,9 @@ int linear_silu_mul_run(uint16_t* mid, int64_t mid_st, const uint16_t* x, int64_
   const bool decode = sk_shape(M, N, K, ldw, ldx) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   const int rw = decode ? gemv_rows_plan(M) : 0;
   if (rw > 0) {
-    // one launch (gate-up 18432 x 2560 and the silu
-    // at N = 8: 18.4 us against 19.0 + 4.1 us for the stream-K GEMV and its consumer)
+    // one launch (gate-up 18432 x 2560 and the silu at N = 8: 18.4 us against 19.0 +
+    // 4.1 us for the stream-K GEMV and its consumer); the two launches above 96 rows
+    // a CU, the most a workgroup takes
     return run_gemv_rows(mid, mid_st, x, ldx, w, ldw, I, N, K, rw, true, st, "linear_silu_mul", err,
                          errn);
   }
