@@ -425,6 +425,39 @@ def test_deltanet_conv_prep(vm, orc, B, T, prefix, bias, hk, hv):
                                    err_msg=key)
 
 
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("T", [1, 7, 8, 9, 25])
+def test_deltanet_conv_prep_runs(vm, taps, T):
+    """The one-pass conv and prep at the edges of its 8-token runs and of its blocks
+    of `taps` tokens, a ring as left context, updated in place, against the two
+    kernels, value for value; one q row's sum of squares overflows."""
+    banner(f"deltanet conv + prep runs taps={taps} T={T}")
+    B, hk, hv = 2, 2, 4
+    n = 2 * hk * DK + hv * DV
+    X = to_dev(normal_bf16((B, T, n), 2090 + T))
+    X[0, T - 1, :DK] = 3e38
+    AB = to_dev(normal_bf16((B, T, 2 * hv), 2091))
+    W = to_dev(normal_bf16((taps, n), 2092, scale=0.5))
+    A, Dt = f32dev(normal_f32(hv, 2095, scale=0.5)), f32dev(normal_f32(hv, 2096, scale=0.5))
+    S1 = to_dev(normal_bf16((B, taps, n), 2094))
+    S2 = S1.clone()
+
+    def outs():
+        f = dict(dtype=torch.float32, device="cuda")
+        return {"Q": torch.empty((B, hk, T, DK), **f), "K": torch.empty((B, hk, T, DK), **f),
+                "V": torch.empty((B, hv, T, DV), **f), "Beta": torch.empty((B, T, hv), **f),
+                "Gate": torch.empty((B, T, hv), **f)}
+
+    conv = vm.causal_conv1d_sequence(X, W, None, sigma="silu", Sp=S1, S=S1)["Y"]
+    two, one = outs(), outs()
+    vm.deltanet_prefill_prep_(two, conv, AB, A, Dt, Dk=DK, Dv=DV, Hk=hk, Hv=hv)
+    vm.deltanet_conv_prep_(one, X, W, AB, A, Dt, None, Dk=DK, Dv=DV, Hk=hk, Hv=hv, Sp=S2, S=S2)
+    torch.cuda.synchronize()
+    for key in one:
+        assert torch.allclose(one[key], two[key], rtol=0, atol=0, equal_nan=True), key
+    assert torch.equal(S1, S2)
+
+
 def test_prep_many_value_heads(vm, orc):
     """The prep with more value heads than a wave has lanes (Hk = 2, Hv = 72): the
     gates of heads 64 .. 71 too."""

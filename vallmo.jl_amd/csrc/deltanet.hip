@@ -1250,22 +1250,32 @@ __global__ __launch_bounds__(256) void conv1d_sequence_kernel(Conv1dArgs a) {
 }
 
 // ---- the prefill's conv and prep in one pass (qwen35.jl:333-356): thread = 8
-// channels x a run of CONV_TC tokens as in conv1d_sequence_kernel, the 16
+// channels x a run of PREP_TC tokens (conv1d_sequence_kernel's form), the 16
 // lanes of a head's 128 channels in one 16-lane group. Per token the conv
 // output is rounded to bf16 (the value the two-kernel form stores between the
 // kernels), then each q / k head row is scaled by its inverse L2 norm (q also
 // by Dk^-1/2) over the group, and the row is written fp32 to Q / K / V, head
 // major, as deltanet_prep_vec_kernel writes it: bit for bit the two-kernel
-// result, without the conv output's round trip through memory. Workgroup
-// column 0 also writes beta and the gate of its run's tokens.
+// result (a zero's sign aside), without the conv output's round trip through
+// memory. Workgroup column 0 also writes beta and the gate of its run's tokens.
+// Bound by VALU issue (silu's exp and division are most of ~400 instructions per
+// token and wave) beside 203 MB at T = 4096, so both are kept under way: the next
+// K tokens' rows load while K are computed, the window turns through K fixed
+// slots (no register moves), eight silus interleave, v skips the division and a
+// row of q or k divides once. Runs of 8 tokens put 8 waves on a SIMD at T = 4096
+// and 4 at 2000. B = 1, 8192 channels, T = 4096 / 2001: 66.5 / 41.0 -> 56.3 / 29.7
+// us; runs of 16 as before 57.6 / 31.9, of 12 58.4 / 32.4; the shorter runs
+// without the rest (9 tokens) 61.5 / 33.3.
+constexpr int PREP_TC = 8;
+
 template <int K>
 __global__ __launch_bounds__(256) void deltanet_conv_prep_kernel(ConvPrepArgs a) {
-  static_assert(CONV_TC >= K - 1, "run 0 must cover the context reads");
+  static_assert(PREP_TC >= K - 1, "run 0 must cover the context reads");
   const Conv1dArgs& c = a.c;
   const DeltaPrepArgs& p = a.p;
   const int run = blockIdx.y, b = blockIdx.z;
-  const int t0 = run * CONV_TC;
-  const int t1 = min(t0 + CONV_TC, c.T);
+  const int t0 = run * PREP_TC;
+  const int t1 = min(t0 + PREP_TC, c.T);
   if (blockIdx.x == 0) {
     const uint16_t* ab = p.ab + (int64_t)b * p.ab_sb;
     for (int i = threadIdx.x; i < (t1 - t0) * p.Hv; i += 256) {
@@ -1297,39 +1307,67 @@ __global__ __launch_bounds__(256) void deltanet_conv_prep_kernel(ConvPrepArgs a)
   float win[K][8];  // win[i] = ext(t - K + 1 + i) for the current t
 #pragma unroll
   for (int i = 0; i < K - 1; ++i) unpack8(conv_ext<K>(c, b, d, t0 - K + 1 + i), win[i]);
-  for (int t = t0; t < t1; ++t) {
-    unpack8(conv_ext<K>(c, b, d, t), win[K - 1]);
-    float acc[8];
+  // the next block's K rows (past the run: its last row again, unused)
+  const uint16_t* xr = c.x + b * c.x_sb + d;
+  uint4 nx[K];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float v = 0.f;
+  for (int j = 0; j < K; ++j)
+    nx[j] = *reinterpret_cast<const uint4*>(xr + (int64_t)min(t0 + j, t1 - 1) * c.x_st);
+  for (int tb = t0; tb < t1; tb += K) {
+    uint4 cur[K];
 #pragma unroll
-      for (int i = 0; i < K; ++i) v += win[i][e] * wf[i][e];
-      v += bias8[e];
-      acc[e] = c.act ? accurate_silu(v) : v;
-    }
-    float x[8];
-    unpack8(pack8(acc), x);  // the conv output, bf16
-    float den = 1.0f;
-    if (qk) {
-      float ss = 0.f;
+    for (int j = 0; j < K; ++j) cur[j] = nx[j];
+    if (tb + K < t1) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
-      ss += xor32<8>(ss);
-      ss += xor32<4>(ss);
-      ss += xor32<2>(ss);
-      ss += xor32<1>(ss);
-      den = sqrtf(ss + 1e-6f);
+      for (int j = 0; j < K; ++j)
+        nx[j] = *reinterpret_cast<const uint4*>(xr + (int64_t)min(tb + K + j, t1 - 1) * c.x_st);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = x[j] / den * sc;
-    float4* d4 = reinterpret_cast<float4*>(dst + (int64_t)t * DN_D);
-    d4[0] = make_float4(x[0], x[1], x[2], x[3]);
-    d4[1] = make_float4(x[4], x[5], x[6], x[7]);
+    for (int u = 0; u < K; ++u) {
+      const int t = tb + u;
+      if (t >= t1) break;
+      unpack8(cur[u], win[(u + K - 1) % K]);  // ext(t - K + 1 + i) is in slot (u + i) % K
+      float acc[8];
 #pragma unroll
-    for (int i = 0; i + 1 < K; ++i)
+      for (int e = 0; e < 8; ++e) {
+        float v = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) win[i][e] = win[i + 1][e];
+        for (int i = 0; i < K; ++i) v += win[(u + i) % K][e] * wf[i][e];
+        acc[e] = v + bias8[e];
+      }
+      if (c.act) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = accurate_silu(acc[e]);
+      }
+      float x[8];
+      unpack8(pack8(acc), x);  // the conv output, bf16
+      if (qk) {  // (v: the value itself)
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+        ss += xor32<8>(ss);
+        ss += xor32<4>(ss);
+        ss += xor32<2>(ss);
+        ss += xor32<1>(ss);
+        const float den = sqrtf(ss + 1e-6f);
+        if (den < INFINITY) {
+          // x / den, correctly rounded, from the row's one reciprocal: the quotient's
+          // exact remainder corrects it
+          const float inv = 1.0f / den;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float y = x[j] * inv;
+            x[j] = fmaf(fmaf(-y, den, x[j]), inv, y) * sc;
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = x[j] / den * sc;
+        }
+      }
+      float4* d4 = reinterpret_cast<float4*>(dst + (int64_t)t * DN_D);
+      d4[0] = make_float4(x[0], x[1], x[2], x[3]);
+      d4[1] = make_float4(x[4], x[5], x[6], x[7]);
+    }
   }
   if (run == 0 && c.s_out) {
     uint4 seed[K];  // column i = ext(T - K + i); every column read first (aliasing)
@@ -1480,7 +1518,7 @@ hipError_t launch_conv1d_update_sk(const Conv1dSkArgs& a, hipStream_t st) {
 
 hipError_t launch_deltanet_conv_prep(const ConvPrepArgs& a, hipStream_t st) {
   if (a.c.B == 0 || a.c.T == 0) return hipSuccess;
-  const int runs = (a.c.T + CONV_TC - 1) / CONV_TC;
+  const int runs = (a.c.T + PREP_TC - 1) / PREP_TC;
   const dim3 grid((unsigned)((a.c.D / 8 + 255) / 256), runs, a.c.B);
   switch (a.c.K) {
 #define X(k) \
