@@ -801,7 +801,7 @@ def bench_deltanet(vm, torch, seed=11):
     yb = torch.empty((B, T, Hv, Dv), dtype=torch.bfloat16, device="cuda")
     us_gn = _profiled_us(vm, torch, vm._lib.VM_K_ROWS,
                          lambda: vm.gated_rms_norm_(yb, o, z, gw, eps=EPS), n=5)
-    # the layer's form: the chunked recurrence with the gated norm in its output kernel
+    # the layer's form: the chunked recurrence and its gated norm
     us_chk_gn = _profiled_us(vm, torch, vm._lib.VM_K_DELTANET,
                              lambda: vm.deltanet_sequence_chunked_gated_norm_(
                                  {"Y": yb, "Sp": S}, z, gw, p["Q"], p["K"], p["V"], p["Beta"],
