@@ -134,6 +134,22 @@ def test_generic_decode_scratch(vm):
     assert rc == vm._lib.VM_E_SCRATCH
 
 
+@pytest.mark.parametrize("B,Hk,n_splits", [(511, 128, 640), (255, 257, 65535)])
+def test_decode_scratch_of_many_splits(vm, B, Hk, n_splits):
+    """At D = 64 a wave count (n_splits B Hk) whose token-heads, at 64 a wave, pass
+    2^31 is the generic kernel's, one (D + 2)-float row per split, sequence and
+    head: the stream kernel's first token-head of such a wave would wrap to a
+    negative one, and its loads with it. Just below the limit the stream kernel
+    takes the problem, one partial row per wave more than that."""
+    lib = vm._lib.load()
+    rows = n_splits * B * Hk
+    assert rows * 64 >= 1 << 31
+    up = lambda n: -(-n // 256) * 256
+    assert lib.vm_decode_scratch_bytes(B, Hk, Hk, 64, 4096, n_splits) == up(rows * 66 * 4)
+    few = (1 << 24) // (B * Hk)
+    assert lib.vm_decode_scratch_bytes(B, Hk, Hk, 64, 4096, few) > up(few * B * Hk * 66 * 4)
+
+
 def test_decode_rejects_unsupported_head_dim(vm):
     lib = vm._lib.load()
     rc = lib.vm_decode_attention(_p(FAKE), 1024, 4096, _p(FAKE), 1024, 4096, _p(FAKE), 1024,

@@ -363,9 +363,10 @@ __device__ __forceinline__ bool stream_partition(const DecodeArgs& a, int w, int
     }
     if (lane == 0) a.geom[0] = chunk;
   }
-  gw0 = w * chunk;
-  if (gw0 >= W) return false;
-  gw1 = min(gw0 + chunk, W);
+  const int64_t first = (int64_t)w * chunk;  // past W for the last of many waves
+  if (first >= W) return false;
+  gw0 = uniform((int)first);
+  gw1 = uniform((int)min(first + chunk, (int64_t)W));
 
   // ---- locate the segment holding gw0: first b whose prefix (token-heads) passes it
   b = 0;

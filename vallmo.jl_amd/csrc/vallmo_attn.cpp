@@ -345,11 +345,26 @@ static size_t generic_decode_scratch_bytes(int B, int H, int Hk, int Dv, int64_t
   return ((size_t)ns * B * H * (Dv + 2) * sizeof(float) + 255) / 256 * 256;
 }
 
+// The problems of the stream kernels: D = 256, 128 and 64, groups up to 8 and
+// fewer than 2^31 token-heads. At D = 128 and 64, which the generic kernel
+// serves as well, also its grid limits, and at most 2^24 waves asked for through
+// n_splits: a wave past the last token-head does nothing but its launch and its
+// share of the workspace, and counts past 2^31 would wrap.
+static bool stream_decode_shape(int B, int H, int Hk, int D, int64_t ctx, int n_splits) {
+  if ((D != vm::HEAD_DIM_ABI && D != 128 && D != 64) || H / Hk > 8 ||
+      (int64_t)B * ctx * Hk >= ((int64_t)1 << 31))
+    return false;
+  const int64_t segs = (int64_t)B * Hk;
+  return D == vm::HEAD_DIM_ABI ||
+         (segs <= 65535 && n_splits <= 65535 && n_splits * segs <= ((int64_t)1 << 24));
+}
+
 size_t vm_decode_scratch_bytes(int B, int H, int Hk, int D, int64_t ctx, int n_splits) {
   if (B <= 0 || H <= 0 || Hk <= 0 || H % Hk || ctx <= 0 || n_splits < 0) return 0;
   if (D < 16 || D > 512 || (D & (D - 1))) return 0;
   const size_t generic = generic_decode_scratch_bytes(B, H, Hk, D, ctx, n_splits);
-  if ((D != vm::HEAD_DIM_ABI && D != 128 && D != 64) || H / Hk > 8) return generic;
+  if (D != vm::HEAD_DIM_ABI ? !stream_decode_shape(B, H, Hk, D, ctx, n_splits) : H / Hk > 8)
+    return generic;
   return std::max(generic, tuned_decode_scratch_bytes(B, H, Hk, D, ctx, n_splits));
 }
 
@@ -401,15 +416,13 @@ int vm_decode_attention(vm_bf16* o, int64_t o_sh, int64_t o_sb, const vm_bf16* q
   TRY(check_gqa(H, Hk));
   REQUIRE(n_splits >= 0, VM_E_ARG, "decode: n_splits = %d", n_splits);
   REQUIRE(ctx > 0, VM_E_ARG, "decode: Ctx = %lld", (long long)ctx);
-  // The stream kernels take D = 256, 128 and 64, groups up to 8, one set of
-  // K/V strides and 2^31 token-heads. At D = 128 and 64 the generic kernel keeps
-  // what only it serves: a workspace sized for it alone, and its own limits.
-  bool tuned = (Dk == vm::HEAD_DIM_ABI || Dk == 128 || Dk == 64) && Dv == Dk && H / Hk <= 8 &&
-               k_st == v_st && k_sh == v_sh && k_sb == v_sb &&
-               (int64_t)B * ctx * Hk < ((int64_t)1 << 31);
+  // The stream kernels take their problems with one set of K/V strides. At D = 128
+  // and 64 the generic kernel keeps what only it serves, among it a workspace
+  // sized for it alone.
+  bool tuned = Dv == Dk && k_st == v_st && k_sh == v_sh && k_sb == v_sb &&
+               stream_decode_shape(B, H, Hk, Dk, ctx, n_splits);
   if (Dk != vm::HEAD_DIM_ABI)
-    tuned = tuned && (int64_t)B * Hk <= 65535 && n_splits <= 65535 &&
-            scratch_bytes >= tuned_decode_scratch_bytes(B, H, Hk, Dk, ctx, n_splits);
+    tuned = tuned && scratch_bytes >= tuned_decode_scratch_bytes(B, H, Hk, Dk, ctx, n_splits);
   if (!tuned) {  // the generic split-KV kernel and its merge
     REQUIRE((int64_t)B * Hk <= 65535 && n_splits <= 65535, VM_E_UNSUPPORTED,
             "decode: B*Hk = %lld, n_splits = %d (at most 65535 each)", (long long)B * Hk,
