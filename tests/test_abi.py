@@ -150,6 +150,20 @@ def test_decode_scratch_of_many_splits(vm, B, Hk, n_splits):
     assert lib.vm_decode_scratch_bytes(B, Hk, Hk, 64, 4096, few) > up(few * B * Hk * 66 * 4)
 
 
+@pytest.mark.parametrize("D,n_splits", [(64, 0), (64, 8), (128, 0), (128, 8), (512, 0)])
+def test_decode_empty_batch(vm, D, n_splits):
+    """An empty batch needs no workspace (vm_decode_scratch_bytes is 0) and launches
+    nothing, at the head dims of the generic kernel and of the stream kernel
+    beside it."""
+    lib = vm._lib.load()
+    assert lib.vm_decode_scratch_bytes(0, 16, 4, D, 512, n_splits) == 0
+    st = (D, 16 * D, D, 512 * D, 4 * 512 * D)
+    rc = lib.vm_decode_attention(_p(FAKE), st[0], st[1], _p(FAKE), st[0], st[1], _p(FAKE), *st[2:],
+                                 _p(FAKE), *st[2:], 512, _p(FAKE), 0, 16, 4, D, D, n_splits,
+                                 _p(FAKE), 0, None)
+    assert rc == 0, lib.vm_last_error().decode()
+
+
 def test_decode_rejects_unsupported_head_dim(vm):
     lib = vm._lib.load()
     rc = lib.vm_decode_attention(_p(FAKE), 1024, 4096, _p(FAKE), 1024, 4096, _p(FAKE), 1024,

@@ -341,6 +341,7 @@ static size_t tuned_decode_scratch_bytes(int B, int H, int Hk, int D, int64_t ct
 // sequence and head (the reference's O_partial, M_partial, L_partial)
 static size_t generic_decode_scratch_bytes(int B, int H, int Hk, int Dv, int64_t ctx,
                                            int n_splits) {
+  if (B == 0) return 0;
   const int ns = vm::attn_any_splits(B, H, Hk, ctx, n_splits);
   return ((size_t)ns * B * H * (Dv + 2) * sizeof(float) + 255) / 256 * 256;
 }
@@ -418,11 +419,12 @@ int vm_decode_attention(vm_bf16* o, int64_t o_sh, int64_t o_sb, const vm_bf16* q
   REQUIRE(ctx > 0, VM_E_ARG, "decode: Ctx = %lld", (long long)ctx);
   // The stream kernels take their problems with one set of K/V strides. At D = 128
   // and 64 the generic kernel keeps what only it serves, among it a workspace
-  // sized for it alone.
+  // sized for it alone and an empty batch, which needs none.
   bool tuned = Dv == Dk && k_st == v_st && k_sh == v_sh && k_sb == v_sb &&
                stream_decode_shape(B, H, Hk, Dk, ctx, n_splits);
   if (Dk != vm::HEAD_DIM_ABI)
-    tuned = tuned && scratch_bytes >= tuned_decode_scratch_bytes(B, H, Hk, Dk, ctx, n_splits);
+    tuned = tuned && B > 0 &&
+            scratch_bytes >= tuned_decode_scratch_bytes(B, H, Hk, Dk, ctx, n_splits);
   if (!tuned) {  // the generic split-KV kernel and its merge
     REQUIRE((int64_t)B * Hk <= 65535 && n_splits <= 65535, VM_E_UNSUPPORTED,
             "decode: B*Hk = %lld, n_splits = %d (at most 65535 each)", (long long)B * Hk,
