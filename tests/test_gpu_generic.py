@@ -193,12 +193,17 @@ def test_decode_splits_agree(vm):
 @pytest.mark.parametrize("Dh,causal,B,H,Hk,L,Lk", [
     (128, True, 2, 8, 2, 65, 65), (128, False, 1, 4, 4, 33, 31), (64, True, 1, 16, 2, 129, 160),
     (128, True, 2, 8, 1, 40, 33), (64, False, 3, 8, 8, 128, 97),
-    (128, True, 8, 80, 8, 32, 96), (64, True, 9, 65, 5, 20, 50), (128, False, 8, 64, 8, 16, 64)])
+    (128, True, 8, 80, 8, 32, 96), (64, True, 9, 65, 5, 20, 50), (128, False, 8, 64, 8, 16, 64),
+    (128, True, 2, 8, 2, 65, 385), (64, True, 1, 16, 2, 129, 257), (128, False, 3, 4, 4, 33, 353),
+    (64, False, 3, 8, 8, 130, 420), (128, True, 2, 8, 1, 400, 356), (64, True, 2, 8, 1, 300, 290),
+    (128, False, 2, 4, 2, 40, 352), (64, False, 2, 4, 2, 40, 256), (128, True, 2, 33, 1, 512, 640),
+    (64, True, 1, 65, 5, 512, 520), (128, False, 9, 29, 1, 16, 400)])
 def test_attention_key_groups(vm, orc, Dh, causal, B, H, Hk, L, Lk):
     """attention! at D = 128 and 64 on both sides of the key-group rule (few query
-    blocks: two groups of waves split the keys; many: one): one key tile, an odd
-    count, more queries than keys (causal rows before the first key give 0),
-    ragged lengths with a sequence of no keys."""
+    blocks and keys enough, or a causal walk that outlasts them: two groups of
+    waves split the keys; else one): one key tile, an odd count, the last key
+    count of one group, more queries than keys (causal rows before the first key
+    give 0), ragged lengths with a sequence of no keys."""
     banner(f"attention_ key groups D={Dh} causal={causal} B={B} H={H}/{Hk} L={L} Lk={Lk}")
     q_bits = normal_bf16((B, H, L, Dh), 428)
     k_bits = normal_bf16((B, Hk, Lk, Dh), 429)

@@ -77,7 +77,7 @@ __device__ __forceinline__ int swz_pf(int r) { return ((r & 3) << 2) | ((r >> 2)
 // of its own; the groups' sums are merged through LDS at the end. At D = 256 one
 // group's ring and registers fill the CU (NG = 1). At D = 128 and 64 a CU holds two
 // and three workgroups of one group, or one of two: either way two waves or more
-// on a SIMD, one's softmax under the other's MFMAs. launch_prefill chooses.
+// on a SIMD, one's softmax under the other's MFMAs. two_key_groups chooses.
 // waves per SIMD to compile for
 template <int D, int NG> constexpr int pf_waves() { return D == 256 ? 1 : NG == 2 || D == 128 ? 2 : 3; }
 
@@ -441,22 +441,39 @@ void prefill_kernel(PrefillArgs a) {
   }
 }
 
-hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st) {
-  const int64_t nwg = (int64_t)a.n_qt * a.H * a.B;
-  if (nwg == 0) return hipSuccess;
-  // Two key groups halve the walk over the keys that a query block makes alone; one
-  // leaves the CU to two independent blocks (three at D = 64), whose waves do not
-  // meet at one barrier. Causal blocks differ in length, so the longest walk
-  // decides while blocks are few: two groups against one, T = 4096, 16 heads (512
-  // blocks) 104 : 122 us at D = 128, 60 : 77 at D = 64; T = 2048 (256 blocks) 41 :
-  // 54; 576 blocks 86 : 86; 768 blocks 83 : 70. Without the mask all are as long,
-  // and one group wins once every CU has two blocks: 512 blocks 158 : 153. Before
-  // (one group, one block per CU at a time): 131 us causal, 231 without the mask.
+// Two key groups (D = 128 and 64) halve the walk over the keys that a query block
+// makes alone, and pay for it with a merge, a second wave per SIMD to start and
+// a CU to themselves; one group leaves the CU to two independent blocks (three at
+// D = 64), whose waves do not meet at one barrier. One group everywhere is faster
+// than the kernel before either (one block per CU); two groups measured against
+// one (us, D = 64 / D = 128, 256 CUs):
+//   - no more blocks than CUs: two, from 8 key tiles (D = 64) and 11 (D = 128) on.
+//     64 blocks: 64 keys 6.1 : 5.4 / 8.3 : 6.5, 256 9.1 : 9.0 / 12.8 : 11.9, 384 10.6 :
+//     11.3 / 14.9 : 15.1; 256 blocks: 2048 30 : 41 / 42 : 55.
+//   - more blocks than CUs: their walks share the CUs either way, so two groups pay
+//     only where the longest walk outlasts the CU's share of all of them: causal,
+//     queries not few against the keys, keys not few against the blocks. L = Lk:
+//     320 blocks of 512 14.6 : 14.6 / 22.9 : 21.4, of 1024 18 : 23 / 27 : 33; 512 of 512
+//     18 : 15 / 29 : 23, of 4096 60 : 78 / 91 : 112; 576 of 2048 46 : 44 / 69 : 63, of 3072
+//     59 : 61 / 87 : 89. L = Lk / 2 = 2048: 288 blocks 67 : 78 / 102 : 112, 448 83 : 80 / 126 :
+//     118. L = 256, 320 blocks of 2048 54 : 49 / 83 : 69. Unmasked: 384 of 2048 56 : 52 /
+//     81 : 73. Blocks times mean walk over CUs, plus the walks' spread still to come,
+//     against 1.5 longest walks separates these.
+static bool two_key_groups(const PrefillArgs& a, int64_t nwg) {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     cus = 256;
-  const bool two = a.causal ? 4 * nwg <= 9 * cus : nwg < 2 * cus;
+  const int64_t Lk = a.Lk, L = min(a.L, a.Lk);
+  if (nwg <= cus) return Lk > (a.D == 64 ? 256 : 352);
+  return a.causal && 4 * nwg <= (Lk >= 3072 ? 9 : 8) * cus && Lk * cus >= 512 * nwg &&
+         nwg * (2 * Lk - L) < cus * (Lk + 2 * L);
+}
+
+hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st) {
+  const int64_t nwg = (int64_t)a.n_qt * a.H * a.B;
+  if (nwg == 0) return hipSuccess;
+  const bool two = (a.D == 128 || a.D == 64) && two_key_groups(a, nwg);
   const dim3 grid((unsigned)nwg);
 #define VM_PREFILL(causal, d, ng) \
   hipLaunchKernelGGL((prefill_kernel<causal, d, ng>), grid, dim3(256 * ng), 0, st, a)
