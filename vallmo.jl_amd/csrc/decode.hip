@@ -363,10 +363,9 @@ __device__ __forceinline__ bool stream_partition(const DecodeArgs& a, int w, int
     }
     if (lane == 0) a.geom[0] = chunk;
   }
-  const int64_t first = (int64_t)w * chunk;  // past W for the last of many waves
-  if (first >= W) return false;
-  gw0 = uniform((int)first);
-  gw1 = uniform((int)min(first + chunk, (int64_t)W));
+  if ((int64_t)w * chunk >= W) return false;  // past 2^31 for the last of very many waves
+  gw0 = w * chunk;
+  gw1 = gw0 + min(chunk, W - gw0);
 
   // ---- locate the segment holding gw0: first b whose prefix (token-heads) passes it
   b = 0;
