@@ -266,6 +266,36 @@ def test_decode_attention_stream_head_dims(vm, orc, Dh, H, Hk, n_splits):
     assert not got[1].any()  # no key: O = 0
 
 
+@pytest.mark.parametrize("Dh,H,Hk,B,n_splits", [(128, 12, 3, 70, 0), (64, 8, 2, 70, 0),
+                                                (128, 8, 1, 5, 1), (64, 6, 2, 9, 3)])
+def test_decode_attention_stream_short_segments(vm, orc, Dh, H, Hk, B, n_splits):
+    """Many segments shorter than a ring slot or a token past one (the stream counts
+    whole slots, 32 or 64 tokens): neighbours' keys, which the padding of a segment
+    reads, must not reach it, and lengths below 0 or past the cache are clamped.
+    More sequences than lanes; NaN in every row past a sequence's length."""
+    banner(f"decode_attention_ short segments D={Dh} H={H}/{Hk} B={B} n_splits={n_splits}")
+    ctx = 131
+    pick = np.array([1, 2, 31, 32, 33, 63, 64, 65, 96, 0, -3, ctx, ctx + 40, 127], np.int32)
+    lens = pick[np.arange(B) * 5 % len(pick)]
+    kl = np.clip(lens, 0, ctx)
+    q_bits = normal_bf16((B, H, Dh), 460)
+    k_bits = normal_bf16((B, Hk, ctx, Dh), 461)
+    v_bits = normal_bf16((B, Hk, ctx, Dh), 462)
+    past = np.arange(ctx)[None, None, :, None] >= kl[:, None, None, None]
+    K, V = (torch.where(torch.from_numpy(past).cuda(), float("nan"), to_dev(b)) for b in (k_bits, v_bits))
+    O = torch.empty((B, H, Dh), dtype=torch.bfloat16, device="cuda")
+    vm.decode_attention_({"O": O}, to_dev(q_bits), K, V, lengths=i32(lens), n_splits=n_splits)
+    torch.cuda.synchronize()
+    vf = bf16_to_f32(v_bits)
+    ref = orc.attention(bf16_to_f32(q_bits)[:, :, None], bf16_to_f32(k_bits), vf, causal=False,
+                        k_lengths=kl)[:, :, 0]
+    got = dev_f32(O)
+    over = (np.abs(got - ref) / _decode_bound(ref, vf)).max()
+    print(f"{over:.3f} of the bound")
+    assert over <= 1.0
+    assert not got[kl == 0].any()
+
+
 def test_decode_attention_stream_limits(vm, orc):
     """At D = 128: an infinity in V reaches its own column of its own sequence
     only; keys that all score -inf give O = 0; a workspace sized for the generic

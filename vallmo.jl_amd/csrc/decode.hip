@@ -74,6 +74,20 @@ __device__ __forceinline__ f32x4 mfma16k16(const uint2& a, const uint2& b, f32x4
                                                   __builtin_bit_cast(s16x4v, b), c, 0, 0, 0);
 }
 
+// a (sequence, kv head) segment's extent in the stream: its length in whole PAD
+// tokens. PAD = 1 at D = 256. At D = 128 and 64 PAD is a ring slot's tokens, so
+// that a wave's chunk counts slots, which all cost the same, and not token-heads:
+// many short segments then spread over the waves, down to one slot each. Chunks of
+// 64 token-heads or more gave 64 one-token segments to one wave. 32 sequences, 4 KV
+// heads of 128, one token: 151 -> 9.1 us (generic split kernel 10.8 to 13.2 by the
+// cache's size), 16 tokens 16.0 -> 9.0; with 64 token-heads a wave at least, 12.2.
+// (With PAD > 1 the cache has fewer than 2^31 rows.)
+template <int PAD>
+__device__ __forceinline__ int stream_extent(int raw, int64_t ctx) {
+  if (PAD == 1) return raw < 0 ? 0 : (raw > ctx ? (int)ctx : raw);
+  return (max(min(raw, (int)ctx), 0) + PAD - 1) & -PAD;
+}
+
 // chunk of the stream partition (token-heads per wave), identical in both kernels
 // (a multiple of the tokens of one ring slot)
 template <int TOK>
@@ -81,12 +95,6 @@ __device__ __forceinline__ int stream_chunk(int W, int NW, int min_chunk) {
   int c = (W + NW - 1) / NW;
   c = max(c, min_chunk);
   return (c + TOK - 1) / TOK * TOK;
-}
-
-__device__ __forceinline__ int clamp_len(const int32_t* lengths, int b, int64_t ctx) {
-  int64_t l = lengths[b];
-  l = l < 0 ? 0 : (l > ctx ? ctx : l);
-  return (int)l;
 }
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -259,15 +267,20 @@ __device__ __forceinline__ void append_row(StepBuf& s, const DecodeArgs& a, int 
   }
 }
 
-// One (b, hk) segment of a wave's chunk: its tokens [lo, hi) (a suffix of the
-// previous segment's end); hm = hi - 1 when the wave appends the new token.
+// One (b, hk) segment of a wave's chunk: its positions [lo, hi) in the stream (a
+// suffix of the previous segment's end); its tokens from the cache are [lo, hm):
+// hm is hi less the segment's padding, or hi - 1 when the wave appends the new
+// token. (With padding, lo is a multiple of PAD below the extent, so below the
+// length too: no part is empty.)
 struct Seg {
-  int b, hk, len, seg_b_start;
+  int b, hk, seg_b_start;
+  int len;  // the segment's extent (stream_extent)
   int raw;  // lengths[b] as passed (may exceed ctx)
   int lo, hi, hm;
   bool append;
 };
 
+template <int PAD>
 __device__ __forceinline__ void seg_bounds(Seg& s, int pos, int gw1, const DecodeArgs& a,
                                            bool fused) {
   const int seg_start = s.seg_b_start + s.hk * s.len;
@@ -277,6 +290,7 @@ __device__ __forceinline__ void seg_bounds(Seg& s, int pos, int gw1, const Decod
   // from the raw projection (in contract only: lengths[b] <= ctx)
   s.append = fused && a.k_new != nullptr && s.hi == s.len && s.raw <= a.ctx;
   s.hm = s.append ? s.hi - 1 : s.hi;
+  if (PAD > 1) s.hm = min(s.hi, min(s.raw, (int)a.ctx));
 }
 
 // lengths[b] for a wave-uniform b: from the register copy of the first 64
@@ -287,6 +301,7 @@ __device__ __forceinline__ int seq_len_raw(const int32_t* lengths, int raw_l, in
 }
 
 // Move to the next non-empty segment of the chunk; false when the chunk ends.
+template <int PAD>
 __device__ __forceinline__ bool seg_next(Seg& s, int gw1, const DecodeArgs& a, bool fused,
                                          int raw_l) {
   const int pos = s.seg_b_start + s.hk * s.len + s.hi;
@@ -297,10 +312,10 @@ __device__ __forceinline__ bool seg_next(Seg& s, int gw1, const DecodeArgs& a, b
     do {
       ++s.b;
       s.raw = seq_len_raw(a.lengths, raw_l, s.b);
-      s.len = s.raw < 0 ? 0 : (s.raw > a.ctx ? (int)a.ctx : s.raw);
+      s.len = stream_extent<PAD>(s.raw, a.ctx);
     } while (s.len == 0 && s.b + 1 < a.B);
   }
-  seg_bounds(s, pos, gw1, a, fused);
+  seg_bounds<PAD>(s, pos, gw1, a, fused);
   return true;
 }
 
@@ -312,7 +327,7 @@ struct Issuer {
   __device__ __forceinline__ bool next(uint16_t* slot, const DecodeArgs& a, int gw1, int64_t last,
                                        int lane, bool fused, int raw_l) {
     while (t >= s.hm) {
-      if (!seg_next(s, gw1, a, fused, raw_l)) return false;
+      if (!seg_next<D == HEAD_DIM ? 1 : STEP_ELEMS / D>(s, gw1, a, fused, raw_l)) return false;
       t = s.lo;
     }
     const int64_t base = (int64_t)s.b * a.c_sb + (int64_t)s.hk * a.c_sh;
@@ -325,16 +340,17 @@ struct Issuer {
 // The stream partition, from the lengths on the device: this wave's chunk
 // [gw0, gw1) of the token-heads and the segment (b, hk) holding gw0; false when
 // the wave has none. raw_l: lengths[lane] (0 past B). Wave 0 writes the
-// snapshot that the merge reads.
-template <int TOK>
+// snapshot that the merge reads. Lengths here are extents (stream_extent).
+template <int TOK, int PAD>
 __device__ __forceinline__ bool stream_partition(const DecodeArgs& a, int w, int lane, int raw_l,
                                                  int& b, int& hk, int& len, int& raw,
                                                  int& seg_b_start, int& gw0, int& gw1) {
   const int Hk = a.Hk;
-  const int len_l = raw_l < 0 ? 0 : (raw_l > a.ctx ? (int)a.ctx : raw_l);
+  const int len_l = stream_extent<PAD>(raw_l, a.ctx);
   // clamped lengths of sequences b0 + lane, b0 a multiple of 64
   auto lens_at = [&](int b0) __attribute__((always_inline)) {
-    return b0 == 0 ? len_l : ((b0 + lane < a.B) ? clamp_len(a.lengths, b0 + lane, a.ctx) : 0);
+    return b0 == 0 ? len_l
+                   : ((b0 + lane < a.B) ? stream_extent<PAD>(a.lengths[b0 + lane], a.ctx) : 0);
   };
   // ---- stream partition: total work and this wave's chunk [gw0, gw1).
   // incl_at(b0): inclusive prefix of len * Hk (token-heads) over sequences
@@ -388,7 +404,7 @@ __device__ __forceinline__ bool stream_partition(const DecodeArgs& a, int w, int
   b = uniform(b);
   seg_b_start = uniform(seg_b_start);
   raw = seq_len_raw(a.lengths, raw_l, b);
-  len = raw < 0 ? 0 : (raw > a.ctx ? (int)a.ctx : raw);
+  len = stream_extent<PAD>(raw, a.ctx);
   hk = (gw0 - seg_b_start) / len;
   return true;
 }
@@ -413,7 +429,7 @@ void decode_stream_kernel(DecodeArgs a) {
     for (int kk = 0; kk < 8; ++kk) qwv[kk] = load16(a.qw + 32 * kk + 8 * g);
   }
   int b, hk, len, raw, seg_b_start, gw0, gw1;
-  if (!stream_partition<DSTEP>(a, w, lane, raw_l, b, hk, len, raw, seg_b_start, gw0, gw1)) return;
+  if (!stream_partition<DSTEP, 1>(a, w, lane, raw_l, b, hk, len, raw, seg_b_start, gw0, gw1)) return;
 
   // 0/1 selection operands for the V transpose: Sel_h[8g+j][n] = (8g+j == n+16h)
   uint4 sel[2];
@@ -452,7 +468,7 @@ void decode_stream_kernel(DecodeArgs a) {
 
   Seg cs;  // compute side
   cs.b = b; cs.hk = hk; cs.len = len; cs.seg_b_start = seg_b_start; cs.raw = raw;
-  seg_bounds(cs, gw0, gw1, a, FUSED);
+  seg_bounds<1>(cs, gw0, gw1, a, FUSED);
   Issuer<HEAD_DIM> is;  // issue side, two steps ahead
   is.s = cs;
   is.t = cs.lo;
@@ -588,7 +604,7 @@ void decode_stream_kernel(DecodeArgs a) {
         a.part_ml[2 * (slot * G + n) + 1] = l_tot;
       }
     }
-    if (!seg_next(cs, gw1, a, FUSED, raw_l)) break;
+    if (!seg_next<1>(cs, gw1, a, FUSED, raw_l)) break;
     ct = cs.lo;
   }
   wait_vmcnt<0>();  // no LDS load may land after the wave is gone
@@ -625,7 +641,7 @@ void decode_stream_hd_kernel(DecodeArgs a) {
   const int G = a.G;
   const int raw_l = lane < a.B ? a.lengths[lane] : 0;
   int b, hk, len, raw, seg_b_start, gw0, gw1;
-  if (!stream_partition<TOK>(a, w, lane, raw_l, b, hk, len, raw, seg_b_start, gw0, gw1)) return;
+  if (!stream_partition<TOK, TOK>(a, w, lane, raw_l, b, hk, len, raw, seg_b_start, gw0, gw1)) return;
 
   // one __shared__ object per ring slot: reads of one slot do not alias the
   // loads still landing in the other
@@ -637,7 +653,7 @@ void decode_stream_hd_kernel(DecodeArgs a) {
 
   Seg cs;  // compute side
   cs.b = b; cs.hk = hk; cs.len = len; cs.seg_b_start = seg_b_start; cs.raw = raw;
-  seg_bounds(cs, gw0, gw1, a, false);
+  seg_bounds<TOK>(cs, gw0, gw1, a, false);
   Issuer<D> is;  // issue side, two slots ahead
   is.s = cs;
   is.t = cs.lo;
@@ -689,17 +705,17 @@ void decode_stream_hd_kernel(DecodeArgs a) {
       // the slot is free once its reads have returned; refill it
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       if (is.next(slot, a, gw1, last, lane, false, raw_l)) ++inflight;
-      const bool tail = ct + TOK > cs.hi;
+      const bool tail = ct + TOK > cs.hm;
       if (tail) {
         // rows past the range may hold anything: p = 0 must meet finite v
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
           uint32_t m01 = 0, m23 = 0;
           const int t0 = ct + 16 * i + 4 * g;
-          if (t0 < cs.hi) m01 |= 0xffffu;
-          if (t0 + 1 < cs.hi) m01 |= 0xffff0000u;
-          if (t0 + 2 < cs.hi) m23 |= 0xffffu;
-          if (t0 + 3 < cs.hi) m23 |= 0xffff0000u;
+          if (t0 < cs.hm) m01 |= 0xffffu;
+          if (t0 + 1 < cs.hm) m01 |= 0xffff0000u;
+          if (t0 + 2 < cs.hm) m23 |= 0xffffu;
+          if (t0 + 3 < cs.hm) m23 |= 0xffff0000u;
 #pragma unroll
           for (int dt = 0; dt < ND; ++dt) {
             v[i][dt].x &= m01;
@@ -720,7 +736,7 @@ void decode_stream_hd_kernel(DecodeArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           sc[i][j] *= SL2;
-          if (tail && ct + 16 * i + 4 * g + j >= cs.hi) sc[i][j] = -INFINITY;
+          if (tail && ct + 16 * i + 4 * g + j >= cs.hm) sc[i][j] = -INFINITY;
           mx = fmaxf(mx, sc[i][j]);
         }
       // running max in log2 units, rescaled lazily: only when it grows by more
@@ -796,7 +812,7 @@ void decode_stream_hd_kernel(DecodeArgs a) {
         a.part_ml[2 * (slot * G + n) + 1] = l_tot;
       }
     }
-    if (!seg_next(cs, gw1, a, false, raw_l)) break;
+    if (!seg_next<TOK>(cs, gw1, a, false, raw_l)) break;
     ct = cs.lo;
   }
   wait_vmcnt<0>();  // no LDS load may land after the wave is gone

@@ -92,7 +92,7 @@ struct DecodeArgs {
   float* part_ml;       // [slots][G][2]  (shift m in log2 units, sum l)
   int B, Hk, G;
   int NW;               // waves of the stream partition (multiple of 4)
-  int min_chunk;        // smallest per-wave chunk (token-heads, multiple of 16)
+  int min_chunk;        // smallest per-wave chunk (token-heads; rounded up to a ring slot)
   int32_t* geom;        // partition snapshot for the merge: [chunk | len_b (B) | start_b (B)]
 };
 

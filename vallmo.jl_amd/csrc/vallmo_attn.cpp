@@ -347,17 +347,22 @@ static size_t generic_decode_scratch_bytes(int B, int H, int Hk, int Dv, int64_t
 }
 
 // The problems of the stream kernels: D = 256, 128 and 64, groups up to 8 and
-// fewer than 2^31 token-heads. At D = 128 and 64, which the generic kernel
+// fewer than 2^31 token-heads, at D = 128 and 64 counted in whole ring slots of
+// 4096 / D tokens. At D = 128 and 64, which the generic kernel
 // serves as well, also its grid limits, and at most 2^24 waves asked for through
 // n_splits: a wave past the last token-head does nothing but its launch and its
-// share of the workspace, and counts past 2^31 would wrap.
+// share of the workspace, and counts past 2^31 would wrap. At D = 64 a cache of one
+// 32-key tile and groups up to 4 stay with the generic kernel, a single launch of
+// one tile there: 8.4 to 9.0 us against 9.1 to 9.8 (1 to 4 sequences); at D = 128 9.8 to
+// 10.6 against 9.6 to 10.7, and two tiles 11.1 against 9.4.
 static bool stream_decode_shape(int B, int H, int Hk, int D, int64_t ctx, int n_splits) {
-  if ((D != vm::HEAD_DIM_ABI && D != 128 && D != 64) || H / Hk > 8 ||
-      (int64_t)B * ctx * Hk >= ((int64_t)1 << 31))
-    return false;
-  const int64_t segs = (int64_t)B * Hk;
+  if ((D != vm::HEAD_DIM_ABI && D != 128 && D != 64) || H / Hk > 8) return false;
+  const int64_t segs = (int64_t)B * Hk, limit = (int64_t)1 << 31;
+  const int pad = D == vm::HEAD_DIM_ABI ? 1 : 4096 / D;
+  if (segs > 0 && (ctx >= limit || segs * ((ctx + pad - 1) / pad * pad) >= limit)) return false;
   return D == vm::HEAD_DIM_ABI ||
-         (segs <= 65535 && n_splits <= 65535 && n_splits * segs <= ((int64_t)1 << 24));
+         (segs <= 65535 && n_splits <= 65535 && n_splits * segs <= ((int64_t)1 << 24) &&
+          !(D == 64 && H / Hk <= 4 && ctx <= 32));
 }
 
 size_t vm_decode_scratch_bytes(int B, int H, int Hk, int D, int64_t ctx, int n_splits) {
@@ -455,6 +460,10 @@ int vm_decode_attention(vm_bf16* o, int64_t o_sh, int64_t o_sb, const vm_bf16* q
   vm::CombineArgs c{};
   TRY(decode_common(a, c, scratch, scratch_bytes, B, H, Hk, Dk, ctx, n_splits));
   if (B == 0) return VM_OK;
+  // down to one ring slot a wave (see stream_extent) while each SIMD has one wave; with
+  // more waves than that (n_splits) a part's start and merge outweigh a slot: 32
+  // sequences of 512, n_splits = 64: 26.7 us against 21.7 with 64 token-heads at least
+  if (Dk != vm::HEAD_DIM_ABI && a.NW <= vm::decode_stream_waves(B, Hk, 0)) a.min_chunk = 1;
   a.q = q; a.q_sh = q_sh; a.q_sb = q_sb;
   // read-only here: the unfused operator appends nothing (k_new stays NULL)
   a.kc = const_cast<uint16_t*>(kc); a.vc = const_cast<uint16_t*>(vc);
