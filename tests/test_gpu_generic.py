@@ -266,6 +266,38 @@ def test_decode_attention_stream_head_dims(vm, orc, Dh, H, Hk, n_splits):
     assert not got[1].any()  # no key: O = 0
 
 
+@pytest.mark.parametrize("Dh,H,Hk", [(128, 8, 2), (64, 8, 2), (128, 6, 1), (64, 8, 1), (32, 8, 2)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_decode_attention_nan_scores(vm, Dh, H, Hk, bad):
+    """A NaN or an infinity in an attended key (scores NaN, or +inf for some heads,
+    whose softmax is NaN) gives NaN for the query heads that attend it, at the head
+    dims of the stream kernel as of the generic one (D = 32 here); the other heads
+    and sequences keep their bits."""
+    banner(f"decode_attention_ nan scores D={Dh} H={H}/{Hk} {bad}")
+    B, ctx, G = 3, 200, H // Hk
+    q = to_dev(normal_bf16((B, H, Dh), 470))
+    k = to_dev(normal_bf16((B, Hk, ctx, Dh), 471))
+    v = to_dev(normal_bf16((B, Hk, ctx, Dh), 472))
+    lens = i32(np.array([200, 77, 150], np.int32))
+
+    def run():
+        O = torch.empty((B, H, Dh), dtype=torch.bfloat16, device="cuda")
+        vm.decode_attention_({"O": O}, q, k, v, lengths=lens)
+        torch.cuda.synchronize()
+        return dev_f32(O)
+
+    base = run()
+    q[1, (Hk - 1) * G, 3] = q[1, (Hk - 1) * G, 3].abs() + 0.5
+    base_q = run()[1, (Hk - 1) * G]
+    k[1, Hk - 1, 40, 3] = bad
+    got = run()
+    assert np.isfinite(base).all() and np.isfinite(base_q).all()
+    assert np.isnan(got[1, (Hk - 1) * G]).all()   # its score: NaN, or +inf
+    heads = np.ones((B, H), bool)
+    heads[1, (Hk - 1) * G:] = False
+    assert np.array_equal(got[heads], base[heads])
+
+
 @pytest.mark.parametrize("Dh,H,Hk,B,n_splits", [(128, 12, 3, 70, 0), (64, 8, 2, 70, 0),
                                                 (128, 8, 1, 5, 1), (64, 6, 2, 9, 3)])
 def test_decode_attention_stream_short_segments(vm, orc, Dh, H, Hk, B, n_splits):

@@ -906,7 +906,9 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgs a) {
         Of += so[i * DW + t] * c;
       }
     }
-    float out = Lf > 0.f ? Of / Lf : 0.f;  // no valid key: o = 0 (attention_decode.jl:126-128)
+    // no valid key: o = 0 (attention_decode.jl:126-128). At D = 128 and 64 a sum that is
+    // NaN (a NaN in an attended key) gives NaN, as the generic kernel does
+    float out = (D == HEAD_DIM ? Lf > 0.f : Lf != 0.f) ? Of / Lf : 0.f;
     const int dd = dr * DW + t;
     if (a.gate) out *= sigmoidf(gate);
     a.out[(int64_t)b * a.o_sb + (int64_t)h * a.o_sh + dd] = f2bf(out);
