@@ -228,9 +228,9 @@ def test_attention_key_groups(vm, orc, Dh, causal, B, H, Hk, L, Lk):
 
 def _decode_bound(ref, v):
     """The bf16 rounding of the result (half an ulp: 2^-8 of the result's power of
-    two) plus what the fp32 products leave: p is held to 2^-17 of itself (its two
-    bf16 parts), sums and exp2 to a few 2^-23 of the convex combination's largest
-    |v|."""
+    two) plus a slack for sums, scores and exp2 in fp32: 2^-15 of the largest |v| of
+    the convex combination, of which they take a few 2^-23 per unit of the scores
+    (test_decode_attention_keeps_p measures that part)."""
     binade = np.exp2(np.floor(np.log2(np.maximum(np.abs(ref), 1e-30))))
     return 2.0 ** -8 * binade * 1.001 + 2.0 ** -15 * np.abs(v).max()
 
@@ -264,6 +264,34 @@ def test_decode_attention_stream_head_dims(vm, orc, Dh, H, Hk, n_splits):
     print(f"max {np.abs(got - ref).max():.3e}, {over:.3f} of the bound")
     assert over <= 1.0
     assert not got[1].any()  # no key: O = 0
+
+
+@pytest.mark.parametrize("Dh,H,Hk", [(128, 16, 4), (64, 16, 4), (128, 24, 4), (64, 16, 2), (32, 16, 4)])
+def test_decode_attention_keeps_p(vm, Dh, H, Hk):
+    """The probabilities keep fp32's 24 bits through the bf16 products of the stream
+    kernel (three parts of 8). The output's bf16 rounding hides them but for one
+    trace: an error e of a result x (both relative to x's power of two, of spacing
+    2^-7) leaves the bf16 nearest to the float64 result with probability about 2^7
+    e. fp32 scores up to 6, exp2 and sums make e a few 2^-21 (the generic kernel, D
+    = 32, as well): 0.02%; probabilities of 16 bits make it up to 2^-16: 0.2% and more."""
+    banner(f"decode_attention_ keeps p D={Dh} H={H}/{Hk}")
+    B, ctx, G = 24, 48, H // Hk
+    lens = np.array([3 + 2 * (b % 20) for b in range(B)], np.int32)
+    q_bits = normal_bf16((B, H, Dh), 480)
+    k_bits = normal_bf16((B, Hk, ctx, Dh), 481)
+    v_bits = normal_bf16((B, Hk, ctx, Dh), 482)
+    O = torch.empty((B, H, Dh), dtype=torch.bfloat16, device="cuda")
+    vm.decode_attention_({"O": O}, to_dev(q_bits), to_dev(k_bits), to_dev(v_bits), lengths=i32(lens))
+    torch.cuda.synchronize()
+    q, k, v = (bf16_to_f32(x).astype(np.float64) for x in (q_bits, k_bits, v_bits))
+    s = np.einsum("bhgd,bhkd->bhgk", q.reshape(B, Hk, G, Dh), k) * Dh ** -0.5
+    s[np.broadcast_to(np.arange(ctx) >= lens[:, None, None, None], s.shape)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = (np.einsum("bhgk,bhkd->bhgd", p, v) / p.sum(-1, keepdims=True)).reshape(B, H, Dh)
+    near = torch.from_numpy(ref).to(torch.bfloat16)  # one rounding, to nearest
+    off = float((O.cpu() != near).float().mean())
+    print(f"not the nearest bf16: {100 * off:.3f}% of {near.numel()}")
+    assert off <= 1e-3
 
 
 @pytest.mark.parametrize("Dh,H,Hk", [(128, 8, 2), (64, 8, 2), (128, 6, 1), (64, 8, 1), (32, 8, 2)])

@@ -613,13 +613,17 @@ void decode_stream_kernel(DecodeArgs a) {
 // decode_attention! at D = 128 and 64 (q already normalised): the same stream
 // partition, ring and partials, with 4096 / D tokens per ring slot, so that a
 // slot is 8 KB of K and 8 KB of V at every D and a wave keeps 32 KB in flight.
-// HBM-bound: per 32 tokens 2 D/32 + D/16 MFMAs against 128 D bytes.
-//   - P stays at fp32 precision through the bf16 MFMA: a group has at most 8
-//     heads and the MFMA 16 columns, so columns n and n + 8 both score head n;
-//     column n multiplies hi = p truncated to bf16, column n + 8 the rest
-//     p - hi (p - hi - lo <= 2^-17 p), and the two accumulators are added once
-//     per segment. That costs no MFMA. hi is truncated and lo kept positive, so
-//     an infinite v times p stays infinite.
+// HBM-bound: per 32 tokens 2 D/32 + D/16 (QUAD; else 2 D/16) MFMAs against 128 D
+// bytes.
+//   - P keeps its 24 bits through the bf16 MFMA, as hi + mid + lo of 8 bits each, in
+//     the columns that a group leaves free of the MFMA's 16: up to 4 heads (QUAD)
+//     columns n, n + 4, n + 8 and n + 12 all score head n and hold hi, mid, lo and
+//     nothing; up to 8, columns n and n + 8 hold hi and mid, then lo and nothing
+//     in a second product. The columns' accumulators are added once per segment.
+//     The parts are truncated, and none is below 2^-30 p (P_TINY), nothing among
+//     them, so that an infinite v times p stays infinite while p = 0 stays 0.
+//     (hi and a rounded rest alone leave 2^-16 of p: the result was off the nearest
+//     bf16 in 0.3% of its elements; in 0.03% with all bits, as with fp32 products.)
 //   - V^T operands are LDS transpose reads: no value of one key or column
 //     touches another's (a 0/1 selection MFMA would multiply an infinity by 0).
 //   - q is not scaled in bf16 (1/sqrt(128) is no power of two): the scale is in
@@ -627,7 +631,23 @@ void decode_stream_kernel(DecodeArgs a) {
 // Measured at D = 128, B = 32, 16/4 heads, lengths U{1024..32768} (900 MB): 143.5
 // us with the merge, 6.3 TB/s; the generic split kernel, bound by its fp32 VALU
 // products, took 575 us (1.6 TB/s).
-template <int D>
+constexpr float P_TINY = 0x1p-30f;
+constexpr uint32_t HIGH = 0xffff0000u;
+// x less the float of its bits in mask (exact)
+__device__ __forceinline__ float cut(float x, uint32_t mask) {
+  return x - __uint_as_float(__float_as_uint(x) & mask);
+}
+// the value N lanes on within the row of 16 lanes
+template <int N>
+__device__ __forceinline__ float row_ror(float x) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + N, 0xf, 0xf, true));
+}
+// the upper halves of lo and hi (bf16, truncated), packed
+__device__ __forceinline__ uint32_t high2(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
+template <int D, bool QUAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void decode_stream_hd_kernel(DecodeArgs a) {
   constexpr int TOK = STEP_ELEMS / D;  // tokens per ring slot
@@ -650,6 +670,10 @@ void decode_stream_hd_kernel(DecodeArgs a) {
   uint16_t* const r0 = ring0[threadIdx.x >> 6];
   uint16_t* const r1 = ring1[threadIdx.x >> 6];
   const int64_t last = a.ctx - 1;
+  // QUAD: the bits taken off p, then off the rest, for this column's part of P: none
+  // for hi, the upper half for mid, twice for lo, and all of the rest for nothing
+  const uint32_t cut1 = n < 4 ? 0u : HIGH;
+  const uint32_t cut2 = n < 8 ? 0u : n < 12 ? HIGH : ~0u;
 
   Seg cs;  // compute side
   cs.b = b; cs.hk = hk; cs.len = len; cs.seg_b_start = seg_b_start; cs.raw = raw;
@@ -661,10 +685,10 @@ void decode_stream_hd_kernel(DecodeArgs a) {
   bool primed = false;
 
   while (true) {
-    // Q operand for (b, hk): lane (n, g) holds q[head n % 8][32kk + 8g + j]
+    // Q operand for (b, hk): lane (n, g) holds q[head n % 8 (QUAD: 4)][32kk + 8g + j]
     uint4 qop[NK];
     {
-      const int hn = n & 7;
+      const int hn = n & (QUAD ? 3 : 7);
       const uint16_t* qp = a.q + (int64_t)cs.b * a.q_sb +
                            (int64_t)(cs.hk * G + (hn < G ? hn : 0)) * a.q_sh + 8 * g;
 #pragma unroll
@@ -754,31 +778,39 @@ void decode_stream_hd_kernel(DecodeArgs a) {
         m_run = m_use;
       }
       const float m_eff = m_run == -INFINITY ? 0.f : m_run;  // every key so far scored -inf
-      uint2 pop[NB];
+      uint2 pop[NB], pop2[NB];  // the parts of P by column; pop2: the second product's
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
-        uint32_t h[4];
-        float lo[4];
+        float x[4], y[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float p = fast_exp2(sc[i][j] - m_eff);
           l_part += p;
-          h[j] = __float_as_uint(p) & 0xffff0000u;
-          lo[j] = p > 0.f ? fmaxf(p - __uint_as_float(h[j]), 0x1p-100f) : p;
+          const float tiny = p * P_TINY;
+          if (QUAD) {
+            x[j] = fmaxf(cut(cut(p, cut1), cut2), tiny);
+          } else {
+            const float rest = cut(p, HIGH);
+            x[j] = n < 8 ? p : fmaxf(rest, tiny);
+            y[j] = n < 8 ? fmaxf(cut(rest, HIGH), tiny) : tiny;
+          }
         }
-        const uint2 hi2 = make_uint2((h[0] >> 16) | h[1], (h[2] >> 16) | h[3]);
-        const uint2 lo2 = make_uint2(pack2(lo[0], lo[1]), pack2(lo[2], lo[3]));
-        pop[i] = n < 8 ? hi2 : lo2;
+        pop[i] = make_uint2(high2(x[0], x[1]), high2(x[2], x[3]));
+        if (!QUAD) pop2[i] = make_uint2(high2(y[0], y[1]), high2(y[2], y[3]));
       }
       // O^T += V^T P^T over 32 tokens: k index 8g + j is token 4g + j of the first
       // block (j < 4) or of the second
 #pragma unroll
       for (int i = 0; i < NB; i += 2) {
         const uint4 pb = make_uint4(pop[i].x, pop[i].y, pop[i + 1].x, pop[i + 1].y);
+        uint4 pb2;
+        if (!QUAD) pb2 = make_uint4(pop2[i].x, pop2[i].y, pop2[i + 1].x, pop2[i + 1].y);
 #pragma unroll
-        for (int dt = 0; dt < ND; ++dt)
-          acc[dt] = mfma16(make_uint4(v[i][dt].x, v[i][dt].y, v[i + 1][dt].x, v[i + 1][dt].y), pb,
-                           acc[dt]);
+        for (int dt = 0; dt < ND; ++dt) {
+          const uint4 vt = make_uint4(v[i][dt].x, v[i][dt].y, v[i + 1][dt].x, v[i + 1][dt].y);
+          acc[dt] = mfma16(vt, pb, acc[dt]);
+          if (!QUAD) acc[dt] = mfma16(vt, pb2, acc[dt]);
+        }
       }
       ct += TOK;
     };
@@ -794,13 +826,16 @@ void decode_stream_hd_kernel(DecodeArgs a) {
       cslot = 0;
     }
 
-    // partial for (w, segment): slot w + b*Hk + hk; columns n and n + 8 added
+    // partial for (w, segment): slot w + b*Hk + hk; a head's columns added
     const float l_tot = col_sum4(l_part);
     const int64_t slot = (int64_t)w + (int64_t)cs.b * a.Hk + cs.hk;
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[dt][j] += __shfl_xor(acc[dt][j], 8, 64);
+      for (int j = 0; j < 4; ++j) {
+        acc[dt][j] += row_ror<8>(acc[dt][j]);
+        if (QUAD) acc[dt][j] += row_ror<4>(acc[dt][j]);
+      }
     if (n < G) {
       float* dst = a.part_o + (slot * G + n) * D + 4 * g;
 #pragma unroll
@@ -934,10 +969,14 @@ hipError_t launch_decode(const DecodeArgs& a, bool fused_q, int D, hipStream_t s
   dim3 grid(a.NW / 4);
   if (fused_q)
     hipLaunchKernelGGL(decode_stream_kernel<true>, grid, dim3(256), 0, st, a);
+  else if (D == 128 && a.G <= 4)
+    hipLaunchKernelGGL((decode_stream_hd_kernel<128, true>), grid, dim3(256), 0, st, a);
   else if (D == 128)
-    hipLaunchKernelGGL(decode_stream_hd_kernel<128>, grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((decode_stream_hd_kernel<128, false>), grid, dim3(256), 0, st, a);
+  else if (D == 64 && a.G <= 4)
+    hipLaunchKernelGGL((decode_stream_hd_kernel<64, true>), grid, dim3(256), 0, st, a);
   else if (D == 64)
-    hipLaunchKernelGGL(decode_stream_hd_kernel<64>, grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((decode_stream_hd_kernel<64, false>), grid, dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL(decode_stream_kernel<false>, grid, dim3(256), 0, st, a);
   return hipGetLastError();
