@@ -216,10 +216,12 @@ def step_asm():
 
 
 def test_step_kernels_no_async_or_mfma_hazard(step_asm):
-    """The lm head, the split-K GEMV and the stream-K GEMV issue their LDS
-    operand reads from asm too: the same check over every kernel of step.hip."""
+    """The lm head, the split-K GEMV, the stream-K GEMV and the whole-K row kernel
+    issue their LDS operand reads from asm too: the same check over every kernel of
+    step.hip."""
     ks = kernels(step_asm)
-    for want in ("lm_head_split_kernel", "gemv_kernel", "gemv_sk_kernel", "silu_mul_sk_kernel"):
+    for want in ("lm_head_split_kernel", "gemv_kernel", "gemv_sk_kernel", "silu_mul_sk_kernel",
+                 "gemv_rows_kernel"):
         assert any(want in k for k in ks), want
     for name, body in ks.items():
         bad = check(body)

@@ -787,6 +787,18 @@ __device__ __forceinline__ void gr_read(lm_u32x4& o, uint32_t addr) {
   asm volatile("ds_read_b128 %0, %1" : "=v"(o) : "v"(addr));
 }
 
+// the products of k steps ST .. 3, each once its operands are in
+template <int T, int ST>
+__device__ __forceinline__ void gr_mult(lm_u32x4 (&o)[4][T + 1], f32x16 (&acc)[T]) {
+  if constexpr (ST < 4) {
+    lm_take<(3 - ST) * (T + 1), T + 1>(o[ST]);
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      acc[t] = mfma32(__builtin_bit_cast(uint4, o[ST][t]), __builtin_bit_cast(uint4, o[ST][T]), acc[t]);
+    gr_mult<T, ST + 1>(o, acc);
+  }
+}
+
 // wait until at most `left` groups of PER loads, issued after the one about to be
 // multiplied, are still out (left <= NS - 1 <= 3)
 template <int PER, int NS>
@@ -858,23 +870,22 @@ __device__ __forceinline__ void gemv_rows(const GemvRowsArgs& a) {
     else if (nx == 2) gr_wait<NR + 2, NS>(left);
     else gr_wait<NR + 4, NS>(left);
     const uint32_t base = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)slot;
+    // operands from asm (a compiler-visible read would drain every load in
+    // flight), those of the group's four k steps at once, so that a group waits
+    // for one LDS latency and not for four; tile rows past the pieces repeat the
+    // last one, and are unused
+    lm_u32x4 o[4][T + 1];
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
-      // operands from asm (a compiler-visible read would drain every load in
-      // flight); tile rows past the pieces repeat the last one, and are unused
       const uint32_t q = 8 * ((2 * st + h) ^ (j & 7));
-      lm_u32x4 o[T + 1];
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         const int r = min(32 * t + j, 8 * NR - 8 + (j & 7));
-        gr_read(o[t], base + 2u * (64 * r + q));
+        gr_read(o[st][t], base + 2u * (64 * r + q));
       }
-      gr_read(o[T], base + 2u * (512 * NR + 64 * (j & (8 * nx - 1)) + q));
-      lm_take<0, T + 1>(o);
-#pragma unroll
-      for (int t = 0; t < T; ++t)
-        acc[t] = mfma32(__builtin_bit_cast(uint4, o[t]), __builtin_bit_cast(uint4, o[T]), acc[t]);
+      gr_read(o[st][T], base + 2u * (512 * NR + 64 * (j & (8 * nx - 1)) + q));
     }
+    gr_mult<T, 0>(o, acc);
     if (g + NS < n) issue(g + NS, slot);  // every read of the slot is in
     s = s + 1 == NS ? 0 : s + 1;
   }
