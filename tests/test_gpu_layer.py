@@ -195,11 +195,14 @@ def test_linear_narrow_misaligned_view(vm, orc):
 
 
 @pytest.mark.parametrize("M,N,K", [(2560, 1, 64), (2564, 8, 320), (2560, 9, 4096), (4604, 16, 192),
-                                   (10240, 17, 2560), (12352, 32, 2560), (24576, 5, 448)])
+                                   (10240, 17, 2560), (12352, 32, 2560), (24576, 5, 448),
+                                   (2564, 20, 1088), (4096, 32, 4096), (3068, 25, 576),
+                                   (2560, 17, 2368), (5120, 32, 128), (12292, 12, 320)])
 def test_linear_rows(vm, orc, M, N, K):
-    """The kernel that cuts the rows over the CUs (K whole): 1 to 12 row pieces a
-    workgroup, a last workgroup that is not full, the batch at its 8-column
-    edges, runs of no, one and many 64-k groups per wave; y a view at 8-byte
+    """The kernel that cuts the rows over the CUs (K whole): 2 to 12 row pieces a
+    workgroup, the last a half piece or not, a last workgroup that is not full,
+    the batch at its 8-column edges, runs of no, one and many 64-k groups per wave;
+    y a view at 8-byte
     alignment whose neighbours stay, a second call bitwise equal, every element
     within the narrow product's bar."""
     banner(f"linear rows M={M} N={N} K={K}")

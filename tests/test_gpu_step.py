@@ -560,11 +560,13 @@ def test_identity_mixed_model_step(vm):
 
 
 @pytest.mark.parametrize("D_,N,K", [(2560, 32, 4096), (2560, 3, 9216), (2560, 16, 64),
-                                   (2560, 64, 4096), (1024, 25, 1024)])
+                                   (2560, 64, 4096), (1024, 25, 1024), (2816, 17, 1536),
+                                   (3072, 20, 2560), (4096, 32, 4096), (2568, 31, 832),
+                                   (2560, 32, 512), (4096, 24, 2048), (2560, 16, 4096)])
 def test_linear_add_rms_norm_is_the_two_calls(vm, D_, N, K):
     """linear! + fused_add_rms_norm! in one call (the split GEMV's slices summed
-    by the norm; one slice; the GEMM library's path at N = 64) is bit-identical
-    to the two calls, residual updated in place."""
+    by the norm, K = 9216 and 1024 x 1024; the row kernel; the GEMM library's path at
+    N = 64) is bit-identical to the two calls, residual updated in place."""
     banner(f"linear_add_rms_norm D={D_} N={N} K={K}")
     a = to_dev(normal_bf16((N, K), 990 + K))
     W = to_dev(normal_bf16((D_, K), 991 + D_, scale=K ** -0.5))

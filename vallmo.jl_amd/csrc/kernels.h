@@ -313,7 +313,7 @@ size_t gemv_sk_workspace_bytes(int M, int K);
 hipError_t launch_gemv_sk(const GemvSkArgs& a, hipStream_t st);
 // y (M, N) = W^T x, or mid (M, N) = silu .* mul of the packed gate-up projection
 // (2 M rows, gate rows first), N <= 32, whole K per workgroup of rw rows
-// (gemv_rows_plan of the rows of W; 0: not for this kernel); K % 64 == 0, M % 4
+// (gemv_rows_plan of the rows of W and the form; 0: not for this kernel); K % 64 == 0, M % 4
 // == 0, 16-byte aligned columns of W and x, 8-byte aligned columns of y
 struct GemvRowsArgs {
   const uint16_t* w;
@@ -324,7 +324,7 @@ struct GemvRowsArgs {
   int64_t y_st;
   int M, N, K, rw;
 };
-int gemv_rows_plan(int M);
+int gemv_rows_plan(int M, bool silu);
 hipError_t launch_gemv_rows(const GemvRowsArgs& a, bool silu, hipStream_t st);
 // mid = silu(bf16(g)) .* bf16(u) from the stream-K partials of the packed
 // gate-up projection (gate rows 0 .. I-1, up rows I .. 2I-1)

@@ -252,15 +252,14 @@ int get_plan(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy, const P
   return rc;
 }
 
-// Narrow problems run on the library's own split-K MFMA kernel (launch_gemv):
-// every N <= 16, and N <= 32 when M <= 4096 (the short, deep out projections
-// and the MLP's down projection). Measured under graph replay on MI355X with
-// the weights cold (rotating copies larger than the 256 MB last-level cache),
-// against the GEMM library's pick: N = 1..16 faster on every decode shape
-// (18432 x 2560 gate-up: 25 vs 56 us), at N = 32 faster for 2560 x 4096 (11.1
-// vs 12.4 us) and 2560 x 9216 (15.6 vs 20.5 us) and 3-6% slower for the
-// wide 10-18K-row projections, which stay on the library. Its loads need
-// 16-byte aligned columns of W and x and 8-byte aligned columns of y.
+// Narrow problems, every N <= 16 and N <= 32 when M <= 4096, run on the library's own
+// MFMA kernels: those of rows_shape below, which takes wide ones up to N = 32 as
+// well, on the row kernel, the others on the split-K kernel (launch_gemv). Measured
+// under graph replay on MI355X with the weights cold (rotating copies larger than
+// the 256 MB last-level cache), against the GEMM library's pick: the split kernel
+// faster at N = 1..16 on every decode shape (18432 x 2560 gate-up: 25 vs 56 us), at N =
+// 32 for 2560 x 4096 (11.1 vs 12.4 us) and 2560 x 9216 (15.6 vs 20.5 us). Their loads
+// need 16-byte aligned columns of W and x and 8-byte aligned columns of y.
 bool gemv_shape(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy) {
   const bool narrow = N <= 16 || (N <= 32 && M <= 4096);
   return narrow && K % 64 == 0 && M % 4 == 0 && ldw % 8 == 0 && ldx % 8 == 0 && ldy % 4 == 0;
@@ -269,19 +268,23 @@ bool gemv_shape(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy) {
 // whole, their rows cut over the CUs (launch_gemv_rows), 0 for the others: no
 // partials, no reduce launch, and less batch traffic than the split kernel.
 // Measured as above, at N = 1 / 8 / 32, split kernel or GEMM library against it:
-// 18432 x 2560 25.2 / 26.2 / 23.3 -> 18.5 / 18.7 / 20.5 us; 10240 x 2560 13.5 /
-// 15.4 / 19.0 -> 11.2 / 12.3 / 14.5; 4608 x 2560 (rows that fill 192 of 256 CUs)
-// 9.4 / 10.2 / 12.0 -> 7.1 / 7.7 / 10.5; 2560 x 4096 10.2 / 11.0 / 11.4 -> 7.9 /
-// 8.1 / 10.1. Deep products of few rows stay split: 2560 x 9216 13.8 / 14.1 /
-// 15.3 against 15.8 / 15.8 / 19.4, 4096 x 9216 at N = 32 19.0 against 23.5; and so
-// do few rows, where the batch tile outweighs the weights (2048 x 2560 at N = 32
-// 7.5 against 7.2).
+// 18432 x 2560 24.9 / 25.7 / 23.3 -> 17.4 / 17.5 / 20.2 us; 10240 x 2560 13.6 / 14.6 / 17.6 ->
+// 10.6 / 10.7 / 13.9; 4608 x 2560 9.5 / 10.3 / 12.1 -> 6.1 / 6.3 / 10.0; 2560 x 4096 10.0 / 10.5 /
+// 11.0 -> 7.1 / 7.0 / 9.0.
+// The lines lie where the projection with its norm (linear_add_norm_run, which must
+// stay bit for bit linear! and the norm) is the shorter one, since there the split
+// kernel has no reduce launch either: 2560 x 4096 11.1 / 11.5 / 12.0 -> 9.7 / 9.9 / 11.9
+// (all shapes to 4096 x 4096 0.83 to 1.05 of the split kernel's, above 1.02 only at N =
+// 32); 2048 x 2560 7.0 / 7.6 / 8.2 against 7.5 / 7.8 / 8.9; 2560 x 9216 14.3 / 14.9 / 16.1 against
+// 15.4 / 15.6 / 20.3. Deep products of more than 8192 rows (rw > 32) are shorter whole:
+// 10240 x 9216 at N = 32 50 -> 37. (Of 4097 to 8192 rows they would be as well, 0.76 to 0.94
+// at K = 4608 to 9216; they are with the split kernel still.)
 int rows_shape(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy) {
   if (N < 1 || N > 32 || M < 2560 || K <= 0 || K % 64 != 0 || M % 4 != 0 || ldw % 8 != 0 ||
       ldx % 8 != 0 || ldy % 4 != 0)
     return 0;
-  const int rw = gemv_rows_plan(M);
-  return K <= 4096 || rw >= 40 ? rw : 0;
+  const int rw = gemv_rows_plan(M, false);
+  return K <= 4096 || rw > 32 ? rw : 0;
 }
 int run_gemv_rows(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const uint16_t* w,
                   int64_t ldw, int M, int N, int K, int rw, bool silu, hipStream_t st,
@@ -616,11 +619,11 @@ int linear_silu_mul_run(uint16_t* mid, int64_t mid_st, const uint16_t* x, int64_
     return VM_E_SCRATCH;
   }
   const bool decode = sk_shape(M, N, K, ldw, ldx) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
-  const int rw = decode ? gemv_rows_plan(M) : 0;
+  const int rw = decode ? gemv_rows_plan(M, true) : 0;
   if (rw > 0) {
-    // one launch (gate-up 18432 x 2560 and the silu at N = 8: 18.4 us against 19.0 +
-    // 4.1 us for the stream-K GEMV and its consumer); the two launches above 96 rows
-    // a CU, the most a workgroup takes
+    // one launch: gate-up 18432 x 2560 and the silu at N = 1 / 8 / 32 22.7 / 23.2 / 25.4 -> 18.2 /
+    // 17.9 / 20.1 us against the stream-K GEMV and its consumer; the two launches above 96
+    // rows a CU, the most a workgroup takes
     return run_gemv_rows(mid, mid_st, x, ldx, w, ldw, I, N, K, rw, true, st, "linear_silu_mul", err,
                          errn);
   }

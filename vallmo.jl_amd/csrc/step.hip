@@ -775,11 +775,19 @@ __global__ __launch_bounds__(RT) void silu_mul_sk_kernel(SiluMulSkArgs a) {
 // with the rows cut over the CUs and K whole: workgroup b owns rows [b RW, (b +
 // 1) RW) of y, or RW / 2 gate rows and the same up rows, so nothing passes through
 // memory between launches: no partials, no reduce or silu launch (4 us each, a
-// tenth of an MLP at decode, for kernels that move next to nothing). HBM-bound:
-// each weight byte is read once, 8 rows x 128 bytes per 1-KB direct load, by one
-// of four waves that split K in contiguous runs and add their sums through LDS
-// in wave order (bitwise repeatable). Where it is used, and its times against
-// the other kernels: rows_shape and linear_silu_mul_run in linear.cpp.
+// tenth of an MLP at decode, for kernels that move next to nothing). HBM-bound
+// where rows are many: each weight byte is read once, 8 rows x 128 bytes per 1-KB
+// direct load, by one of four waves that split K in contiguous runs and add their
+// sums through LDS in wave order (bitwise repeatable). Of few rows the batch, which
+// every workgroup reads whole, is most of what a CU loads (256 KB beside 96 KB of
+// weights for 2560 x 4096 at N = 32), at about 90 GB/s a CU. There it counts that
+//   - rows come in fours, so that 2560 are 214 workgroups and not 160,
+//   - a wave's loop control is scalar and a group's operands are read at once,
+//   - the ring has three slots: with more the first group waits for the loads of all
+//     the waves' others.
+// 2560 x 4096 at N = 1 / 16 / 32: 7.1 / 7.5 / 9.0 us; without the three 7.9 / 8.6 / 10.0. Where it
+// is used, and its times against the other kernels: rows_shape and
+// linear_silu_mul_run in linear.cpp.
 constexpr int GR_RING = 78 * 1024;  // bf16 of the four waves' rings (156 KB)
 constexpr int GR_MAX = 12;         // row pieces (8 rows) per workgroup, at most
 
@@ -816,11 +824,12 @@ template <int NR, bool SILU>
 __device__ __forceinline__ void gemv_rows(const GemvRowsArgs& a) {
   constexpr int T = (NR + 3) / 4;     // 32-row MFMA tiles
   constexpr int SL = (NR + 4) * 512;  // bf16 per slot: NR row pieces, the batch tile
-  constexpr int NS = GR_RING / 4 / SL < 4 ? GR_RING / 4 / SL : 4;
+  constexpr int NS = GR_RING / 4 / SL < 3 ? GR_RING / 4 / SL : 3;
   static_assert(NS >= 2 && (NR + 4) * (NS - 1) < 64, "ring");
   static_assert(4 * T * 16 * 64 * 4 <= GR_RING * 2, "reduction space");
   __shared__ __attribute__((aligned(16))) uint16_t ring_all[GR_RING];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, j = lane & 31, h = lane >> 5;
+  const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar loop control
   const int cl = lane >> 3, p = lane & 7, chunk = 8 * (p ^ cl);
   uint16_t* const ring = ring_all + wv * (NS * SL);
   // local row r of the workgroup: SILU: gate rows r < RW / 2, then the up rows
@@ -833,6 +842,7 @@ __device__ __forceinline__ void gemv_rows(const GemvRowsArgs& a) {
       return min((int)blockIdx.x * a.rw + r, a.M - 1);
     }
   };
+  const bool tail = SILU || 8 * (NR - 1) + cl < a.rw;
   const uint16_t* wp[NR];
 #pragma unroll
   for (int i = 0; i < NR; ++i) wp[i] = a.w + (int64_t)row_of(min(8 * i + cl, a.rw - 1)) * a.w_st + chunk;
@@ -846,8 +856,9 @@ __device__ __forceinline__ void gemv_rows(const GemvRowsArgs& a) {
     const int k = 64 * (g0 + g);
 #pragma unroll
     for (int i = 0; i < NR; ++i)
-      __builtin_amdgcn_global_load_lds(wp[i] + k, (__attribute__((address_space(3))) void*)(slot + 512 * i),
-                                       16, 0, 2);
+      if (i < NR - 1 || tail)  // the last piece may be a half
+        __builtin_amdgcn_global_load_lds(
+            wp[i] + k, (__attribute__((address_space(3))) void*)(slot + 512 * i), 16, 0, 2);
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // the batch stays in L2: default cache policy
       if (i < nx)
@@ -889,24 +900,25 @@ __device__ __forceinline__ void gemv_rows(const GemvRowsArgs& a) {
     if (g + NS < n) issue(g + NS, slot);  // every read of the slot is in
     s = s + 1 == NS ? 0 : s + 1;
   }
-  // the four waves' sums: wave w's tile t, register r, lane l at [w][t][r][l]
-  float* const red = reinterpret_cast<float*>(ring_all);
+  // the four waves' sums: wave w's tile t, registers 4 q .. 4 q + 3 of lane l (rows 8 q
+  // + 4 (l / 32) .. +3 of batch column l % 32) at [w][t][q][l]
+  f32x4* const red = reinterpret_cast<f32x4*>(ring_all);
   __syncthreads();  // every wave is done with its ring
 #pragma unroll
   for (int t = 0; t < T; ++t)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) red[((wv * T + t) * 16 + r) * 64 + lane] = acc[t][r];
+    for (int q = 0; q < 4; ++q)
+      red[((wv * T + t) * 4 + q) * 64 + lane] =
+          f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
   __syncthreads();
   // local rows r .. r + 3 (r % 4 == 0) of batch column c
   auto sum4 = [&](int r, int c, float (&v)[4]) __attribute__((always_inline)) {
-    const float* src = red + ((r >> 5) * 16 + 4 * ((r >> 3) & 3)) * 64 + 32 * ((r >> 2) & 1) + c;
+    const f32x4* src = red + ((r >> 5) * 4 + ((r >> 3) & 3)) * 64 + 32 * ((r >> 2) & 1) + c;
+    f32x4 x = src[0];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float x = src[e * 64];
+    for (int w = 1; w < 4; ++w) x += src[w * T * 256];
 #pragma unroll
-      for (int w = 1; w < 4; ++w) x += src[(w * T * 16 + e) * 64];
-      v[e] = x;
-    }
+    for (int e = 0; e < 4; ++e) v[e] = x[e];
   };
   const int rows = SILU ? hr : a.rw;
   for (int i = threadIdx.x; i < rows / 4 * 32; i += 256) {
@@ -942,18 +954,18 @@ template <bool SILU>
 static void launch_gemv_rows_t(const GemvRowsArgs& a, int wgs, hipStream_t st) {
 #define VM_ROWS(nr) \
   case nr: hipLaunchKernelGGL((gemv_rows_kernel<nr, SILU>), dim3(wgs), dim3(256), 0, st, a); break;
-  switch (a.rw / 8) {
+  switch ((a.rw + 7) / 8) {
     VM_ROWS(1) VM_ROWS(2) VM_ROWS(3) VM_ROWS(4) VM_ROWS(5) VM_ROWS(6)
     VM_ROWS(7) VM_ROWS(8) VM_ROWS(9) VM_ROWS(10) VM_ROWS(11) VM_ROWS(12)
   }
 #undef VM_ROWS
 }
 
-// rows per workgroup, one workgroup per CU (a multiple of 8; of the packed gate-up:
-// RW / 2 gate and as many up rows), 0 where they are more than a workgroup takes
-int gemv_rows_plan(int M) {
-  const int cus = max(1, lm_head_waves() / 4);
-  const int rw = 8 * ((M + 8 * cus - 1) / (8 * cus));
+// rows per workgroup, one workgroup per CU (a multiple of 4; of the packed gate-up,
+// RW / 2 gate and as many up rows, of 8), 0 where they are more than a workgroup takes
+int gemv_rows_plan(int M, bool silu) {
+  const int cus = max(1, lm_head_waves() / 4), unit = silu ? 8 : 4;
+  const int rw = unit * ((M + unit * cus - 1) / (unit * cus));
   return rw <= 8 * GR_MAX ? rw : 0;
 }
 
