@@ -247,7 +247,8 @@ def _silu_mul_bar(orc, x, W, I):
 
 @pytest.mark.parametrize("I,N,K", [(9216, 32, 2560), (9216, 1, 2560), (1000, 20, 640),
                                    (1024, 7, 512), (512, 40, 256), (12288, 9, 192),
-                                   (12296, 3, 256)])
+                                   (12296, 3, 256), (512, 20, 9216), (512, 20, 9280),
+                                   (640, 16, 12288), (640, 16, 12352)])
 def test_linear_silu_mul(vm, orc, I, N, K):
     """linear! + silu .* mul in one call (the MLP's first half, qwen35.jl:234-243):
     at N <= 32 the stream-K GEMV's fp32 partials summed by the silu kernel (I =

@@ -620,10 +620,15 @@ int linear_silu_mul_run(uint16_t* mid, int64_t mid_st, const uint16_t* x, int64_
   }
   const bool decode = sk_shape(M, N, K, ldw, ldx) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0;
   const int rw = decode ? gemv_rows_plan(M, true) : 0;
-  if (rw > 0) {
+  if (rw > 32 || (rw > 0 && K <= (N <= 16 ? 12288 : 9216))) {
     // one launch: gate-up 18432 x 2560 and the silu at N = 1 / 8 / 32 22.7 / 23.2 / 25.4 -> 18.2 /
-    // 17.9 / 20.1 us against the stream-K GEMV and its consumer; the two launches above 96
-    // rows a CU, the most a workgroup takes
+    // 17.9 / 20.1 us against the stream-K GEMV and its consumer, 1024 rows x 1024 10.7 /
+    // 12.0 / 12.5 -> 4.0 / 3.7 / 4.2. The two launches above 96 rows a CU, the most a workgroup
+    // takes, and for few rows that are deep, each on its CU alone while stream-K cuts K
+    // over all: 5120 x 16384 at N = 32 37.7 against 44.2, x 12288 30.9 against 35.4 (N = 16
+    // 0.95), x 9216 26.2 against 26.9 and 4096 x 9216 21.8 against 20.2; of 40 such shapes the
+    // worst 1.03 at K = 9216 and below, 1.15 at 12288. More than 4096 rows of each half:
+    // 0.9 or less at every K.
     return run_gemv_rows(mid, mid_st, x, ldx, w, ldw, I, N, K, rw, true, st, "linear_silu_mul", err,
                          errn);
   }
