@@ -551,7 +551,7 @@ int vm_deltanet_sequence(float* o, const float* q, const float* k, const float* 
  * function: the reference runs the sequential loop (deltanet_recurrent.jl:
  * 109-172); this is the same operator, parallel over each chunk: a chunk
  * kernel, then one sequential scan over the chunks' states that also forms O;
- * T <= 36 runs the sequential kernel. workspace:
+ * a few tokens (36 to 54, by B Hv) run the sequential kernel. workspace:
  * vm_deltanet_sequence_workspace_bytes(T, Hv, B) bytes, 256-byte aligned
  * (about 132 KB per 64-token chunk per value head and sequence). */
 size_t vm_deltanet_sequence_workspace_bytes(int T, int Hv, int B);

@@ -530,12 +530,14 @@ def test_deltanet_sequence_chunked(vm, orc, B, T):
 
 
 @pytest.mark.parametrize("Hk,Hv,B,T", [(2, 2, 1, 36), (2, 2, 1, 37), (1, 3, 2, 64), (8, 8, 1, 129),
-                                       (2, 8, 1, 191)])
+                                       (2, 8, 1, 191), (2, 8, 8, 40), (2, 8, 8, 41),
+                                       (2, 12, 16, 54), (2, 12, 16, 55)])
 def test_deltanet_sequence_chunked_groups(vm, orc, Hk, Hv, B, T):
-    """The chunked form at value-head groups of 1, 3 and 4 (phase 1 takes two value
+    """The chunked form at value-head groups of 1, 3, 4 and 6 (phase 1 takes two value
     heads a workgroup, the last one alone), qk heads that do and do not spread
-    over the XCDs, both sides of the sequential kernel's range (T = 36) and
-    chunk edges: 5e-4 of the largest value, as the tests above."""
+    over the XCDs, both sides of the sequential kernel's range (T = 36 with few
+    heads, 40 with 64, 54 with 192) and chunk edges: 5e-4 of the largest value, as
+    the tests above."""
     banner(f"deltanet sequence chunked Hk={Hk} Hv={Hv} B={B} T={T}")
     rng = np.random.default_rng(Hk * 1000 + Hv * 100 + T)
     unit = lambda x: (x / np.linalg.norm(x, axis=-1, keepdims=True)).astype(np.float32)

@@ -1431,11 +1431,20 @@ size_t deltanet_chunk_workspace_bytes(int T, int Hv, int B) {
   return (NC * (UNIT + KQ_UNIT) + (size_t)T * DN_D) * Hv * B * sizeof(float);
 }
 
-// Up to SEQ_T tokens the sequential kernel is the faster form: it takes 2 us + 0.6
-// us a token whatever the batch, the two chunked launches 24 us (B = 1, Hv = 32)
-// to 39 us (B = 4) for a chunk of any length. Measured at B = 1 / 4, T = 32: 21.3 /
-// 23.7 us sequential, 23.9 / 38.5 chunked; T = 40: 26.0 / 30.0 and 24.1 / 38.9.
-constexpr int SEQ_T = 36;
+// Up to this many tokens the sequential kernel is the faster form, by the scan's
+// rounds (its 8 workgroups per value head and sequence, one on a CU at a time): the
+// sequential kernel takes about 0.6 us a token up to 64 heads (B Hv) and from there
+// on as well time in proportion to them, the two chunked launches the same for every
+// T up to 64, one round after the other. Crossing points measured at 2 to 2048 heads,
+// 1 to 4 value heads per qk head, 256 CUs: 35 to 38 tokens up to 32 heads (T = 36: 24.6 us
+// sequential, 24.6 chunked), 43 at 48 and 64 (40: 27.2, 29.3; 48: 31.8, 29.6), 48 at 96 and 128
+// (48: 38.6, 40.0), 52 at 144, 53 to 57 from 192 to 1024 (256 heads, 48: 52.1, 59.5; 56: 60.0,
+// 60.1; 64: 66.7, 60.3), 60 and more beyond.
+static int sequential_tokens(int64_t heads) {
+  const int64_t cus = max(1, lm_head_waves() / 4);
+  const int64_t rounds = (heads * (DN_D / CBW) + cus - 1) / cus;
+  return (int)min((int64_t)54, 36 + 4 * (rounds - 1));
+}
 hipError_t launch_deltanet_sequence_chunked(const DeltaChunkArgs& args, hipStream_t st) {
   DeltaChunkArgs a = args;
   const DeltaSeqArgs& q = a.s;
@@ -1446,7 +1455,7 @@ hipError_t launch_deltanet_sequence_chunked(const DeltaChunkArgs& args, hipStrea
     a.g.o = a.s.o;
   }
   const int R = q.Hv / q.Hk;  // value heads per qk head, two a workgroup
-  if (q.T <= SEQ_T) {
+  if (q.T <= sequential_tokens((int64_t)q.B * q.Hv)) {
     hipError_t e = launch_deltanet_sequence(a.s, st);
     if (e != hipSuccess || !a.g.y) return e;
     return launch_gated_rms_norm(a.g, st);
