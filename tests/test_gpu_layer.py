@@ -222,6 +222,29 @@ def test_linear_rows(vm, orc, M, N, K):
     assert bool((buf[:, :16] == 3.0).all()) and bool((buf[:, 16 + M:] == 3.0).all())
 
 
+def test_linear_rows_wide_without_the_library(vm):
+    """A wide problem of the row kernel at N = 17 .. 32 runs none of the GEMM library:
+    vm_linear_tune leaves its plan as the heuristic's first, untimed, and a y whose
+    columns start at every 4 elements takes the same kernel (same bits)."""
+    banner("linear rows wide, no library")
+    lib = vm._lib
+    M, N, K = 8216, 21, 640
+    prob = (M, N, K, K, K, M)
+    assert lib.load().vm_linear_plan_state(*prob) == -2  # a shape of this test alone
+    lib.call("vm_linear_tune", *prob)
+    assert lib.load().vm_linear_plan_state(*prob) <= -1
+    xd = to_dev(normal_bf16((N, K), 780))
+    Wd = to_dev(normal_bf16((M, K), 781, scale=K ** -0.5))
+    y = vm.linear(xd, Wd)["y"]
+    for pad, off in ((4, 0), (4, 4), (8, 4)):
+        buf = torch.full((N, M + pad), 3.0, dtype=torch.bfloat16, device="cuda")
+        vm.linear_({"y": buf[:, off:off + M]}, xd, Wd)
+        torch.cuda.synchronize()
+        assert torch.equal(buf[:, off:off + M].contiguous().view(torch.int16), y.view(torch.int16))
+        rest = torch.cat((buf[:, :off], buf[:, off + M:]), 1)
+        assert bool((rest == 3.0).all())
+
+
 def _silu_mul_bar(orc, x, W, I):
     """The oracle's mid (orc.linear's fp32 gate-up rounded to bf16, as the
     reference stores gu, then orc.silu_mul, rounded) and a per-element bar:

@@ -345,9 +345,9 @@ int run_gemm_any(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const
 
 int linear_tune(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy, char* err, size_t errn) {
   if (general_strides(ldw, ldx, ldy)) return VM_OK;  // the general kernel: nothing to tune
-  if (gemv_shape(M, N, K, ldw, ldx, ldy)) {
-    // aligned views run the GEMV, which has nothing to tune; the plan stays
-    // the heuristic's first (it only serves misaligned views)
+  if (gemv_shape(M, N, K, ldw, ldx, ldy) || rows_shape(M, N, K, ldw, ldx, ldy)) {
+    // the narrow kernels, which have nothing to tune; the plan stays the heuristic's
+    // first (it only sizes the workspace)
     const Plan* p = nullptr;
     const int rc = get_plan(M, N, K, ldw, ldx, ldy, &p, err, errn);
     return rc == VM_E_UNSUPPORTED ? VM_OK : rc;
@@ -448,10 +448,17 @@ int linear_run(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const u
     }
     return VM_OK;
   }
-  if (general_view(y, x, w, ldw, ldx, ldy))
+  // a wide problem of the row kernel: the library's plan, where it has one, only
+  // sizes the workspace that vm_linear_workspace_bytes asks for
+  const int rw = gemv_aligned(y, x, w) ? rows_shape(M, N, K, ldw, ldx, ldy) : 0;
+  if (rw > 0 && general_strides(ldw, ldx, ldy))
+    return run_gemv_rows(y, ldy, x, ldx, w, ldw, M, N, K, rw, false, st, "linear", err, errn);
+  if (general_view(y, x, w, ldw, ldx, ldy) && rw == 0)
     return run_gemm_any(y, ldy, x, ldx, w, ldw, M, N, K, st, err, errn);
   const Plan* p = nullptr;
   int rc = get_plan(M, N, K, ldw, ldx, ldy, &p, err, errn);
+  if (rc == VM_E_UNSUPPORTED && rw > 0)
+    return run_gemv_rows(y, ldy, x, ldx, w, ldw, M, N, K, rw, false, st, "linear", err, errn);
   if (rc == VM_E_UNSUPPORTED) return run_gemm_any(y, ldy, x, ldx, w, ldw, M, N, K, st, err, errn);
   if (rc != VM_OK) return rc;
   if (p->workspace > 0 && (workspace == nullptr || workspace_bytes < p->workspace)) {
@@ -459,7 +466,7 @@ int linear_run(uint16_t* y, int64_t ldy, const uint16_t* x, int64_t ldx, const u
              workspace_bytes, p->workspace);
     return VM_E_SCRATCH;
   }
-  if (const int rw = rows_shape(M, N, K, ldw, ldx, ldy))
+  if (rw > 0)
     return run_gemv_rows(y, ldy, x, ldx, w, ldw, M, N, K, rw, false, st, "linear", err, errn);
   hipblasLtHandle_t h;
   {
