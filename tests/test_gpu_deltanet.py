@@ -458,6 +458,49 @@ def test_deltanet_conv_prep_runs(vm, taps, T):
     assert torch.equal(S1, S2)
 
 
+def test_deltanet_conv_prep_signs_and_tiny(vm):
+    """The one-pass conv and prep against the two kernels where its one division a
+    row could differ: q and k elements that silu takes to -0 (conv outputs below
+    -104) keep their sign, bit for bit; rows of 1e-30 to 1e-37, whose remainders are
+    no longer exact, have quotients within one ulp (k), which q's scale, below a power
+    of two, and its rounding can make two."""
+    banner("deltanet conv + prep signs and tiny rows")
+    B, T, hk, hv, taps = 1, 24, 2, 2, 2
+    n = 2 * hk * DK + hv * DV
+    X = to_dev(normal_bf16((B, T, n), 2110))
+    W = torch.ones((taps, n), dtype=torch.bfloat16, device="cuda")
+    X[0, 4:12, ::3] = -300.0
+    for i, t in enumerate(range(14, T)):
+        X[0, t] = to_dev(normal_bf16((n,), 2111 + t)) * 10.0 ** (-30 - 7 * i / 9)
+    AB = to_dev(normal_bf16((B, T, 2 * hv), 2112))
+    A, Dt = f32dev(normal_f32(hv, 2113, scale=0.5)), f32dev(normal_f32(hv, 2114, scale=0.5))
+
+    def outs():
+        f = dict(dtype=torch.float32, device="cuda")
+        return {"Q": torch.empty((B, hk, T, DK), **f), "K": torch.empty((B, hk, T, DK), **f),
+                "V": torch.empty((B, hv, T, DV), **f), "Beta": torch.empty((B, T, hv), **f),
+                "Gate": torch.empty((B, T, hv), **f)}
+
+    conv = vm.causal_conv1d_sequence(X, W, None, sigma="silu")["Y"]
+    two, one = outs(), outs()
+    vm.deltanet_prefill_prep_(two, conv, AB, A, Dt, Dk=DK, Dv=DV, Hk=hk, Hv=hv)
+    vm.deltanet_conv_prep_(one, X, W, AB, A, Dt, None, Dk=DK, Dv=DV, Hk=hk, Hv=hv)
+    torch.cuda.synchronize()
+    bits = lambda a: a.contiguous().view(torch.int32)
+    for key in one:
+        a, b = one[key], two[key]
+        if key in ("Q", "K"):
+            a, b = a[:, :, :14], b[:, :, :14]
+        assert torch.equal(bits(a), bits(b)), key
+    zeros = two["Q"][..., :14, :] == 0
+    assert bool((zeros & (bits(two["Q"][..., :14, :]) < 0)).any())  # there are some -0
+    for key, most in (("Q", 2), ("K", 1)):
+        a, b = bits(one[key][..., 14:, :]), bits(two[key][..., 14:, :])
+        d = int((a - b).abs().max())
+        print(f"{key}: tiny rows differ by at most {d} ulp")
+        assert d <= most
+
+
 def test_prep_many_value_heads(vm, orc):
     """The prep with more value heads than a wave has lanes (Hk = 2, Hv = 72): the
     gates of heads 64 .. 71 too."""

@@ -1256,8 +1256,7 @@ __global__ __launch_bounds__(256) void conv1d_sequence_kernel(Conv1dArgs a) {
 // kernels), then each q / k head row is scaled by its inverse L2 norm (q also
 // by Dk^-1/2) over the group, and the row is written fp32 to Q / K / V, head
 // major, as deltanet_prep_vec_kernel writes it: bit for bit the two-kernel
-// result (a zero's sign aside), without the conv output's round trip through
-// memory. Workgroup column 0 also writes beta and the gate of its run's tokens.
+// result, without the conv output's round trip through memory. Workgroup column 0 also writes beta and the gate of its run's tokens.
 // Bound by VALU issue (silu's exp and division are most of ~400 instructions per
 // token and wave) beside 203 MB at T = 4096, so both are kept under way: the next
 // K tokens' rows load while K are computed, the window turns through K fixed
@@ -1265,7 +1264,10 @@ __global__ __launch_bounds__(256) void conv1d_sequence_kernel(Conv1dArgs a) {
 // row of q or k divides once. Runs of 8 tokens put 8 waves on a SIMD at T = 4096
 // and 4 at 2000. B = 1, 8192 channels, T = 4096 / 2001: 66.5 / 41.0 -> 56.3 / 29.7
 // us; runs of 16 as before 57.6 / 31.9, of 12 58.4 / 32.4; the shorter runs
-// without the rest (9 tokens) 61.5 / 33.3.
+// without the rest (9 tokens) 61.5 / 33.3. Runs of 8 against 16 over 2, 4 and 8 taps
+// (8 re-read 7 rows of context a run), tokens B T: 16 to 64 10.5 to 12.1 against 17.7 to
+// 19.4 us, 1024 17.1 to 20.3 against 20.7 to 23.5, 4096 43.0 / 47.4 / 56.6 against 44.3 / 48.0 /
+// 56.6, 16384 199 / 205 / 230 against 199 / 200 / 226.
 constexpr int PREP_TC = 8;
 
 template <int K>
@@ -1351,13 +1353,15 @@ __global__ __launch_bounds__(256) void deltanet_conv_prep_kernel(ConvPrepArgs a)
         ss += xor32<1>(ss);
         const float den = sqrtf(ss + 1e-6f);
         if (den < INFINITY) {
-          // x / den, correctly rounded, from the row's one reciprocal: the quotient's
-          // exact remainder corrects it
+          // x / den from the row's one reciprocal by Markstein's correction: y = x inv is
+          // within an ulp, and the remainder x - y den, exact in an fma where |x| is
+          // above 2^-102 (below that within 2^-150), brings it to the rounded quotient.
+          // The remainder is formed negated, so that a zero keeps x's sign.
           const float inv = 1.0f / den;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
             const float y = x[j] * inv;
-            x[j] = fmaf(fmaf(-y, den, x[j]), inv, y) * sc;
+            x[j] = fmaf(-fmaf(y, den, -x[j]), inv, y) * sc;
           }
         } else {
 #pragma unroll
