@@ -146,7 +146,9 @@ int vm_knorm_rope_append(vm_bf16* k_cache, int64_t kc_st, int64_t kc_sh, int64_t
  * scratch holds one fp32 partial (G*D values + G (max, sum) pairs) per wave
  * and per (b, hk) segment, then a snapshot of the partition (1 + 2B int32
  * in whole 256-byte blocks) that the merge reads instead of lengths.
- * D = 128 and 64 run the same way (chunks of whole ring slots, 4096 / D tokens).
+ * D = 128 and 64 run the same way, lengths counted in whole ring slots of 4096 / D
+ * tokens and chunks of one slot or more, while n_splits * B * Hk is at most 2^24 (and,
+ * at D = 64, Ctx > 32 or H / Hk > 4).
  *
  * Other shapes run a generic kernel with the reference's split: n_splits
  * tile-aligned key ranges per (b, hk) (n_splits = 0: about four workgroups
@@ -307,10 +309,11 @@ int vm_gated_attn_prefill_staged(vm_bf16* out, int64_t out_st, int64_t out_sb,
  * reference: x :: (K, N) with column stride ldx >= K, W :: (K, M) (K-major,
  * the checkpoint's orientation) with column stride ldw >= K, y :: (M, N) with
  * column stride ldy >= M; all bf16, fp32 accumulation (linear.jl:29). Narrow
- * problems (N <= 16, or N <= 32 with M <= 4096; K % 64 == 0, M % 4 == 0,
- * 16-byte aligned W and x columns)
- * run on the library's split-K MFMA GEMV, whose K slices add in a fixed order
- * (bitwise reproducible); the rest on hipBLASLt. A plan per
+ * problems (N <= 16, or N <= 32 with M <= 4096, or N <= 32 with 2560 <= M and K <=
+ * 4096 or M of more than 32 rows per CU, up to 96 rows per CU; K % 64 == 0, M % 4
+ * == 0, 16-byte aligned W and x columns, 8-byte aligned y columns) run on the
+ * library's own MFMA kernels, one with K whole and one whose K slices add in a
+ * fixed order (both bitwise reproducible); the rest on hipBLASLt. A plan per
  * problem (hipBLASLt) is built on the first call and cached (linear.jl:17-38)
  * with the heuristic's first algorithm, as the reference takes it: building it
  * is host work only, so the first call of a shape may run inside a capture;
@@ -333,7 +336,7 @@ size_t vm_linear_workspace_bytes(int M, int N, int K, int64_t ldw, int64_t ldx, 
  * Call it at load, before vm_linear_workspace_bytes (a tuned plan may need a
  * larger workspace); once per problem (later calls return at once).
  * VM_LINEAR_TUNE=0 in the environment keeps the first. Narrow problems that
- * run the GEMV have nothing to tune.
+ * run the library's own kernels have nothing to tune.
  * vm_linear_plan_state: -2 no plan, -1 the heuristic's first, k >= 0 tuned
  * (candidate k kept, 0 = the heuristic's first).                              */
 int vm_linear_tune(int M, int N, int K, int64_t ldw, int64_t ldx, int64_t ldy);
@@ -371,9 +374,10 @@ int vm_linear_add_rms_norm(vm_bf16* y, int64_t y_st, vm_bf16* x, int64_t x_st, c
  * for callers that want the bf16 gu never written. At N <= 32 (a decode
  * batch; K a multiple of 64, aligned columns) one launch does both while a CU's
  * share of the 2I rows is at most 96, each workgroup holding its gate rows and
- * the same up rows; above that a stream-K GEMV runs whose fp32 partials the
- * silu kernel adds in a fixed order. Both are bitwise repeatable, with the same
- * rounding points as the two calls and the sums in another order. Otherwise it is linear! + silu .* mul. I a multiple of 8; mid a
+ * the same up rows; above that, and for few rows that are deep, a stream-K GEMV
+ * runs whose fp32 partials the silu kernel adds in a fixed order. Both are bitwise
+ * repeatable, with the same rounding points as the two calls and the sums in
+ * another order. Otherwise it is linear! + silu .* mul. I a multiple of 8; mid a
  * 16-byte aligned (I, N) with an element column stride (a multiple of 8);
  * workspace (256-byte aligned) of vm_linear_silu_mul_workspace_bytes bytes
  * ((size_t)-1 on a bad shape).                                              */

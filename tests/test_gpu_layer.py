@@ -140,7 +140,7 @@ def test_linear_narrow_split_workspace(vm):
     graph replayed with other problems run eagerly between the replays all give
     the fresh-workspace results, bit for bit."""
     banner("linear narrow split workspace")
-    probs = [(DM, 32, 9216), (DM, 16, HQ * D), (DM, 3, HQ * D), (4096, 25, 1024)]
+    probs = [(DM, 32, 9216), (2048, 16, HQ * D), (1280, 3, HQ * D), (1024, 25, 1024)]
     xs, Ws, refs = [], [], []
     for i, (M, N, K) in enumerate(probs):
         x = to_dev(normal_bf16((N, K), 740 + i))
@@ -274,9 +274,10 @@ def _silu_mul_bar(orc, x, W, I):
                                    (640, 16, 12288), (640, 16, 12352)])
 def test_linear_silu_mul(vm, orc, I, N, K):
     """linear! + silu .* mul in one call (the MLP's first half, qwen35.jl:234-243):
-    at N <= 32 the stream-K GEMV's fp32 partials summed by the silu kernel (I =
-    9216: the decode step's shape; 1000: row groups past the end of W), at N =
-    40 linear! + silu .* mul. Every element within the bar of the propagated
+    at N <= 32 one launch (I = 9216: the decode step's shape; 1000: a last workgroup
+    that is not full) or, of more than 96 rows a CU (I = 12296) or few deep ones (K
+    = 9280 at N = 20, 12352 at N = 16), the stream-K GEMV's fp32 partials summed by
+    the silu kernel; at N = 40 linear! + silu .* mul. Every element within the bar of the propagated
     bf16 roundings of gate and up; a second call bitwise equal; a strided mid
     honoured."""
     banner(f"linear_silu_mul I={I} N={N} K={K}")

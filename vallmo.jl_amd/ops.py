@@ -314,7 +314,8 @@ def linear_add_rms_norm_(outs, a, W, norm_w, *, eps, offset, workspace=None):
     h = bf16(W^T a); X = bf16(X + h) in place; Y = rms_norm(X) (w + offset).
     outs: "Y" (D, N) and "X" (D, N), the residual stream updated in place;
     a :: (K, N), W :: (K, D) K-major (torch (D, K)). No reference counterpart
-    as one op; saves the reduce launch of a split GEMV and the bf16 h."""
+    as one op; a split GEMV's slices go straight to the norm, without its reduce
+    launch and the bf16 h."""
     Y, X = _out(outs, "Y"), _out(outs, "X")
     D, N, ys = _cols(Y, "Y")
     Dx, Nx, xs = _cols(X, "X")
@@ -348,9 +349,9 @@ def linear_silu_mul_(mid, x, W, *, workspace=None):
     """linear! then silu .* mul in one call (the MLP's first half,
     src/llm/qwen35.jl:234-243): gu = bf16(W^T x), mid = bf16(silu(gate) .* up).
     x :: (K, N), W :: (K, 2I) K-major (torch (2I, K)), gate rows first; mid ::
-    (I, N) (torch (..., I)). No reference counterpart as one op: at N <= 32 the
-    projection's fp32 partials go straight to the silu kernel, gu is never
-    written."""
+    (I, N) (torch (..., I)). No reference counterpart as one op: at N <= 32 one
+    kernel does both (or, of very many rows or few deep ones, the projection's fp32
+    partials go straight to the silu kernel), and gu is never written."""
     I, N, ms = _cols(mid, "mid")
     K, Nx, xs = _cols(x, "x")
     if W.dim() != 2 or tuple(W.shape) != (2 * I, K) or Nx != N:
