@@ -1,6 +1,6 @@
 """Benchmark of the gated full-attention path on one MI355X.
 
-Headline (BASELINE.json ``metric``, configs[1]): causal gated-attention prefill,
+Headline (config 2): causal gated-attention prefill,
 B=1, T=4096, 16 q / 4 kv heads, head_dim 256, 64-dim partial RoPE (theta 1e7).
 One step = vm_gated_attn_prefill over one synthetic packed projection: one
 kernel for the K/V norm+RoPE cache append and the V -> V^T workspace staging,
@@ -8,7 +8,7 @@ then the flash-attention kernel with the q norm+RoPE prologue and sigmoid-gate
 epilogue. ``value`` = algorithmic TFLOP/s =
 4*D*Hq*sum_{i=1..T} i / step time (QK^T + PV over unmasked pairs only).
 
-Also reported (same JSON line, key "decode"): BASELINE configs 3 (B=32 batched
+Also reported (same JSON line, key "decode"): configs 3 (B=32 batched
 decode, lengths ~U{1024..32768}) and 4 (B=1 at 131072 tokens, one step captured
 in a hipGraph and replayed 256 times on a dedicated stream with the position
 advancing on the device; under the HIP runtime's default graph launch path, and
@@ -19,7 +19,7 @@ and config 1 (B=1 at 512 tokens, launch-latency-bound) as time per step.
 Key "prefill_config2_online_max": the config-2 prefill with one K-norm weight
 of 4 (kw[0] = 4), whose logit bound passes the static shift's 64 so the kernel
 takes its online-max softmax; "decode.config3_running_max" likewise for config 3.
-Key "prefill_config5": BASELINE config 5 (B=4 ragged chunks after 8-32 K
+Key "prefill_config5": config 5 (B=4 ragged chunks after 8-32 K
 priors) in algorithmic TFLOP/s, step and attention kernel, and the step with the
 layer's V^T workspace kept between chunks (staging the chunk only). Key "decode_step": the
 whole captured decode step of a Qwen3.5-4B-shaped model (24 Gated DeltaNet + 8
@@ -872,7 +872,7 @@ def _dev_normal(vm, torch, shape, seed, scale=1.0):
 
 def cpu_baseline(vm, torch):
     """The fp32 C oracle (oracle/, test infrastructure) timed on this host's cores
-    for every BASELINE config, on the same seeded inputs as the GPU legs (generated
+    for every config, on the same seeded inputs as the GPU legs (generated
     on the device by the same generator and copied to host memory):
       config 1, 3: one decode step (median of repeated steps);
       config 4: 8 consecutive decode steps at 131072.. (per-step median);
@@ -1137,7 +1137,7 @@ def main():
                     help="skip the config-4 measurement with the runtime's packet capture off")
     args = ap.parse_args()
     if args.gpus != 1:
-        print(f"bench.py: this build measures one GPU only (--gpus {args.gpus} requested); "
+        print(f"bench.py: this benchmark measures one GPU only (--gpus {args.gpus} requested); "
               "the multi-GPU sharding is a design note, not a measured path", file=sys.stderr)
         sys.exit(2)
 

@@ -355,7 +355,8 @@ int vm_linear(vm_bf16* y, int64_t ldy, const vm_bf16* x, int64_t ldx, const vm_b
  *   y = x rstd (w + offset)  rstd over the fp32 x + h, y from the stored x
  * bit-identical to the two calls. A narrow problem whose GEMV splits K hands
  * its fp32 slices straight to the norm, which adds them in slice order (no
- * reduce launch, no h in HBM). M a multiple of 8, at most 16384; workspace
+ * reduce launch, no h in HBM); one whose GEMV takes whole K writes h to the
+ * workspace, as a wide one does. M a multiple of 8, at most 16384; workspace
  * (256-byte aligned) of vm_linear_add_rms_norm_workspace_bytes bytes
  * ((size_t)-1 on a bad shape).                                              */
 size_t vm_linear_add_rms_norm_workspace_bytes(int M, int N, int K, int64_t ldw, int64_t lda);

@@ -2,7 +2,7 @@
 (DeltaNet + conv1d) layer parts — TEST INFRASTRUCTURE.
 
 Only tests/, ``__graft_entry__.smoke()`` and ``bench.py``'s ``cpu_baseline`` leg
-may import this package, and only as the checker (never as the measured or
+may import this package, and only as the oracle (never as the measured or
 shipped path). ``liboracle.so`` is built from ``oracle.c`` and ``deltanet.c`` by
 ``oracle/Makefile``.
 

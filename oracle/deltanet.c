@@ -2,7 +2,7 @@
  * deltanet.c — CPU fp32 restatement of the reference's linear-attention layer
  * parts: the depthwise causal conv1d and the gated delta-rule recurrence.
  *
- * TEST INFRASTRUCTURE ONLY (the parity checker, like oracle.c): only tests/,
+ * TEST INFRASTRUCTURE ONLY (the parity oracle, like oracle.c): only tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it. The
  * product path does not link or call it.
  *

@@ -1,7 +1,7 @@
 /*
  * oracle.c — CPU fp32 restatement of the reference's gated full-attention path.
  *
- * TEST INFRASTRUCTURE ONLY. This file is the parity checker: only tests/,
+ * TEST INFRASTRUCTURE ONLY. This file is the parity oracle: only tests/,
  * __graft_entry__.smoke() and bench.py's cpu_baseline leg may load it, and
  * never as the thing measured or shipped. The product path (libvallmo_attn.so)
  * does not link or call it.

@@ -1,6 +1,6 @@
 """Decode path on the GPU vs the oracle: decode!(::AttnLayer) fused step (a7 =
 a3+a4+a5+a6), decode_attention! (a5) alone, split-count invariance, GQA group
-sizes, ragged/edge lengths, BASELINE config 1 and config 3 at full size (sampled
+sizes, ragged/edge lengths, config 1 and config 3 at full size (sampled
 sequences against the oracle), and config 4 as a hipGraph replayed with the
 position advancing on the device (replays == eager steps, bit for bit)."""
 from __future__ import annotations
@@ -60,7 +60,7 @@ def run_decode_vs_oracle(vm, orc, B, ctx, pos, Hq=HQ, Hk=HK, seed=0, n_splits=0,
 
 
 def test_config1_decode_parity(vm, orc):
-    """B=1, 16/4 heads, ctx 512, position 511 (0-based)."""
+    """Config 1: B=1, 16/4 heads, ctx 512, position 511 (0-based)."""
     banner("config1 decode B=1 ctx=512 pos=512")
     (mx, mn), (kmx, kmn), vexact, _, _ = run_decode_vs_oracle(vm, orc, 1, 512, [512], seed=100)
     print(f"config1: out max {mx:.3e} mean {mn:.3e}; K max {kmx:.3e} mean {kmn:.3e}")
@@ -158,7 +158,7 @@ def test_decode_attention_operator(vm, orc):
 
 
 def test_config3_batched_decode_full_size(vm, orc):
-    """BASELINE config 3 at full size: B=32, capacity 32768, attended lengths
+    """Config 3 at full size: B=32, capacity 32768, attended lengths
     ~U{1024..32768} (seeded); every sequence re-evaluated by the oracle (its
     caches copied to the host one sequence at a time), with its appended row."""
     banner("config3 decode B=32 ctx=32768")
@@ -198,7 +198,7 @@ def test_config3_batched_decode_full_size(vm, orc):
 
 
 def test_config4_graph_replay_matches_eager(vm, orc):
-    """one decode step (append, split-K, merge, gate, advance)
+    """Config 4: one decode step (append, split-K, merge, gate, advance)
     captured once in a hipGraph; replays advance the device clock. 256 replays
     (positions 131072..131327) equal 256 eager steps bit for bit (outputs and the
     256 appended cache rows), and the last step matches the oracle."""

@@ -1,7 +1,7 @@
 """The projections around the block and whole attention layers on the GPU vs the
 oracle: linear! (hipBLASLt, src/linear.jl:40-57) alone for the decode GEMV and
 prefill GEMM shapes, decode!(h, ::AttnLayer, m, gen, xn) (qwen35.jl:187-208) at
-BASELINE config 1 and forward(::AttnLayer, m, xn, T, B) (qwen35.jl:292-318) at
+config 1 and forward(::AttnLayer, m, xn, T, B) (qwen35.jl:292-318) at
 config 2, hidden state to hidden state, and the whole decode layer step captured
 in a hipGraph and replayed with the position advancing (replays == eager)."""
 from __future__ import annotations
@@ -388,7 +388,7 @@ def _layer(vm, cfg, seed):
 
 
 def test_decode_layer_config1(vm, orc):
-    """BASELINE config 1 through the whole layer: xn -> qkv GEMV -> gated decode
+    """Config 1 through the whole layer: xn -> qkv GEMV -> gated decode
     -> Wo GEMV -> h, against the oracle; the appended cache row too."""
     banner("decode layer config1 B=1 ctx=512 pos=512")
     B, ctx, pos = 1, 512, 512
@@ -416,7 +416,7 @@ def test_decode_layer_config1(vm, orc):
 
 
 def test_prefill_layer_config2(vm, orc):
-    """BASELINE config 2 through the whole layer: xn -> qkv GEMM -> gated prefill
+    """Config 2 through the whole layer: xn -> qkv GEMM -> gated prefill
     -> Wo GEMM -> h, T = 4096; every 16th row against the oracle."""
     banner("prefill layer config2 T=4096")
     B, T = 1, 4096

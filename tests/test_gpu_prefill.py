@@ -1,6 +1,6 @@
 """Prefill path on the GPU vs the oracle: attention! (a8) alone, the fused
 forward(::AttnLayer) (a9 prologue + a8 + a10 gate epilogue, a11) including
-ragged chunked prefill, BASELINE configs 2 and 5 at full size (sampled query
+ragged chunked prefill, configs 2 and 5 at full size (sampled query
 rows against the oracle, every appended cache row checked), and the
 cross-kernel identities: decode == last prefill row, chunked == full prefill."""
 from __future__ import annotations
@@ -112,7 +112,7 @@ def test_fused_prefill_cache_ends_in_tile(vm, orc, ctx):
 
 
 def test_config2_prefill_full_size(vm, orc):
-    """causal prefill, B=1, T=4096, offset 0; every query row
+    """Config 2: causal prefill, B=1, T=4096, offset 0; every query row
     re-evaluated by the oracle, every appended K/V row checked."""
     banner("config2 prefill T=4096")
     (mx, mn), (kmx, kmn), ok, _ = _fused(vm, orc, 1, 4096, 4096, np.array([0], np.int32),
@@ -122,7 +122,7 @@ def test_config2_prefill_full_size(vm, orc):
 
 
 def test_config5_chunked_prefill_full_size(vm, orc):
-    """B=4 ragged chunks (a seeded permutation of
+    """Config 5: B=4 ragged chunks (a seeded permutation of
     {512, 1024, 2048, 2048}) after prior caches ~U{8192..32768}; every query row
     of every sequence re-evaluated by the oracle."""
     rng = np.random.default_rng(5)
